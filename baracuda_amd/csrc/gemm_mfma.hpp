@@ -378,8 +378,8 @@ __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, i
     constexpr int XCDS = 8;
     constexpr int GROUP_M = 4;
     const int total = tiles_m * tiles_n;
-    int t = pid;
-    if (total % XCDS == 0) t = (pid % XCDS) * (total / XCDS) + pid / XCDS;
+    const int x = pid % XCDS, q = total / XCDS, r = total % XCDS;
+    const int t = x * q + (x < r ? x : r) + pid / XCDS;
     const int group_span = GROUP_M * tiles_n;
     const int g = t / group_span;
     const int first_m = g * GROUP_M;

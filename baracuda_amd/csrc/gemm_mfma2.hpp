@@ -3,7 +3,8 @@
 //
 // C[m,n] = sum_k A[m,k] * B[n,k]; A row-major [M,K], B row-major [N,K] (the
 // RCR "column-major [K,N]" operand).  Requirements checked by the launcher:
-// K % 128 == 0, lda % 16 == 0, ldb % 16 == 0, 16-byte aligned bases.
+// K % 16 == 0 (bytes; a partial last stage is zero-filled), lda % 16 == 0,
+// ldb % 16 == 0, 16-byte aligned bases.
 //
 // Block tile 256(M) x 256(N); Cfg<WAVES_M, WAVES_N> picks the wave
 // grid (the int8 and FP8 kernels use 2 x 4 wave64s, each owning a 128 x 64
@@ -47,21 +48,25 @@ constexpr int OPER = BM * BK;        // 32 KiB per operand per stage
 // wave of the SIMD.  (Measured slower and removed: double-buffered
 // fragments, a mid-stage barrier, pinned read/MFMA interleaving, a
 // ping-pong of the two waves of a SIMD, one wave per SIMD.)
-// TB: square block tile edge (256 by default; the A and B stage regions are
-// TB x BK bytes each, B at stage + OPER).
-template <int WAVES_M_, int WAVES_N_, int TB_ = 256>
+// TB x TBN: block tile (256 x 256 by default); a stage holds its TB A rows of
+// BK bytes, then its TBN B rows at stage + OPER.
+template <int WAVES_M_, int WAVES_N_, int TB_ = 256, int TBN_ = TB_>
 struct Cfg {
     static constexpr int WAVES_M = WAVES_M_;
     static constexpr int WAVES_N = WAVES_N_;
     static constexpr int TB = TB_;
-    static constexpr int OPER = TB * BK;                    // bytes per operand per stage
+    static constexpr int TBN = TBN_;
+    static constexpr int OPER = TB * BK;                    // bytes of A per stage
+    static constexpr int STAGE = (TB + TBN) * BK;           // bytes per stage
     static constexpr int WAVES = WAVES_M * WAVES_N;
     static constexpr int NT = 64 * WAVES;
     static constexpr int WM = TB / WAVES_M;
-    static constexpr int WN = TB / WAVES_N;
-    static constexpr int ROWS_PER_WAVE = TB / WAVES;       // DMA rows per wave per operand
+    static constexpr int WN = TBN / WAVES_N;
+    static constexpr int ROWS_PER_WAVE = TB / WAVES;        // A rows DMA'd per wave
+    static constexpr int ROWS_PER_WAVE_B = TBN / WAVES;     // B rows DMA'd per wave
     static constexpr int DMA_PER_WAVE = ROWS_PER_WAVE / 8;  // 1 KiB DMA instructions
-    static_assert(ROWS_PER_WAVE % 8 == 0, "whole 1 KiB DMA groups per wave");
+    static constexpr int DMA_PER_STAGE = (ROWS_PER_WAVE + ROWS_PER_WAVE_B) / 8;
+    static_assert(ROWS_PER_WAVE % 8 == 0 && ROWS_PER_WAVE_B % 8 == 0, "whole 1 KiB DMA groups per wave");
 };
 
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -421,10 +426,9 @@ struct DmaOperand<true> {
 
 // Interior operand: tile rows r0 .. r0+255 of a row-major operand with
 // leading dimension ld (bytes), starting at byte `tile_off` of the buffer.
-template <class C>
+template <class C, int ROWS_PER_WAVE = C::ROWS_PER_WAVE>
 __device__ __forceinline__ DmaOperand<false> make_dma_interior(const int8_t *base, uint32_t bytes,
                                                                int ld, int tile_off) {
-    constexpr int ROWS_PER_WAVE = C::ROWS_PER_WAVE;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     DmaOperand<false> d;
     d.rsrc = make_rsrc(base, bytes);
@@ -521,24 +525,22 @@ inline int last_rows_pass(int M, int N, int limit) {
     return rem;
 }
 
-template <class C>
+template <class C, int ROWS_PER_WAVE>
 __device__ __forceinline__ void dma_operand(int8_t *dst, const DmaOperand<false> &d, int kbyte) {
-    constexpr int ROWS_PER_WAVE = C::ROWS_PER_WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-    for (int i = 0; i < C::DMA_PER_WAVE; ++i) {
+    for (int i = 0; i < ROWS_PER_WAVE / 8; ++i) {
         const int soff = __builtin_amdgcn_readfirstlane(kbyte + i * d.row_stride);
         dma16(d.rsrc, (i & 1) ? d.odd : d.even, soff, dst + (wave * ROWS_PER_WAVE + i * 8) * BK);
     }
 }
 
-template <class C>
+template <class C, int ROWS_PER_WAVE>
 __device__ __forceinline__ void dma_operand(int8_t *dst, const DmaOperand<true> &d, int kbyte) {
-    constexpr int ROWS_PER_WAVE = C::ROWS_PER_WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int soff = __builtin_amdgcn_readfirstlane(kbyte);
 #pragma unroll
-    for (int i = 0; i < C::DMA_PER_WAVE; ++i) dma16(d.rsrc, d.off[i], soff, dst + (wave * ROWS_PER_WAVE + i * 8) * BK);
+    for (int i = 0; i < ROWS_PER_WAVE / 8; ++i) dma16(d.rsrc, d.off[i], soff, dst + (wave * ROWS_PER_WAVE + i * 8) * BK);
 }
 
 // Row-major B operand ([K, N], leading dimension ld): one DMA instruction
@@ -569,7 +571,7 @@ __device__ __forceinline__ DmaOperandRowB make_dma_row_b(const int8_t *base, uin
     return d;
 }
 
-template <class C>
+template <class C, int>
 __device__ __forceinline__ void dma_operand(int8_t *dst, const DmaOperandRowB &d, int kbyte) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
@@ -592,18 +594,58 @@ struct DmaRows {
 
 template <class C, class D>
 __device__ __forceinline__ void dma_stage(int8_t *stage, const D &d, int kbyte) {
-    dma_operand<C>(stage, d.a, kbyte);
-    dma_operand<C>(stage + C::OPER, d.b, kbyte);
+    dma_operand<C, C::ROWS_PER_WAVE>(stage, d.a, kbyte);
+    dma_operand<C, C::ROWS_PER_WAVE_B>(stage + C::OPER, d.b, kbyte);
+}
+
+// K not a multiple of BK (but of 16): in the last stage, which starts at
+// byte `kbyte` of K, the 16-byte units at or past K would read the next row.
+// Their lanes get an offset past every extent the DMA path accepts (below
+// 2^31), so they land as zeros.
+constexpr int kPastExtent = 0x7ffffff0;
+
+template <class C, int ROWS_PER_WAVE>
+__device__ __forceinline__ void mask_tail(DmaOperand<false> &d, int kbyte, int K) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int u0 = (lane & 7) ^ swz(wave * ROWS_PER_WAVE + (lane >> 3));
+    if (kbyte + u0 * 16 >= K) d.even = kPastExtent;
+    if (kbyte + (u0 ^ 4) * 16 >= K) d.odd = kPastExtent;
+}
+
+template <class C, int ROWS_PER_WAVE>
+__device__ __forceinline__ void mask_tail(DmaOperand<true> &d, int kbyte, int K) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < ROWS_PER_WAVE / 8; ++i) {
+        const int u = (lane & 7) ^ swz(wave * ROWS_PER_WAVE + i * 8 + (lane >> 3));
+        if (kbyte + u * 16 >= K) d.off[i] = kPastExtent;
+    }
+}
+
+// Row-major B: k-rows at or past K lie past the extent (K * ld bytes).
+template <class C, int>
+__device__ __forceinline__ void mask_tail(DmaOperandRowB &, int, int) {}
+
+// Masks both operands when the stage at byte `kbyte` is a partial last one.
+template <class C, class D>
+__device__ __forceinline__ void mask_stage(D &d, int kbyte, int K) {
+    if (kbyte + BK > K) {
+        mask_tail<C, C::ROWS_PER_WAVE>(d.a, kbyte, K);
+        mask_tail<C, C::ROWS_PER_WAVE_B>(d.b, kbyte, K);
+    }
 }
 
 // One stage: compute from `cur`, stream the next stage into `nxt` (if any).
 template <class P, class D>
 __device__ __forceinline__ void stage_step(AccTile<P> &acc, Frags<P> &f0, Frags<P> &f1,
-                                           const int8_t *cur, int8_t *nxt, const D &d, int next_k,
+                                           const int8_t *cur, int8_t *nxt, D &d, int next_k, int K,
                                            bool has_next, int wave_m, int wave_n, int lane,
                                            typename P::Sums &sums) {
     typedef typename P::Cfg C;
-    if (has_next) dma_stage<C>(nxt, d, next_k);
+    if (has_next) {
+        mask_stage<C>(d, next_k, K);
+        dma_stage<C>(nxt, d, next_k);
+    }
     load_frags<P>(f0, cur, 0, wave_m, wave_n, lane);
     if constexpr (P::FLIP) P::fixup(f0, sums);
     mma_block<P, 0, P::TJ>(acc, f0);
@@ -622,7 +664,7 @@ __device__ __forceinline__ void stage_step(AccTile<P> &acc, Frags<P> &f0, Frags<
 // Full K loop for one 256x256 tile.  s0 / s1 are the two stage buffers
 // (each 2 * OPER bytes: A then B).  Ends with a barrier.
 template <class P, class D>
-__device__ __forceinline__ void mainloop(int8_t *s0, int8_t *s1, const D &d, int K, AccTile<P> &acc,
+__device__ __forceinline__ void mainloop(int8_t *s0, int8_t *s1, D d, int K, AccTile<P> &acc,
                                          typename P::Sums &sums) {
     typedef typename P::Cfg C;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -632,17 +674,18 @@ __device__ __forceinline__ void mainloop(int8_t *s0, int8_t *s1, const D &d, int
 #pragma unroll
         for (int j = 0; j < P::TJ; ++j) acc[i][j] = P::zero();
 
-    const int KT = K / BK;
+    const int KT = (K + BK - 1) / BK;
     Frags<P> f0, f1;
+    mask_stage<C>(d, 0, K);
     dma_stage<C>(s0, d, 0);
     wait_dma();
     __syncthreads();
     int kt = 0;
     for (; kt + 2 <= KT; kt += 2) {
-        stage_step<P>(acc, f0, f1, s0, s1, d, (kt + 1) * BK, true, wave_m, wave_n, lane, sums);
-        stage_step<P>(acc, f0, f1, s1, s0, d, (kt + 2) * BK, kt + 2 < KT, wave_m, wave_n, lane, sums);
+        stage_step<P>(acc, f0, f1, s0, s1, d, (kt + 1) * BK, K, true, wave_m, wave_n, lane, sums);
+        stage_step<P>(acc, f0, f1, s1, s0, d, (kt + 2) * BK, K, kt + 2 < KT, wave_m, wave_n, lane, sums);
     }
-    if (kt < KT) stage_step<P>(acc, f0, f1, s0, s1, d, 0, false, wave_m, wave_n, lane, sums);
+    if (kt < KT) stage_step<P>(acc, f0, f1, s0, s1, d, 0, K, false, wave_m, wave_n, lane, sums);
 }
 
 template <class P, class D>
@@ -656,17 +699,22 @@ __device__ __forceinline__ void mainloop(int8_t *s0, int8_t *s1, const D &d, int
 // MFMAs, for a wave whose output rows are all padding: it still moves its
 // share of every stage and meets every barrier of the waves that compute.
 template <class C, class D>
-__device__ __forceinline__ void mainloop_dma_only(int8_t *s0, int8_t *s1, const D &d, int K) {
-    const int KT = K / BK;
+__device__ __forceinline__ void mainloop_dma_only(int8_t *s0, int8_t *s1, D d, int K) {
+    const int KT = (K + BK - 1) / BK;
+    mask_stage<C>(d, 0, K);
     dma_stage<C>(s0, d, 0);
     wait_dma();
     __syncthreads();
     int kt = 0;
     for (; kt + 2 <= KT; kt += 2) {
+        mask_stage<C>(d, (kt + 1) * BK, K);
         dma_stage<C>(s1, d, (kt + 1) * BK);
         wait_dma();
         __syncthreads();
-        if (kt + 2 < KT) dma_stage<C>(s0, d, (kt + 2) * BK);
+        if (kt + 2 < KT) {
+            mask_stage<C>(d, (kt + 2) * BK, K);
+            dma_stage<C>(s0, d, (kt + 2) * BK);
+        }
         wait_dma();
         __syncthreads();
     }
@@ -674,6 +722,14 @@ __device__ __forceinline__ void mainloop_dma_only(int8_t *s0, int8_t *s1, const 
         wait_dma();
         __syncthreads();
     }
+}
+
+// This wave's WM * 128 bytes of two stage buffers that are free again.
+template <class C>
+__device__ __forceinline__ int8_t *wave_scratch(int8_t *s0, int8_t *s1) {
+    static_assert(C::WM * 128 * C::WAVES / 2 <= C::STAGE, "scratch of half the waves per stage buffer");
+    const int wave = threadIdx.x >> 6;
+    return (wave < C::WAVES / 2 ? s0 : s1) + (wave % (C::WAVES / 2)) * (C::WM * 128);
 }
 
 // W8A8 bf16 epilogue for the int8 16x16 policy, staged through LDS so each
@@ -770,21 +826,22 @@ __device__ __forceinline__ void store_u8x4_staged(const AccTile<P> &acc, int8_t 
 // 32-bit outputs of a policy whose wave tile is WN = 64 columns (256-byte
 // rows): each quad (4 columns of one row) is packed to 16 bytes by
 // pack(r, c, quad) and the wave tile staged in LDS in two halves of WM / 2
-// rows (`scratch`: WM / 2 * 256 bytes private to this wave; unit u of row r
-// at unit u ^ (r & 15)), each half's rows written as 16-byte units, four
-// rows of 256 bytes per store instruction.  row_dst(r) gives row r's
-// destination (nullptr: skip); ncols: valid columns (a multiple of 4).
+// rows (one 16-row tile at a time when TI is odd; `scratch`: 256 bytes per
+// staged row, private to this wave; unit u of row r at unit u ^ (r & 15)),
+// each part's rows written as 16-byte units, four rows of 256 bytes per
+// store instruction.  row_dst(r) gives row r's destination (nullptr: skip);
+// ncols: valid columns (a multiple of 4).
 template <class P, class Pack, class RowDst>
 __device__ __forceinline__ void store_x32x4_staged(const AccTile<P> &acc, int8_t *scratch, Pack &&pack,
                                                    RowDst &&row_dst, int ncols = P::Cfg::WN) {
     typedef typename P::Cfg C;
-    static_assert(C::WN == 64 && P::TI % 2 == 0, "staged 32-bit store assumes 256-byte wave-tile rows");
-    constexpr int HALF = C::WM / 2;
+    static_assert(C::WN == 64, "staged 32-bit store assumes 256-byte wave-tile rows");
+    constexpr int NCH = P::TI % 2 == 0 ? 2 : P::TI, HALF = C::WM / NCH;
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < NCH; ++h) {
 #pragma unroll
-        for (int i = h * (P::TI / 2); i < (h + 1) * (P::TI / 2); ++i)
+        for (int i = h * (P::TI / NCH); i < (h + 1) * (P::TI / NCH); ++i)
 #pragma unroll
             for (int j = 0; j < P::TJ; ++j)
                 P::visit(acc[i][j], i, j, lane, [&](int r, int c, const auto &v) {
@@ -812,23 +869,24 @@ __device__ __forceinline__ void store_x32x4_staged(const AccTile<P> &acc, int8_t
 // 64-bit outputs of the int8 16x16 policy (WN = 64 columns, 512-byte rows):
 // each quad is packed to 32 bytes by pack(r, c, quad) -> {lo, hi} (columns
 // c, c+1 and c+2, c+3) and the wave tile staged in LDS in four quarters of
-// WM / 4 rows (`scratch`: WM / 4 * 512 bytes private to this wave; 16-byte
-// unit u of row r at unit u ^ (r & 15)), two 512-byte rows per store
-// instruction.  row_dst(r): row r's destination (nullptr: skip); ncols:
-// valid columns (a multiple of 2).
+// WM / 4 rows (one 16-row tile at a time when TI is no multiple of 4;
+// `scratch`: 512 bytes per staged row, private to this wave; 16-byte unit u
+// of row r at unit u ^ (r & 15)), two 512-byte rows per store instruction.
+// row_dst(r): row r's destination (nullptr: skip); ncols: valid columns (a
+// multiple of 2).
 struct Quad64 { v4i lo, hi; };
 
 template <class P, class Pack, class RowDst>
 __device__ __forceinline__ void store_x64x4_staged(const AccTile<P> &acc, int8_t *scratch, Pack &&pack,
                                                    RowDst &&row_dst, int ncols = P::Cfg::WN) {
     typedef typename P::Cfg C;
-    static_assert(C::WN == 64 && P::TI % 4 == 0, "staged 64-bit store assumes 512-byte wave-tile rows");
-    constexpr int QR = C::WM / 4;
+    static_assert(C::WN == 64, "staged 64-bit store assumes 512-byte wave-tile rows");
+    constexpr int NCH = P::TI % 4 == 0 ? 4 : P::TI, QR = C::WM / NCH;
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
+    for (int h = 0; h < NCH; ++h) {
 #pragma unroll
-        for (int i = h * (P::TI / 4); i < (h + 1) * (P::TI / 4); ++i)
+        for (int i = h * (P::TI / NCH); i < (h + 1) * (P::TI / NCH); ++i)
 #pragma unroll
             for (int j = 0; j < P::TJ; ++j)
                 P::visit(acc[i][j], i, j, lane, [&](int r, int c, const auto &v) {

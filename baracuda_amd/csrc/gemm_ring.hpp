@@ -1,0 +1,175 @@
+// gemm_ring.hpp -- mid-size block tiles for the RCR GEMMs: a ring of LDS
+// stages with the next stage's DMA spread between the MFMAs, and the rule
+// that picks the tile.
+//
+// What bounds these tiles (int8, one box): one 1 KiB LDS-DMA instruction
+// takes a CU about 26 clocks, so a 128 x 128 stage's 32 take as long as
+// 830 clocks of the 512 its MFMAs need, and a wave that issues its DMAs in
+// one burst stalls in front of its MFMAs for all of that.  Reading the
+// stage's fragments first and issuing one DMA per few MFMAs overlaps the
+// two: 1024 x 4096 x 4096 on 256 tiles of 128 x 128, 23.5 us with the burst
+// ahead of the fragment reads, 21.0 with the burst behind them, 19.1 spread
+// (26.5 us for the two-stage loop of gemm_mfma2.hpp).  A third stage hides
+// the load latency of a tile that has the CU to itself; a fourth gives
+// nothing more (19.2 us).
+#pragma once
+
+#include "gemm_mfma2.hpp"
+
+namespace bk {
+namespace mfma2 {
+
+// One DMA instruction of a stage: I < ROWS_PER_WAVE / 8 moves A row group I,
+// the others B row groups.
+template <class C, int I>
+__device__ __forceinline__ void dma_piece(int8_t *stage, const DmaRows<false, false> &d, int kbyte) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int NA = C::ROWS_PER_WAVE / 8;
+    if constexpr (I < NA) {
+        const int soff = __builtin_amdgcn_readfirstlane(kbyte + I * d.a.row_stride);
+        dma16(d.a.rsrc, (I & 1) ? d.a.odd : d.a.even, soff, stage + (wave * C::ROWS_PER_WAVE + I * 8) * BK);
+    } else {
+        constexpr int J = I - NA;
+        const int soff = __builtin_amdgcn_readfirstlane(kbyte + J * d.b.row_stride);
+        dma16(d.b.rsrc, (J & 1) ? d.b.odd : d.b.even, soff,
+              stage + C::OPER + (wave * C::ROWS_PER_WAVE_B + J * 8) * BK);
+    }
+}
+
+template <class C, int I0, int I1, class D>
+__device__ __forceinline__ void dma_pieces(int8_t *stage, const D &d, int kbyte) {
+    if constexpr (I0 < I1) {
+        dma_piece<C, I0>(stage, d, kbyte);
+        dma_pieces<C, I0 + 1, I1>(stage, d, kbyte);
+    }
+}
+
+// MFMA t of a stage's two sub-steps, then the DMA pieces due after it.
+template <class P, int T, int SPREAD, class D>
+__device__ __forceinline__ void ring_mma(AccTile<P> &acc, const Frags<P> &f0, const Frags<P> &f1, int8_t *nxt, const D &d,
+                                         int kbyte) {
+    typedef typename P::Cfg C;
+    constexpr int SUB = P::H * P::TI * P::TJ, TOT = 2 * SUB, NI = C::DMA_PER_STAGE;
+    if constexpr (T < TOT) {
+        constexpr int r = T % SUB, h = r / (P::TI * P::TJ), j = r / P::TI % P::TJ, i = r % P::TI;
+        const Frags<P> &f = T < SUB ? f0 : f1;
+        P::mma(acc[i][j], f.b[j], f.a[i], h);
+        constexpr int p0 = (T / SPREAD < NI ? T / SPREAD : NI);
+        constexpr int p1 = ((T + 1) / SPREAD < NI ? (T + 1) / SPREAD : NI);
+        constexpr int pe = T + 1 == TOT ? NI : p1;
+        if constexpr (pe > p0) {
+            __builtin_amdgcn_sched_barrier(0);
+            dma_pieces<C, p0, pe>(nxt, d, kbyte);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ring_mma<P, T + 1, SPREAD>(acc, f0, f1, nxt, d, kbyte);
+    }
+}
+
+// K loop over a ring of DEPTH stage buffers at `lds` (DEPTH * C::STAGE bytes,
+// 1 KiB aligned), DEPTH - 1 stages in flight: the wait for stage kt leaves
+// the later stages' DMAs outstanding (they complete in issue order), and the
+// one barrier per stage both publishes stage kt and frees the buffer of
+// stage kt - 1 for the DMA of stage kt + DEPTH - 1.  Ends with a barrier.
+template <class P, int DEPTH, int SPREAD, class D>
+__device__ __forceinline__ void mainloop_ring(int8_t *lds, D d, int K, AccTile<P> &acc) {
+    typedef typename P::Cfg C;
+    static_assert(DEPTH >= 2 && DEPTH <= 4 && DEPTH * C::STAGE <= 160 * 1024, "stage ring");
+    static_assert(!P::SUMS && !P::FLIP, "the ring loop takes signed and float operands");
+    constexpr int NI = C::DMA_PER_STAGE;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wave_m = wave / C::WAVES_N, wave_n = wave % C::WAVES_N;
+#pragma unroll
+    for (int i = 0; i < P::TI; ++i)
+#pragma unroll
+        for (int j = 0; j < P::TJ; ++j) acc[i][j] = P::zero();
+    const int KT = (K + BK - 1) / BK;
+    Frags<P> f0, f1;
+    auto prep = [&](int kt) {
+        if ((kt + 1) * BK > K) {
+            if (kt >= KT) {
+                d.a.rsrc[2] = 0;
+                d.b.rsrc[2] = 0;
+            } else {
+                mask_tail<C, C::ROWS_PER_WAVE>(d.a, kt * BK, K);
+                mask_tail<C, C::ROWS_PER_WAVE_B>(d.b, kt * BK, K);
+            }
+        }
+    };
+    for (int s = 0; s < DEPTH - 1; ++s) {
+        prep(s);
+        dma_stage<C>(lds + s * C::STAGE, d, s * BK);
+    }
+    int cur = 0, nxt = (DEPTH - 1) * C::STAGE;       // byte offsets of the ring slots
+    for (int kt = 0; kt < KT; ++kt) {
+        prep(kt + DEPTH - 1);
+        wait_vmcnt<(DEPTH - 2) * NI>();
+        __syncthreads();
+        const int8_t *st = lds + cur;
+        load_frags<P>(f0, st, 0, wave_m, wave_n, lane);
+        load_frags<P>(f1, st, 1, wave_m, wave_n, lane);
+        if constexpr (SPREAD == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            dma_pieces<C, 0, NI>(lds + nxt, d, (kt + DEPTH - 1) * BK);
+            __builtin_amdgcn_sched_barrier(0);
+            mma_block<P, 0, P::TJ>(acc, f0);
+            mma_block<P, 0, P::TJ>(acc, f1);
+        } else {
+            ring_mma<P, 0, SPREAD>(acc, f0, f1, lds + nxt, d, (kt + DEPTH - 1) * BK);
+        }
+        nxt = cur;
+        cur = cur + C::STAGE == DEPTH * C::STAGE ? 0 : cur + C::STAGE;
+    }
+    wait_dma();
+    __syncthreads();
+}
+
+// ---- which tile -------------------------------------------------------------
+// Tiles of the RCR GEMMs.  The first four run the ring loop (LDS of all
+// stages; 64-row tiles leave room for two workgroups per CU), the last is the
+// 256 x 256 kernel of gemm_mfma2.hpp.
+enum RingTile { RT_64x64, RT_64x128, RT_128x128, RT_128x256, RT_192x256, RT_256x256 };
+struct RingCost {
+    int tm, tn;
+    float stage;    // us per 128-byte stage of K, alone on its CU
+    float paired;   // ... of two workgroups sharing a CU (0: LDS holds one)
+    float fixed;    // us per round besides: launch, first loads, epilogue
+};
+// Measured over K = 1024 .. 8000 (int8, bf16 out, weights from HBM).
+constexpr RingCost kRingCost[] = {
+    {64, 64, 0.20f, 0.39f, 3.6f},   {64, 128, 0.30f, 0.56f, 3.9f},  {128, 128, 0.47f, 0.0f, 3.5f},
+    {128, 256, 0.65f, 0.0f, 5.1f},  {192, 256, 1.00f, 0.0f, 5.8f},  {256, 256, 1.23f, 0.0f, 6.7f},
+};
+
+// Time of one tile shape: rounds over the 256 CUs, each of `fixed` plus the
+// K stages.  The figures rank the shapes; a full chip is slower than they
+// say (power), all shapes alike.  Picks, against the best of the six measured
+// (us): 777 x 11008 x 4096 192x256 47.3 (256x256 49.4, 128x128 51.8), 1500 x
+// 5120 x 2880 128x256 23.7 (192x256 31.6, 128x128 28.9), 810 x 2352 x 1856
+// 64x128 9.3 (128x128 10.9), 200 x 11008 x 4096 128x128 20.3 (64x128 24.3),
+// 3072 x 4096 x 4096 192x256 44.3 (256x256 47.0), 4096^3 256x256 55.5.
+inline float ring_cost(const RingCost &c, int M, int N, int kbytes) {
+    const int64_t tiles = (int64_t)((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn);
+    const float kt = (float)((kbytes + BK - 1) / BK);
+    const int64_t per_cu = (tiles + 255) / 256;
+    if (c.paired == 0.0f) return (float)per_cu * (c.fixed + kt * c.stage);
+    const int64_t pairs = per_cu / 2;
+    return (float)pairs * (c.fixed + kt * c.paired) + (float)(per_cu % 2) * (c.fixed + kt * c.stage);
+}
+
+inline RingTile ring_tile(int M, int N, int kbytes, float *cost = nullptr) {
+    int best = 0;
+    float us = 0.0f;
+    for (int i = 0; i <= RT_256x256; ++i) {
+        const float t = ring_cost(kRingCost[i], M, N, kbytes);
+        if (i == 0 || t < us) {
+            best = i;
+            us = t;
+        }
+    }
+    if (cost) *cost = us;
+    return (RingTile)best;
+}
+
+}  // namespace mfma2
+}  // namespace bk

@@ -17,7 +17,7 @@
 #include <type_traits>
 
 #include "gemm_mfma.hpp"
-#include "gemm_mfma2.hpp"
+#include "gemm_ring.hpp"
 #include "act.hpp"
 
 namespace bk {
@@ -215,29 +215,24 @@ struct TailSplit {
     int split;        // K chunks per tail tile (1: no split)
 };
 
-// Last rows of M run by gemm_s8_rcr_rows_kernel instead of a row of
-// 256-row tiles (N % 16 == 0): M % 256 in [1, kRowsPathMax] (all of M when
-// M <= kRowsPathMax: no tiles at all), when that row of tiles would start
-// another round of tiles on the 256 CUs (it costs nothing extra when it
-// fits the idle CUs of the last round).  Up to kRowsPathAlways rows always;
-// up to kRowsPathMax when K % kRowsStagedSB == 0 (the staged last-rows
-// kernel), otherwise only when no tail-split workspace is given.  At
-// N = K = 4096 the staged pass beats the split tail round and its reduction:
-// M = 100 / 128 / 4196 in 11.9 / 12.8 / 66.1 us against 22.3 / 23.0 / 71.0.
+// Last rows of M run by a last-rows launch instead of a row of 256-row tiles
+// (N % 16 == 0): M % 256 in [1, kRowsPathMax] (all of M when M <=
+// kRowsPathMax: no tiles at all), when that row of tiles would start
+// another round of tiles on the 256 CUs (it costs nothing extra when it fits
+// the idle CUs of the last round).  A tail-split workspace is reported for
+// more than kRowsPathAlways of them when K is no multiple of kRowsStagedSB.
+// At N = K = 4096 the staged pass beats the split tail round and its
+// reduction: M = 100 / 128 / 4196 in 11.9 / 12.8 / 66.1 us against 22.3 /
+// 23.0 / 71.0.
 constexpr int kRowsPathMax = 128;
 constexpr int kRowsPathAlways = 64;
-constexpr int kRowsStagedSB = 512, kRowsStagedDepth = 2;
+constexpr int kRowsStagedSB = 512;
 inline int rows_path_rows(int M, int N, int limit = kRowsPathMax) { return mfma2::last_rows_pass(M, N, limit); }
 
 // Grids of at most kSmallTilesMax 256 x 256 tiles (under half a round on
-// the 256 CUs) run 128 x 128 tiles instead (Cfg<2, 2, 128>: 4 waves of
-// 64 x 64, two workgroups per CU), except that with a tail-split workspace
-// a deep K (>= 4096) on fewer than 64 small tiles splits K.  W8A8, N = K =
-// 4096, 8 rotated weight sets, no workspace: M = 256 / 512 / 1024 / 2048
-// 56 / 56 / 56 / 55 -> 24.2 / 24.9 / 26.7 / 36.0 us (the split workspace:
-// 29.9 / 32.2 / 38.2 / 52.0); 129-255 tiles stay on 256 x 256 (M = 2560 /
-// 3072: 46.5 / 49.6 us against 55.1 / 59.2 with small tiles).  512 x 512 x
-// 8192: small tiles 43.6 us, split 30.5.
+// the 256 CUs) run smaller tiles, except that with a tail-split workspace a
+// deep K (>= 4096) on fewer than 64 tiles of 128 x 128 splits K (512 x 512 x
+// 8192: 30.5 us against 43.6 on 128 x 128 tiles of two stages).
 constexpr int kSmallTilesMax = 128;
 inline bool small_tiles_preferred(int M, int N, int K) {
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
@@ -274,24 +269,23 @@ inline bool dma_extent_ok(int rows, int64_t ld) {
     return ((int64_t)(rows + 255) / 256) * 256 * ld < (1ll << 31);
 }
 
-// Fast path: 256x256 tiles (edge tiles read zeros past M / N), K % 128 == 0,
-// 16-byte aligned rows ->
+// Fast path: 256x256 tiles (edge tiles read zeros past M / N, a partial last
+// stage past K), K % 16 == 0, 16-byte aligned rows ->
 // LDS-DMA mainloop, 8 waves (2 x 4) of 128 x 64, v_mfma_i32_16x16x64_i8.
 typedef mfma2::Cfg<2, 4> DmaCfg;
 
-// int8 outputs of a whole tile through LDS: each wave's 128 x 64 bytes are
-// staged (8 KiB per wave; LDS is free after the mainloop's last barrier) and
+// int8 outputs of a whole tile through LDS: each wave's WM x 64 bytes are
+// staged in its scratch (LDS is free after the mainloop's last barrier) and
 // written as 16-byte row segments instead of 4-byte stores.
 // Partial tiles (the M / N edge, N % 16 == 0): rows past M and 16-byte
 // units past N are neither computed nor stored.
 template <class P, bool HasC, bool Full, class Epi>
-__device__ __forceinline__ void store_s8_tile_staged_as(const mfma2::AccTile<P> &acc, int8_t *stage0, int8_t *stage1,
+__device__ __forceinline__ void store_s8_tile_staged_as(const mfma2::AccTile<P> &acc, int8_t *scratch,
                                                         const S8Args &p, int m_base, int n_base, const Epi &epi) {
     typedef typename P::Cfg C;
     const int wave = threadIdx.x >> 6;
     const int wrow = (wave / C::WAVES_N) * C::WM;
     const int wcol = (wave % C::WAVES_N) * C::WN;
-    int8_t *scratch = (wave < C::WAVES / 2 ? stage0 : stage1) + (wave % (C::WAVES / 2)) * (C::WM * C::WN);
     const int ncols = min(C::WN, p.N - (n_base + wcol));
     mfma2::store_u8x4_staged<P>(
         acc, scratch,
@@ -311,60 +305,28 @@ __device__ __forceinline__ void store_s8_tile_staged_as(const mfma2::AccTile<P> 
 // The C term and the M / N bounds decided once per tile (full: whole tile
 // in range), not per element.
 template <class P, class Epi>
-__device__ __forceinline__ void store_s8_tile_staged(const mfma2::AccTile<P> &acc, int8_t *stage0, int8_t *stage1,
+__device__ __forceinline__ void store_s8_tile_staged(const mfma2::AccTile<P> &acc, int8_t *scratch,
                                                      const S8Args &p, int m_base, int n_base, const Epi &epi) {
     const bool has_c = p.beta != 0.0f && p.c != nullptr;
-    const bool full = m_base + P::Cfg::TB <= p.M && n_base + P::Cfg::TB <= p.N;
+    const bool full = m_base + P::Cfg::TB <= p.M && n_base + P::Cfg::TBN <= p.N;
     if (has_c) {
-        if (full) store_s8_tile_staged_as<P, true, true>(acc, stage0, stage1, p, m_base, n_base, epi);
-        else store_s8_tile_staged_as<P, true, false>(acc, stage0, stage1, p, m_base, n_base, epi);
+        if (full) store_s8_tile_staged_as<P, true, true>(acc, scratch, p, m_base, n_base, epi);
+        else store_s8_tile_staged_as<P, true, false>(acc, scratch, p, m_base, n_base, epi);
     } else {
-        if (full) store_s8_tile_staged_as<P, false, true>(acc, stage0, stage1, p, m_base, n_base, epi);
-        else store_s8_tile_staged_as<P, false, false>(acc, stage0, stage1, p, m_base, n_base, epi);
+        if (full) store_s8_tile_staged_as<P, false, true>(acc, scratch, p, m_base, n_base, epi);
+        else store_s8_tile_staged_as<P, false, false>(acc, scratch, p, m_base, n_base, epi);
     }
 }
 
-// `ts`: workgroups below ts.full_tiles (all of them when ts.split == 1) run
-// whole tiles; the rest run K chunks of the tail tiles (tail_split_plan) and
-// store their accumulators in `slots`.
-template <int EPI, bool VecOut, int ACT = ACT_NONE, typename BiasT = float, class C = DmaCfg>
-__global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_rcr_dma_kernel(S8Args p, TailSplit ts,
-                                                                         int32_t *__restrict__ slots) {
+// Epilogue of a tile of any policy configuration: the staged stores where D
+// allows them, else 4-column quads.  `scratch`: this wave's part of the LDS
+// that the loop left (see the staged stores).
+template <int EPI, bool VecOut, int ACT, typename BiasT, class P>
+__device__ __forceinline__ void s8_store_tile(const mfma2::AccTile<P> &acc, int8_t *scratch, const S8Args &p, int m_base,
+                                              int n_base) {
     namespace M2 = mfma2;
-    typedef M2::PolicyI8<C> P;
-    __shared__ __attribute__((aligned(1024))) int8_t stage0[2 * C::OPER];
-    __shared__ __attribute__((aligned(1024))) int8_t stage1[2 * C::OPER];
-    // Edge tiles (M or N not a multiple of 256): operand rows past M / N
-    // lie past the buffer resources' byte counts and load as zeros.
-    const int tiles_n = (p.N + C::TB - 1) / C::TB;
-    int tm, tn, k0 = 0, klen = p.K, chunk = -1;
-    if (ts.split > 1 && (int)blockIdx.x >= ts.full_tiles) {
-        const int u = blockIdx.x - ts.full_tiles, ti = u / ts.split;
-        chunk = u % ts.split;
-        tm = ts.full_tiles / tiles_n + ti / tiles_n;
-        tn = ti % tiles_n;
-        const int kt = p.K / M2::BK;
-        k0 = chunk * kt / ts.split * M2::BK;
-        klen = (chunk + 1) * kt / ts.split * M2::BK - k0;
-    } else {
-        const int tiles_m = ts.split > 1 ? ts.full_tiles / tiles_n : (p.M + C::TB - 1) / C::TB;
-        tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    }
-    const int m_base = tm * C::TB, n_base = tn * C::TB;
-    M2::DmaRows<false, false> d;
-    d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda + k0);
-    d.b = M2::make_dma_interior<C>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb + k0);
-    M2::AccTile<P> acc;
-    M2::mainloop<P>(stage0, stage1, d, klen, acc);
-    if (chunk >= 0) {
-        // this chunk's int32 accumulators -> its slot (rows / columns in range)
-        int32_t *slot = slots + ((int64_t)(blockIdx.x - ts.full_tiles)) * 65536;
-        M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4i &v) {
-            if (m_base + ml < p.M && n_base + nl < p.N) *reinterpret_cast<v4i *>(slot + ml * 256 + nl) = v;
-        });
-        return;
-    }
-    const bool full = m_base + C::TB <= p.M && n_base + C::TB <= p.N;
+    typedef typename P::Cfg C;
+    const bool full = m_base + C::TB <= p.M && n_base + C::TBN <= p.N;
     if constexpr (EPI == EPI_W8A8_BF16 && VecOut) {
         if (full || p.N % 8 == 0) {
             // Scales fetched once per lane, output staged in LDS (free after the
@@ -382,7 +344,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_rcr_dma_k
                 const int col = wcol + j * 16 + (lane >> 4) * 4;
                 swv[j] = col < p.N ? *reinterpret_cast<const v4f *>(p.sw + col) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
             }
-            int8_t *scratch = (wave < C::WAVES / 2 ? stage0 : stage1) + (wave % (C::WAVES / 2)) * (C::WM * C::WN * 2);
             M2::store_w8a8_bf16_staged<P, false>(
                 acc, scratch, sam, none, swv,
                 [&](int r) {
@@ -399,7 +360,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_rcr_dma_k
             const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
             const int wrow = m_base + (wave / C::WAVES_N) * C::WM;
             const int wcol = n_base + (wave % C::WAVES_N) * C::WN;
-            int8_t *scratch = (wave < C::WAVES / 2 ? stage0 : stage1) + (wave % (C::WAVES / 2)) * (C::WM / 2 * 256);
             auto row_dst = [&](int r) {
                 return wrow + r < p.M ? static_cast<int32_t *>(p.d) + (int64_t)(wrow + r) * p.ldd + wcol : nullptr;
             };
@@ -440,7 +400,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_rcr_dma_k
             const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
             const int wrow = m_base + (wave / C::WAVES_N) * C::WM;
             const int wcol = n_base + (wave % C::WAVES_N) * C::WN;
-            int8_t *scratch = (wave < C::WAVES / 2 ? stage0 : stage1) + (wave % (C::WAVES / 2)) * (C::WM / 4 * 512);
             const double *sa64 = reinterpret_cast<const double *>(p.sa);
             const double *sw64 = reinterpret_cast<const double *>(p.sw);
             float sam[P::TI], swf[P::TJ][4];
@@ -475,12 +434,76 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_rcr_dma_k
         const S8Epilogue<EPI, VecOut, ACT, BiasT> epi{p};
         if constexpr (EPI == EPI_S8 && VecOut) {
             if (p.ldd % 16 == 0 && (reinterpret_cast<uintptr_t>(p.d) & 15u) == 0 && (full || p.N % 16 == 0)) {
-                store_s8_tile_staged<P>(acc, stage0, stage1, p, m_base, n_base, epi);
+                store_s8_tile_staged<P>(acc, scratch, p, m_base, n_base, epi);
                 return;
             }
         }
         M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4i &v) { epi(m_base + ml, n_base + nl, v); });
     }
+}
+
+// `ts`: workgroups below ts.full_tiles (all of them when ts.split == 1) run
+// whole tiles; the rest run K chunks of the tail tiles (tail_split_plan) and
+// store their accumulators in `slots`.
+template <int EPI, bool VecOut, int ACT = ACT_NONE, typename BiasT = float>
+__global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_s8_rcr_dma_kernel(S8Args p, TailSplit ts,
+                                                                      int32_t *__restrict__ slots) {
+    namespace M2 = mfma2;
+    typedef DmaCfg C;
+    typedef M2::PolicyI8<C> P;
+    __shared__ __attribute__((aligned(1024))) int8_t stage0[2 * C::OPER];
+    __shared__ __attribute__((aligned(1024))) int8_t stage1[2 * C::OPER];
+    // Edge tiles (M or N not a multiple of 256): operand rows past M / N
+    // lie past the buffer resources' byte counts and load as zeros.
+    const int tiles_n = (p.N + C::TB - 1) / C::TB;
+    int tm, tn, k0 = 0, klen = p.K, chunk = -1;
+    if (ts.split > 1 && (int)blockIdx.x >= ts.full_tiles) {
+        const int u = blockIdx.x - ts.full_tiles, ti = u / ts.split;
+        chunk = u % ts.split;
+        tm = ts.full_tiles / tiles_n + ti / tiles_n;
+        tn = ti % tiles_n;
+        const int kt = p.K / M2::BK;
+        k0 = chunk * kt / ts.split * M2::BK;
+        klen = (chunk + 1) * kt / ts.split * M2::BK - k0;
+    } else {
+        const int tiles_m = ts.split > 1 ? ts.full_tiles / tiles_n : (p.M + C::TB - 1) / C::TB;
+        tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    }
+    const int m_base = tm * C::TB, n_base = tn * C::TB;
+    M2::DmaRows<false, false> d;
+    d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda + k0);
+    d.b = M2::make_dma_interior<C>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb + k0);
+    M2::AccTile<P> acc;
+    M2::mainloop<P>(stage0, stage1, d, klen, acc);
+    if (chunk >= 0) {
+        // this chunk's int32 accumulators -> its slot (rows / columns in range)
+        int32_t *slot = slots + ((int64_t)(blockIdx.x - ts.full_tiles)) * 65536;
+        M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4i &v) {
+            if (m_base + ml < p.M && n_base + nl < p.N) *reinterpret_cast<v4i *>(slot + ml * 256 + nl) = v;
+        });
+        return;
+    }
+    s8_store_tile<EPI, VecOut, ACT, BiasT, P>(acc, M2::wave_scratch<C>(stage0, stage1), p, m_base, n_base);
+}
+
+// The same GEMM on the tiles of gemm_ring.hpp: C's block tile over a ring of
+// DEPTH stages (dynamic LDS of DEPTH * C::STAGE bytes), SPREAD MFMAs per DMA.
+template <int EPI, bool VecOut, int ACT, typename BiasT, class C, int DEPTH, int SPREAD>
+__global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_rcr_ring_kernel(S8Args p) {
+    namespace M2 = mfma2;
+    typedef M2::PolicyI8<C> P;
+    constexpr int SCRATCH = DEPTH * C::STAGE / C::WAVES;   // bytes per wave after the loop
+    static_assert(SCRATCH >= C::WM * 128 && SCRATCH >= 16 * 512 && SCRATCH % 1024 == 0, "staged stores");
+    extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+    int tm, tn;
+    tile_coords(blockIdx.x, (p.M + C::TB - 1) / C::TB, (p.N + C::TBN - 1) / C::TBN, tm, tn);
+    const int m_base = tm * C::TB, n_base = tn * C::TBN;
+    M2::DmaRows<false, false> d;
+    d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
+    d.b = M2::make_dma_interior<C, C::ROWS_PER_WAVE_B>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb);
+    M2::AccTile<P> acc;
+    M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    s8_store_tile<EPI, VecOut, ACT, BiasT, P>(acc, lds + (threadIdx.x >> 6) * SCRATCH, p, m_base, n_base);
 }
 
 // Tail tiles of a split launch: a tile's K-chunk slots added in chunk order
@@ -506,83 +529,13 @@ __global__ __launch_bounds__(256) void gemm_s8_tail_reduce_kernel(S8Args p, Tail
     epi(m, n0, acc);
 }
 
-// The last M - m0 (<= kRowsPathMax) rows of an RCR GEMM whose other rows
-// run as whole 256-row tiles (K % 128 == 0, 16-byte aligned rows, N % 16 ==
-// 0).  A 256-row tile for them would stream its whole B panel at the pace of
-// a full tile; here one workgroup of 8 waves owns 16 output columns, the
-// waves split K into 8 contiguous runs of 64-byte chunks and stream their
-// 16 B rows and the (at most 16 RF) A rows straight from global memory, U
-// chunks in flight per batch, one v_mfma_i32_16x16x64_i8 per chunk and
-// 16-row fragment of A (B first, A second, both taking k = 64 c + 16
-// (lane / 16) + byte, so lane l ends with row m0 + 16 f + l % 16 and columns
-// 4 (l / 16) .. + 3 of its 16).  The eight partial sums are added in LDS
-// (int32 wrap-around, so the order does not matter) and go through the
-// tiles' epilogue.
-template <int EPI, bool VecOut, int ACT, typename BiasT, int RF>
-__global__ __launch_bounds__(512) void gemm_s8_rcr_rows_kernel(S8Args p, int m0) {
-    constexpr int U = RF == 1 ? 8 : RF <= 4 ? 4 : 2, WAVES = 8;
-    __shared__ v4i part[WAVES][RF][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r16 = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * 16;
-    const int8_t *arow[RF];
-#pragma unroll
-    for (int f = 0; f < RF; ++f) arow[f] = p.a + (int64_t)min(m0 + 16 * f + r16, p.M - 1) * p.lda + g * 16;
-    const int8_t *brow = p.b + (int64_t)(n0 + r16) * p.ldb + g * 16;
-    const int chunks = p.K >> 6;
-    v4i acc[RF];
-#pragma unroll
-    for (int f = 0; f < RF; ++f) acc[f] = v4i{0, 0, 0, 0};
-    // Wave w takes the contiguous chunks [c0, c1): 64 * (c1 - c0) bytes of
-    // each of its 16 B rows in one span.
-    const int c1 = (wave + 1) * chunks / WAVES;
-    int c = wave * chunks / WAVES;
-    for (; c + U <= c1; c += U) {
-        v4i bv[U], av[U][RF];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            bv[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(brow + (int64_t)(c + u) * 64));
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int f = 0; f < RF; ++f) av[u][f] = *reinterpret_cast<const v4i *>(arow[f] + (int64_t)(c + u) * 64);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int f = 0; f < RF; ++f) acc[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bv[u], av[u][f], acc[f], 0, 0, 0);
-    }
-    for (; c < c1; ++c) {
-        const v4i bv = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(brow + (int64_t)c * 64));
-#pragma unroll
-        for (int f = 0; f < RF; ++f) {
-            const v4i av = *reinterpret_cast<const v4i *>(arow[f] + (int64_t)c * 64);
-            acc[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bv, av, acc[f], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int f = 0; f < RF; ++f) part[wave][f][lane] = acc[f];
-    __syncthreads();
-    // wave w < RF adds up fragment w over the 8 waves
-    if (wave >= RF) return;
-    v4i sum = part[0][wave][lane];
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w) {
-        const v4i v = part[w][wave][lane];
-        sum = v4i{(int)((uint32_t)sum[0] + (uint32_t)v[0]), (int)((uint32_t)sum[1] + (uint32_t)v[1]),
-                  (int)((uint32_t)sum[2] + (uint32_t)v[2]), (int)((uint32_t)sum[3] + (uint32_t)v[3])};
-    }
-    const S8Epilogue<EPI, VecOut, ACT, BiasT> epi{p};
-    epi(m0 + 16 * wave + r16, n0 + 4 * g, sum);   // rows past M are not stored
-}
-
 template <bool VecOut, int ACT, typename BiasT>
 struct U8Epilogue;
 // Zero row / column sums for U8Epilogue when the correction is already in
 // the accumulator.
 __device__ const int kZeroSums[16] = {0};
 
-// One last row (M = 1 decode steps; K % (1024 BT) == 0): a workgroup of 4
+// One last row (M = 1 decode steps; K % 16 == 0, % 2048 for BT = 2): a workgroup of 4
 // waves owns 4 output columns and wave w streams B row n0 + w over all of K,
 // 16 bytes per lane of every kilobyte straight into registers (BT kilobytes
 // requested before their dot products), beside the same 16 bytes of the A
@@ -605,6 +558,20 @@ __global__ __launch_bounds__(256) void gemm_s8_rcr_row1_kernel(S8Args p, int m0)
     const int8_t *brow = p.b + (int64_t)(n0 + wave) * p.ldb + lane * 16;
     const int8_t *arow = p.a + (int64_t)m0 * p.lda + lane * 16;
     int acc = 0;
+    if constexpr (BT == 1) {
+        // the part of a kilobyte at the end of K % 1024 != 0
+        if (nch * 1024 + lane * 16 < p.K) {
+            const v4i av = *reinterpret_cast<const v4i *>(arow + (int64_t)nch * 1024);
+            const v4i bv = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(brow + (int64_t)nch * 1024));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (U8)
+                    acc = (int)__builtin_amdgcn_udot4((uint32_t)av[q], (uint32_t)bv[q], (uint32_t)acc, false);
+                else
+                    acc = __builtin_amdgcn_sdot4(av[q], bv[q], acc, false);
+            }
+        }
+    }
     for (int c0 = 0; c0 < nch; c0 += BT) {
         v4i av[BT], bv[BT];
 #pragma unroll
@@ -650,18 +617,15 @@ __global__ __launch_bounds__(256) void gemm_s8_rcr_row1_kernel(S8Args p, int m0)
 // contiguous kilobyte.  After one barrier wave w multiplies its contiguous
 // K/16 bytes: B fragments from LDS, the RF 16-row A fragments of those
 // bytes from global memory (issued before the barrier), one
-// v_mfma_i32_16x16x64_i8 per 64 bytes and fragment with the operand roles
-// of gemm_s8_rcr_rows_kernel, so lane l ends with row 16 f + l % 16 and
+// v_mfma_i32_16x16x64_i8 per 64 bytes and fragment, B first and A second,
+// so lane l ends with row 16 f + l % 16 and
 // columns 4 (l / 16) .. + 3.  The 16 partial sums go through LDS (int32
 // wrap-around, order-free) and the tiles' epilogue.
 constexpr int kRowsDmaMaxK = 8192;
-// Up to this many last rows take gemm_s8_rcr_rows_dma_kernel (N = K = 4096,
-// rotated weights: M = 1 / 16 in 5.45 / 6.8 us against 6.7 / 7.9 for
-// gemm_s8_rcr_rows_kernel, and against 6.2 / 6.6 us for the staged kernel
-// below with 1 KiB stages three deep).  From 17 rows on the staged kernel
-// is faster: M = 17 / 24 / 32 in 6.96 / 7.05 / 7.18 us against 7.4 / 7.9 /
-// 8.6 for this kernel with two fragments.
-constexpr int kRowsDmaMaxRows = 16;
+// N = K = 4096, rotated weights: M = 1 / 16 in 5.45 / 6.8 us, against 6.2 /
+// 6.6 us for the staged kernel below with 1 KiB stages three deep; M = 17 /
+// 24 / 32 6.96 / 7.05 / 7.18 us staged against 7.4 / 7.9 / 8.6 here with two
+// fragments (launch_last_rows has the line).
 constexpr int kRowsDmaWaves = 16;
 
 template <int EPI, bool VecOut, int ACT, typename BiasT, int RF>
@@ -730,15 +694,13 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_dma_kernel(S8Args p, in
     epi(mb + 16 * wave + r16, n0 + 4 * g, sum);   // rows past M are not stored
 }
 
-// The last rows, 17 to 16 RF of them, with A and B streamed through LDS in
-// K stages of SB bytes, DEPTH stages in flight (K % SB == 0; A and B 16-byte
+// The last rows, at most 16 RF of them, with A and B streamed through LDS in
+// K stages of SB bytes, DEPTH stages in flight (K % 16 == 0; A and B 16-byte
 // aligned, (m0 + 16 RF) * lda and N * ldb below 2^31; dynamic LDS of
-// DEPTH * (16 RF + 16) * SB bytes).  gemm_s8_rcr_rows_kernel reads its A
-// fragments from global memory as 64-byte pieces of 16 rows, and every one
-// of the N / 16 workgroups reads all of A: that pattern moves L2-resident
-// bytes 2.5x slower than whole kilobytes (64 MB of A at M = 64: 8.1
-// against 3.2 us) and dominated the pass.  Here a workgroup of 16 waves
-// LDS-DMAs each K stage of its 16 RF A rows (rows past M land as zeros) and
+// DEPTH * (16 RF + 16) * SB bytes).  Every one of the N / 16 workgroups reads
+// all of A; as 64-byte pieces of 16 rows that moves L2-resident bytes 2.5x
+// slower than as whole kilobytes (64 MB of A at M = 64: 8.1 against 3.2
+// us).  So a workgroup of 16 waves LDS-DMAs each K stage of its 16 RF A rows (rows past M land as zeros) and
 // of its 16 B rows, 1024 / SB whole row pieces per instruction, all before
 // anything waits.  16-byte unit u of row r of a stage sits at slot
 // u ^ (r & 15), so fragment reads are conflict-free.  Wave w owns 64-byte
@@ -749,7 +711,7 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_dma_kernel(S8Args p, in
 // 512-byte stages, two in flight: at N = K = 4096 (M = 33 / 64 / 100 / 128)
 // 8.0 / 8.8 / 11.3 / 11.6 us, against 9.8-10.3 / 10.0-10.5 / 12.0-13.2 /
 // 12.3-13.5 us for 256-byte stages two to four deep; three 512-byte stages
-// measure the same as two (kRowsStagedSB, kRowsStagedDepth).
+// measure the same as two.
 
 // U8: u8 x u8 operands (RCR u8 SKUs; EPI unused) through the signed MFMA:
 // fragments flipped to u - 128 and the correction of
@@ -805,21 +767,24 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_staged_kernel(S8Args p,
             const int idx = 64 * j + lane;
             const int r = idx / UPR, slot = idx % UPR;
             const int unit = slot ^ (r & 15);
+            // units at or past K (a partial last stage) land as zeros
+            const bool past = k0 + 16 * unit >= p.K;
             if (r < 16 * RF) {
-                mfma2::dma16(ra, (int)((int64_t)(m0 + r) * p.lda) + 16 * unit, k0, buf + j * 1024);
+                mfma2::dma16(ra, past ? mfma2::kPastExtent : (int)((int64_t)(m0 + r) * p.lda) + 16 * unit, k0, buf + j * 1024);
             } else if constexpr (RowB) {
                 // unit ib of the B region: k-row ib / NB, 16 columns ib % NB
                 const int ib = idx - 16 * RF * UPR;
                 mfma2::dma16(rb, (ib / NB) * (int)p.ldb + n0 + 16 * (ib % NB),
                              __builtin_amdgcn_readfirstlane(k0 * (int)p.ldb), buf + j * 1024);
             } else {
-                mfma2::dma16(rb, (int)((int64_t)(n0 + r - 16 * RF) * p.ldb) + 16 * unit, k0, buf + j * 1024);
+                mfma2::dma16(rb, past ? mfma2::kPastExtent : (int)((int64_t)(n0 + r - 16 * RF) * p.ldb) + 16 * unit, k0,
+                             buf + j * 1024);
             }
         }
     };
     // waves below NI % 16 issue HI instructions per stage, the others LO
     const bool hi = NI % WAVES == 0 || wave < NI % WAVES;
-    const int ns = p.K / SB;
+    const int ns = (p.K + SB - 1) / SB;
     for (int st = 0; st < DEPTH && st < ns; ++st) dma_stage(st, lds + st * STAGE);
     const int c = wave % CH, f0 = wave / CH;
     const bool active = ALL || wave < RF * CH;   // wave-uniform
@@ -882,8 +847,9 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_staged_kernel(S8Args p,
     }
     __syncthreads();
     const S8Epilogue<EPI, VecOut, ACT, BiasT> epi{p};
-    // u8: au = acc - kcorr with zero sums, kcorr = -16384 K (mod 2^32)
-    const U8Epilogue<VecOut, ACT, BiasT> epi_u8{p, kZeroSums, kZeroSums, 0u - 16384u * (uint32_t)p.K};
+    // u8: au = acc - kcorr with zero sums, kcorr = -16384 K (mod 2^32), K
+    // rounded up to whole stages (a zero-filled k adds (-128)^2 - 128 * 256)
+    const U8Epilogue<VecOut, ACT, BiasT> epi_u8{p, kZeroSums, kZeroSums, 0u - 16384u * (uint32_t)(ns * SB)};
     for (int e = wave; e < RF * NB; e += WAVES) {
         const int f = e % RF, nb = e / RF;
         v4i sum = part[((f * NB + nb) * CH) * 64 + lane];
@@ -922,7 +888,7 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_s8_rrr_dma_kernel(S8Args p
     const bool full = m_base + M2::BM <= p.M && n_base + M2::BN <= p.N;
     if constexpr (VecOut) {
         if (p.ldd % 16 == 0 && (reinterpret_cast<uintptr_t>(p.d) & 15u) == 0 && (full || p.N % 16 == 0)) {
-            store_s8_tile_staged<P>(acc, stage0, stage1, p, m_base, n_base, epi);
+            store_s8_tile_staged<P>(acc, mfma2::wave_scratch<DmaCfg>(stage0, stage1), p, m_base, n_base, epi);
             return;
         }
     }
@@ -1534,178 +1500,194 @@ int32_t launch_u8_rcr(const S8Args &p, hipStream_t stream) {
     return launch_status();
 }
 
+template <int EPI, bool VecOut, int ACT, typename BiasT, class C, int DEPTH, int SPREAD>
+void launch_ring(const S8Args &p, hipStream_t stream) {
+    const int tiles = ((p.M + C::TB - 1) / C::TB) * ((p.N + C::TBN - 1) / C::TBN);
+    hipLaunchKernelGGL((gemm_s8_rcr_ring_kernel<EPI, VecOut, ACT, BiasT, C, DEPTH, SPREAD>), dim3(tiles), dim3(C::NT),
+                       (size_t)DEPTH * C::STAGE, stream, p);
+}
+
+// All of M as tiles of the cheapest shape (mfma2::ring_tile); outputs
+// without 4-column stores take the 128 x 128 tiles on small grids.
 template <int EPI, bool VecOut, int ACT, typename BiasT>
-void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *workspace, size_t workspace_bytes) {
-    if (fast_k) {
-        TailSplit ts = tail_split_plan(p.M, p.N, p.K);
-        const size_t need = tail_split_workspace(p.M, p.N, p.K);
-        const bool split_ws = ts.split > 1 && workspace != nullptr && workspace_bytes >= need &&
-                              (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
-        const int rem = split_ws ? 0 : rows_path_rows(p.M, p.N);
-        // Small problems (129-512 rows) whose 128-row blocks of the staged
-        // last-rows kernel fit one round of workgroups run that way instead of
-        // tiles.  K = 4096, M = 129 / 256 / 512: N = 4096 12.8 / 13.4 / 17.9 us
-        // against 24.2 / 24.4 / 25.1 on 128x128 tiles; at N = 14336 the blocks
-        // need 2-4 rounds and lose from 384 rows (48.9 against 37.0).
-        // 64-row blocks first, when they still fit one round of workgroups
-        // (K = 4096, M = 129 / 256: N = 4096 12.5 / 13.0 -> 11.0 / 11.4 us;
-        // N = 2048 9.8 / 10.3 -> 7.6 / 7.8 us, M = 512 12.1 -> 10.9 us; N =
-        // 8192 level).  Letting the 128-row blocks run two rounds was mixed
-        // (N = 14336, M = 129: 34.6 -> 32.7 us; N = 6144, M = 384: 25.2 ->
-        // 31.7 us), so they keep one.
-        if (rem == 0 && !split_ws && p.M > 128 && p.M <= 512 && p.N % 16 == 0 && p.K % 512 == 0) {
-            const int b4 = (p.M + 63) / 64;
-            const int n4 = mfma2::last_rows_col_frags(p.N, b4);
-            if (b4 * (p.N / (16 * n4)) <= 256) {
+void launch_tiles(const S8Args &p, hipStream_t stream) {
+    using mfma2::Cfg;
+    const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+    const mfma2::RingTile t = VecOut ? mfma2::ring_tile(p.M, p.N, p.K)
+                                     : tiles <= kSmallTilesMax ? mfma2::RT_128x128 : mfma2::RT_256x256;
+    if constexpr (VecOut) {
+        if (t == mfma2::RT_64x64) return launch_ring<EPI, VecOut, ACT, BiasT, Cfg<4, 1, 64, 64>, 4, 0>(p, stream);
+        if (t == mfma2::RT_64x128) return launch_ring<EPI, VecOut, ACT, BiasT, Cfg<2, 2, 64, 128>, 3, 2>(p, stream);
+        if (t == mfma2::RT_128x256) return launch_ring<EPI, VecOut, ACT, BiasT, Cfg<2, 4, 128, 256>, 3, 4>(p, stream);
+        if (t == mfma2::RT_192x256) return launch_ring<EPI, VecOut, ACT, BiasT, Cfg<2, 4, 192, 256>, 2, 0>(p, stream);
+    }
+    if (t == mfma2::RT_128x128) return launch_ring<EPI, VecOut, ACT, BiasT, Cfg<4, 2, 128, 128>, 3, 2>(p, stream);
+    hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, p,
+                       TailSplit{0, 0, 1}, (int32_t *)nullptr);
+}
+
+// Every row of the problem as `blocks` row blocks of 16 rf rows on the
+// staged last-rows kernel; false when the workgroups exceed one round.
+template <int EPI, bool VecOut, int ACT, typename BiasT>
+bool launch_row_blocks(const S8Args &p, hipStream_t stream) {
+    // 64-row blocks first, when they fit one round of workgroups (K = 4096,
+    // M = 129 / 256: N = 2048 9.8 / 10.3 -> 7.6 / 7.8 us, M = 512 12.1 ->
+    // 10.9 us against 128-row blocks).  Letting the 128-row blocks run two
+    // rounds was mixed (N = 14336, M = 129: 34.6 -> 32.7 us; N = 6144, M =
+    // 384: 25.2 -> 31.7 us), so they keep one.
+    const int b4 = (p.M + 63) / 64;
+    const int n4 = mfma2::last_rows_col_frags(p.N, b4);
+    if (b4 * (p.N / (16 * n4)) <= 256) {
 #define BK_S8BLK4(NB)                                                                                        \
-                if (n4 == (NB)) {                                                                            \
-                    hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, 4, NB, 512, 2>), \
-                                       dim3(p.N / (16 * (NB)), b4), dim3(1024),                              \
-                                       std::max((size_t)2 * (64 + 16 * (NB)) * 512, (size_t)4 * (NB) * 8 * 1024), \
-                                       stream, p, 0);                                                        \
-                    return;                                                                                  \
-                }
-                BK_S8BLK4(1) BK_S8BLK4(2) BK_S8BLK4(4)
+        if (n4 == (NB)) {                                                                                    \
+            hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, 4, NB, 512, 2>),     \
+                               dim3(p.N / (16 * (NB)), b4), dim3(1024),                                      \
+                               std::max((size_t)2 * (64 + 16 * (NB)) * 512, (size_t)4 * (NB) * 8 * 1024),    \
+                               stream, p, 0);                                                                \
+            return true;                                                                                     \
+        }
+        BK_S8BLK4(1) BK_S8BLK4(2) BK_S8BLK4(4)
 #undef BK_S8BLK4
-            }
-        }
-        const int blocks = (p.M + 127) / 128;
-        const int nbb = mfma2::last_rows_col_frags(p.N, blocks);
-        if (rem == 0 && !split_ws && p.M > 128 && p.M <= 512 && p.N % 16 == 0 && p.K % 512 == 0 &&
-            blocks * (p.N / (16 * nbb)) <= 256) {
-            const int nb = nbb;
+    }
+    const int blocks = (p.M + 127) / 128;
+    const int nb = mfma2::last_rows_col_frags(p.N, blocks);
+    if (blocks * (p.N / (16 * nb)) > 256) return false;
 #define BK_S8BLOCKS(NB, SB)                                                                                  \
-            if (nb == (NB)) {                                                                                \
-                const size_t lds = std::max((size_t)2 * (128 + 16 * (NB)) * (SB), (size_t)8 * (NB) * ((SB) / 64) * 1024); \
-                hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, 8, NB, SB, 2>),    \
-                                   dim3(p.N / (16 * (NB)), blocks), dim3(1024), lds, stream, p, 0);          \
-                return;                                                                                      \
-            }
-            BK_S8BLOCKS(1, 512)
-            BK_S8BLOCKS(2, 512)
-            BK_S8BLOCKS(4, 256)
+    if (nb == (NB)) {                                                                                        \
+        const size_t lds = std::max((size_t)2 * (128 + 16 * (NB)) * (SB), (size_t)8 * (NB) * ((SB) / 64) * 1024); \
+        hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, 8, NB, SB, 2>),          \
+                           dim3(p.N / (16 * (NB)), blocks), dim3(1024), lds, stream, p, 0);                  \
+        return true;                                                                                         \
+    }
+    BK_S8BLOCKS(1, 512)
+    BK_S8BLOCKS(2, 512)
+    BK_S8BLOCKS(4, 256)
 #undef BK_S8BLOCKS
-        }
-        if (rem != 0) {
-            // whole 256-row tiles, then the last rows (gemm_s8_rcr_rows_kernel)
-            S8Args pm = p;
-            pm.M = p.M - rem;
-            const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-            if (tiles > 0)
-                hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT),
-                                   0, stream, pm, TailSplit{0, 0, 1}, (int32_t *)nullptr);
-            // fast_k already holds A and B 16-byte aligned, lda and ldb multiples
-            // of 16 and both extents (rows rounded up to 256) below 2^31
-            // With 32- or 64-column workgroups the staged kernel also beats the
-            // B-only DMA kernel from 9 rows (N = 14336, K = 4096: M = 8 / 16
-            // 14.3 / 17.5 us on the DMA kernel, 14.5 us staged at 17 rows).
-            const int nb = mfma2::last_rows_col_frags(p.N);
-            if (nb == 1 && rem > 32 && p.K % 512 == 0) {
-                // 33-128 rows where 16-column workgroups would each read all
-                // of them: 2-4 row blocks (last_rows_blocks).  K = 4096,
-                // rotated weights, graph replay: N = 4096, M = 48 / 100 / 128
-                // 8.5 / 11.6 / 11.9 -> 7.8 / 9.1 / 9.5 us; N = 2048, M = 48 /
-                // 128 6.8 / 9.9 -> 5.8 / 6.5 us
-                int rf, blk, nbb;
-                mfma2::last_rows_blocks(rem, p.N, rf, blk, nbb);
+    return false;
+}
+
+// The last `rem` (<= kRowsPathMax) rows, from row m0 (N % 16 == 0).
+template <int EPI, bool VecOut, int ACT, typename BiasT>
+void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
+    const int nb = mfma2::last_rows_col_frags(p.N);
+    if (nb == 1 && rem > 32) {
+        // 33-128 rows where 16-column workgroups would each read all
+        // of them: 2-4 row blocks (last_rows_blocks).  K = 4096,
+        // rotated weights, graph replay: N = 4096, M = 48 / 100 / 128
+        // 8.5 / 11.6 / 11.9 -> 7.8 / 9.1 / 9.5 us; N = 2048, M = 48 /
+        // 128 6.8 / 9.9 -> 5.8 / 6.5 us
+        int rf, blk, nbb;
+        mfma2::last_rows_blocks(rem, p.N, rf, blk, nbb);
 #define BK_S8RBLK(RF, NB)                                                                                     \
-                if (rf == (RF) && nbb == (NB)) {                                                               \
-                    hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, RF, NB, 512, 2>), \
-                                       dim3(p.N / (16 * (NB)), blk), dim3(1024),                               \
-                                       std::max((size_t)2 * (16 * (RF) + 16 * (NB)) * 512, (size_t)(RF) * (NB) * 8 * 1024), \
-                                       stream, p, pm.M);                                                       \
-                    return;                                                                                    \
-                }
-                BK_S8RBLK(2, 1) BK_S8RBLK(4, 1) BK_S8RBLK(2, 2) BK_S8RBLK(4, 2) BK_S8RBLK(2, 4) BK_S8RBLK(4, 4)
+        if (rf == (RF) && nbb == (NB)) {                                                                       \
+            hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, RF, NB, 512, 2>),      \
+                               dim3(p.N / (16 * (NB)), blk), dim3(1024),                                       \
+                               std::max((size_t)2 * (16 * (RF) + 16 * (NB)) * 512, (size_t)(RF) * (NB) * 8 * 1024), \
+                               stream, p, m0);                                                                 \
+            return;                                                                                            \
+        }
+        BK_S8RBLK(2, 1) BK_S8RBLK(4, 1) BK_S8RBLK(2, 2) BK_S8RBLK(4, 2) BK_S8RBLK(2, 4) BK_S8RBLK(4, 4)
 #undef BK_S8RBLK
-            }
-            if (nb == 1 && rem > 10 && rem <= 16 && p.K % 512 == 0) {
-                // 11-16 rows below N = 6144: one fragment, 8 waves multiplying
-                // (K = 4096, M = 12 / 16: N = 4096 6.55 / 6.93 -> 6.37 /
-                // 6.42 us, N = 2048 4.95 / 5.27 -> 4.87 / 4.90 us against the
-                // B-through-LDS kernel, which stays ahead up to 8 rows)
-                hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, 1, 1, 512, 3>),
-                                   dim3(p.N / 16), dim3(1024), (size_t)3 * 32 * 512, stream, p, pm.M);
-                return;
-            }
-            // staged from 6 rows at 64 columns (one fragment: N = 14336 / 12288,
-            // M = 8 14.2 / 11.6 -> 13.2 / 10.8 us against the B-through-LDS
-            // kernel, level at 2-5 rows), from 9 at 32 columns, from 17 at 16
-            if (rem > (nb > 1 ? (nb == 4 ? 5 : 8) : kRowsDmaMaxRows) && p.K % kRowsStagedSB == 0) {
+    }
+    if (rem == 1) {
+        if (p.K % 2048 == 0)
+            hipLaunchKernelGGL((gemm_s8_rcr_row1_kernel<EPI, VecOut, ACT, BiasT, 2>), dim3(p.N / 4), dim3(256),
+                               0, stream, p, m0);
+        else
+            hipLaunchKernelGGL((gemm_s8_rcr_row1_kernel<EPI, VecOut, ACT, BiasT, 1>), dim3(p.N / 4), dim3(256),
+                               0, stream, p, m0);
+        return;
+    }
+    // Few rows with K % 1024 == 0: the B-through-LDS kernel up to 10 rows at
+    // 16 columns (K = 4096, M = 12 / 16 on one staged fragment against it: N =
+    // 4096 6.55 / 6.93 -> 6.37 / 6.42 us, N = 2048 4.95 / 5.27 -> 4.87 / 4.90;
+    // it stays ahead up to 8 rows), 8 at 32 columns, 5 at 64 (N = 14336 /
+    // 12288, M = 8 14.2 / 11.6 -> 13.2 / 10.8 us staged, level at 2-5 rows).
+    if (rem <= (nb == 1 ? 10 : nb == 2 ? 8 : 5) && p.K % 1024 == 0 && p.K <= kRowsDmaMaxK) {
+        // B rows; the 16 waves' partial sums reuse the same LDS
+        const size_t lds = std::max((size_t)16 * p.K, (size_t)kRowsDmaWaves * 1024);
+        hipLaunchKernelGGL((gemm_s8_rcr_rows_dma_kernel<EPI, VecOut, ACT, BiasT, 1>), dim3(p.N / 16),
+                           dim3(1024), lds, stream, p, m0);
+        return;
+    }
 #define BK_S8ROWS(RF, NB, SB, DEPTH)                                                                        \
-    if (rem <= 16 * (RF) && nb == (NB) && p.K % (SB) == 0) {                                                 \
+    if (rem <= 16 * (RF) && nb == (NB)) {                                                                    \
         hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, RF, NB, SB, DEPTH>),     \
                            dim3(p.N / (16 * (NB))), dim3(1024),                                             \
                            std::max((size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), (size_t)(RF) * (NB) * ((SB) / 64) * 1024), \
-                           stream, p, pm.M);                                                                \
+                           stream, p, m0);                                                                  \
         return;                                                                                             \
     }
-                BK_S8ROWS(2, 1, 512, 3)
-                BK_S8ROWS(4, 1, 512, 2)
-                BK_S8ROWS(8, 1, 512, 2)
-                // up to 16 rows from N = 6144: one fragment, 8 waves
-                // multiplying (N = 14336 / 8192, M = 12-16: 13.85 / 8.6-8.7
-                // -> 13.3 / 8.5 us against two fragments)
-                BK_S8ROWS(1, 2, 512, 2)
-                BK_S8ROWS(1, 4, 512, 2)
-                BK_S8ROWS(2, 2, 512, 3)
-                BK_S8ROWS(4, 2, 512, 2)
-                BK_S8ROWS(8, 2, 512, 2)
-                BK_S8ROWS(2, 4, 512, 3)
-                BK_S8ROWS(4, 4, 512, 2)
-                BK_S8ROWS(8, 4, 256, 2)
+    // up to 16 rows: one fragment, 8 of the 16 waves multiplying (N = 14336 /
+    // 8192, M = 12-16: 13.85 / 8.6-8.7 -> 13.3 / 8.5 us against two)
+    BK_S8ROWS(1, 1, 512, 3)
+    BK_S8ROWS(2, 1, 512, 3)
+    BK_S8ROWS(1, 2, 512, 2)
+    BK_S8ROWS(1, 4, 512, 2)
+    BK_S8ROWS(2, 2, 512, 3)
+    BK_S8ROWS(4, 2, 512, 2)
+    BK_S8ROWS(8, 2, 512, 2)
+    BK_S8ROWS(2, 4, 512, 3)
+    BK_S8ROWS(4, 4, 512, 2)
+    BK_S8ROWS(8, 4, 256, 2)
 #undef BK_S8ROWS
-            }
-            if (rem == 1 && p.K % 1024 == 0) {
-                if (p.K % 2048 == 0)
-                    hipLaunchKernelGGL((gemm_s8_rcr_row1_kernel<EPI, VecOut, ACT, BiasT, 2>), dim3(p.N / 4), dim3(256),
-                                       0, stream, p, pm.M);
-                else
-                    hipLaunchKernelGGL((gemm_s8_rcr_row1_kernel<EPI, VecOut, ACT, BiasT, 1>), dim3(p.N / 4), dim3(256),
-                                       0, stream, p, pm.M);
-                return;
-            }
-            if (rem <= kRowsDmaMaxRows && p.K % 1024 == 0 && p.K <= kRowsDmaMaxK) {
-                // B rows; the 16 waves' partial sums reuse the same LDS
-                const size_t lds = std::max((size_t)16 * p.K, (size_t)kRowsDmaWaves * 1024);
-                hipLaunchKernelGGL((gemm_s8_rcr_rows_dma_kernel<EPI, VecOut, ACT, BiasT, 1>), dim3(p.N / 16),
-                                   dim3(1024), lds, stream, p, pm.M);
-                return;
-            }
-            const dim3 grid(p.N / 16), block(512);
-            if (rem <= 16)
-                hipLaunchKernelGGL((gemm_s8_rcr_rows_kernel<EPI, VecOut, ACT, BiasT, 1>), grid, block, 0, stream, p, pm.M);
-            else if (rem <= 32)
-                hipLaunchKernelGGL((gemm_s8_rcr_rows_kernel<EPI, VecOut, ACT, BiasT, 2>), grid, block, 0, stream, p, pm.M);
-            else if (rem <= 64)
-                hipLaunchKernelGGL((gemm_s8_rcr_rows_kernel<EPI, VecOut, ACT, BiasT, 4>), grid, block, 0, stream, p, pm.M);
-            else
-                hipLaunchKernelGGL((gemm_s8_rcr_rows_kernel<EPI, VecOut, ACT, BiasT, 8>), grid, block, 0, stream, p, pm.M);
-            return;
-        }
-        const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-        if (split_ws) {
-            int32_t *slots = static_cast<int32_t *>(workspace);
-            hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>),
-                               dim3(ts.full_tiles + ts.tail_tiles * ts.split), dim3(DmaCfg::NT), 0, stream, p, ts,
-                               slots);
-            hipLaunchKernelGGL((gemm_s8_tail_reduce_kernel<EPI, VecOut, ACT, BiasT>), dim3(ts.tail_tiles, 64),
-                               dim3(256), 0, stream, p, ts, (const int32_t *)slots);
-            return;
-        }
-        if (tiles <= kSmallTilesMax) {
-            typedef mfma2::Cfg<2, 2, 128> SmallCfg;
-            const int tiles128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
-            hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT, SmallCfg>), dim3(tiles128),
-                               dim3(SmallCfg::NT), 0, stream, p, TailSplit{0, 0, 1}, (int32_t *)nullptr);
-            return;
-        }
-        hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, p,
-                           TailSplit{0, 0, 1}, (int32_t *)nullptr);
-    } else {
+}
+
+// Row blocks of the staged last-rows kernel instead of tiles (33-512 rows)
+// where 64 x 64 tiles would leave half of the CUs idle: they split K over
+// their waves, which a tile does not.  us, blocks against the best tile: 200 x
+// 1024 x 4096 7.0 / 9.8, 128 x 4096 x 4096 8.5 / 10.0, 512 x 1024 x 4096 8.3 /
+// 10.1, 128 x 4096 x 14336 25.9 / 33; past the line 200 x 4096 x 4096 11.5 /
+// 10.2, 384 x 2048 x 1024 5.7 / 4.9, 128 x 8192 x 4096 14.9 / 11.7, 64 x
+// 14336 x 4096 17.8 / 15.7.
+inline bool few_tiles(int M, int N) { return (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 128; }
+
+// Whole 256-row tiles and a last-rows pass for more than 512 rows, against
+// the cheapest tile over all rows: the pass reads the weights once more, at
+// about 3.6 TB/s behind the tiles, and takes at least a launch.
+inline bool last_rows_pay(int M, int N, int K, int rem) {
+    float all;
+    mfma2::ring_tile(M, N, K, &all);
+    return mfma2::ring_cost(mfma2::kRingCost[mfma2::RT_256x256], M - rem, N, K) + 3.0f + (float)N * (float)K / 3.6e6f < all;
+}
+
+template <int EPI, bool VecOut, int ACT, typename BiasT>
+void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *workspace, size_t workspace_bytes) {
+    if (!fast_k) {
         const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
         hipLaunchKernelGGL((gemm_s8_rcr_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(NT), 0, stream, p);
+        return;
     }
+    const TailSplit ts = tail_split_plan(p.M, p.N, p.K);
+    if (ts.split > 1 && workspace != nullptr && workspace_bytes >= tail_split_workspace(p.M, p.N, p.K) &&
+        (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0) {
+        int32_t *slots = static_cast<int32_t *>(workspace);
+        hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>),
+                           dim3(ts.full_tiles + ts.tail_tiles * ts.split), dim3(DmaCfg::NT), 0, stream, p, ts,
+                           slots);
+        hipLaunchKernelGGL((gemm_s8_tail_reduce_kernel<EPI, VecOut, ACT, BiasT>), dim3(ts.tail_tiles, 64),
+                           dim3(256), 0, stream, p, ts, (const int32_t *)slots);
+        return;
+    }
+    const int rem = rows_path_rows(p.M, p.N);
+    if (rem == p.M) {
+        if (VecOut && rem > 32 && !few_tiles(p.M, p.N)) launch_tiles<EPI, VecOut, ACT, BiasT>(p, stream);
+        else launch_last_rows<EPI, VecOut, ACT, BiasT>(p, 0, rem, stream);
+        return;
+    }
+    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && (!VecOut || few_tiles(p.M, p.N)) &&
+        launch_row_blocks<EPI, VecOut, ACT, BiasT>(p, stream))
+        return;
+    if (rem != 0 && (!VecOut || last_rows_pay(p.M, p.N, p.K, rem))) {
+        S8Args pm = p;
+        pm.M = p.M - rem;
+        const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+        hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT),
+                           0, stream, pm, TailSplit{0, 0, 1}, (int32_t *)nullptr);
+        launch_last_rows<EPI, VecOut, ACT, BiasT>(p, pm.M, rem, stream);
+        return;
+    }
+    launch_tiles<EPI, VecOut, ACT, BiasT>(p, stream);
 }
 
 // workspace (optional): tail_split_workspace(M, N, K) bytes, 16-byte aligned,
@@ -1714,10 +1696,10 @@ void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *works
 template <int EPI, int ACT = ACT_NONE, typename BiasT = float>
 int32_t launch(const S8Args &p, hipStream_t stream, void *workspace = nullptr, size_t workspace_bytes = 0) {
     const int out_elem = (EPI == EPI_I32 || EPI == EPI_W8A8_F32) ? 4 : EPI == EPI_W8A8_F64 ? 8 : (EPI == EPI_S8 ? 1 : 2);
-    // The DMA path needs whole K stages and 16-byte rows; edge tiles read
-    // zeros past the operands, so the byte offsets of the padded extents
-    // must stay below 2^31.
-    const bool fast_k = p.K > 0 && p.K % BK == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 &&
+    // The DMA path needs 16-byte units of K and rows; edge tiles and a
+    // partial last stage read zeros past the operands, so the byte offsets of
+    // the padded extents must stay below 2^31.
+    const bool fast_k = p.K > 0 && p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 &&
                         aligned16(p.a) && aligned16(p.b) && dma_extent_ok(p.M, p.lda) &&
                         dma_extent_ok(p.N, p.ldb);
     // 4-wide vector stores need every 4-column group of D (and sw) aligned;

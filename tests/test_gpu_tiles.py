@@ -1,0 +1,84 @@
+"""The mid-size block tiles of the RCR GEMMs and depths off the 128-byte stage.
+
+Shapes pick each tile of the chooser (64x64 to 256x256) with ragged M and N
+edges and K a multiple of 16 only (last stages of 16, 64 and 112 bytes), and
+the last-rows kernels with partial last stages.  Integer results are exact
+against float64 products (sums below 2^53).
+"""
+import numpy as np
+import pytest
+import torch
+
+from baracuda_amd import plans as P
+from baracuda_amd.ffi import lib
+from oracle.inputs import int8_uniform, rng
+from tests.gpu_util import dev, host_bits16, sync
+
+pytestmark = pytest.mark.gpu
+
+TILE_SHAPES = [(300, 1700, 208), (450, 2896, 1040), (1000, 2500, 1136), (1500, 5120, 336), (2300, 5008, 400),
+               (3070, 4100, 336), (4000, 4100, 48), (513, 2064, 16)]
+# one row (partial kilobyte), one / two / four / eight fragments, each column
+# width, row blocks, whole tiles with last rows
+ROW_SHAPES = [(1, 4096, 4080), (1, 272, 48), (5, 512, 1040), (9, 12288, 304), (13, 6160, 1552), (24, 4096, 2752),
+              (60, 12288, 304), (100, 272, 656), (120, 6144, 176), (200, 1024, 1072), (400, 1024, 208),
+              (4160, 4096, 144)]
+
+
+def _acc(a, b):
+    return (torch.from_numpy(a).double() @ torch.from_numpy(b).double().T).to(torch.int64).numpy()
+
+
+@pytest.mark.parametrize("shape", TILE_SHAPES + ROW_SHAPES)
+def test_int8_tiles_and_depth_tails(gpu, shape):
+    m, n, k = shape
+    print(f"case: int8 tiles {shape}", flush=True)
+    g = rng(m + 3 * n + 7 * k)
+    a, b, c = int8_uniform(g, (m, k)), int8_uniform(g, (n, k)), int8_uniform(g, (m, n))
+    acc = _acc(a, b)
+    ta, tb = dev(a), dev(b)
+    d = torch.full((m, n), -7, dtype=torch.int32, device="cuda:0")
+    P.IntGemmPlan.select(P.IntGemmDescriptor(m, n, k, output=P.ElementKind.I32)).run(ta, tb, d)
+    sync()
+    assert np.array_equal(d.cpu().numpy(), acc)
+    accf = acc.astype(np.float32)
+    # int8 out with C: f32 products and sum, round half to even, saturate
+    alpha = np.float32(1.0 / (60.0 * np.sqrt(k)))
+    d8 = torch.full((m, n), 99, dtype=torch.int8, device="cuda:0")
+    P.IntGemmPlan.select(P.IntGemmDescriptor(m, n, k)).run(ta, tb, d8, c=dev(c), alpha=float(alpha), beta=0.5)
+    sync()
+    z = alpha * accf + np.float32(0.5) * c.astype(np.float32)
+    assert np.array_equal(d8.cpu().numpy(), np.clip(np.rint(z), -128, 127).astype(np.int8))
+    # W8A8: (sa * sw) * acc, bf16 / f32 / f64
+    sa, sw = g.uniform(0.005, 0.02, m).astype(np.float32), g.uniform(0.001, 0.01, n).astype(np.float32)
+    y = (sa[:, None] * sw[None, :]) * accf
+    dw = torch.empty((m, n), dtype=torch.bfloat16, device="cuda:0")
+    P.IntGemmPlan.select(P.IntGemmDescriptor(m, n, k, output=P.ElementKind.Bf16)).run(
+        ta, tb, dw, scale_a=dev(sa), scale_b=dev(sw))
+    out = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+    out64 = torch.empty((m, n), dtype=torch.float64, device="cuda:0")
+    stream = torch.cuda.current_stream().cuda_stream
+    tsa, tsw, tsa64, tsw64 = dev(sa), dev(sw), dev(sa.astype(np.float64)), dev(sw.astype(np.float64))
+    assert lib().quantized_linear_w8a8_f32_gfx950_run(m, n, k, tb.data_ptr(), ta.data_ptr(), tsa.data_ptr(),
+                                                      tsw.data_ptr(), out.data_ptr(), None, 0, stream) == 0
+    assert lib().quantized_linear_w8a8_f64_gfx950_run(m, n, k, tb.data_ptr(), ta.data_ptr(), tsa64.data_ptr(),
+                                                      tsw64.data_ptr(), out64.data_ptr(), None, 0, stream) == 0
+    sync()
+    assert np.array_equal(host_bits16(dw), host_bits16(torch.from_numpy(y).to(torch.bfloat16)))
+    assert np.array_equal(out.cpu().numpy(), y)
+    assert np.array_equal(out64.cpu().numpy(), y.astype(np.float64))
+
+
+@pytest.mark.parametrize("shape", [(300, 1700, 208), (1500, 5120, 336), (2300, 5008, 400), (60, 12288, 304),
+                                   (4160, 4096, 144)])
+def test_int8_depth_tail_reads_stay_in_the_row(gpu, shape):
+    """Rows wider than K: what lies past K in a row must not reach the sums."""
+    m, n, k = shape
+    g = rng(m + n + k)
+    pa, pb = int8_uniform(g, (m, k + 112)), int8_uniform(g, (n, k + 64))
+    print(f"case: int8 padded rows {shape}", flush=True)
+    d = torch.empty((m, n), dtype=torch.int32, device="cuda:0")
+    P.IntGemmPlan.select(P.IntGemmDescriptor(m, n, k, output=P.ElementKind.I32)).run(
+        dev(pa)[:, :k], dev(pb)[:, :k], d)
+    sync()
+    assert np.array_equal(d.cpu().numpy(), _acc(np.ascontiguousarray(pa[:, :k]), np.ascontiguousarray(pb[:, :k])))
