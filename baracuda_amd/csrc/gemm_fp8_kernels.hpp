@@ -10,15 +10,15 @@
 //   F8_F32   D = alpha * acc                                           new SKU
 // (baracuda_fp8_rcr_sm89.cuh:102-323, baracuda_fp8_rrr_sm89.cuh:60-272).
 //
-// Whole 256x256 tiles with K % 128 == 0 and 16-byte rows take the LDS-DMA
-// mainloop (v_mfma_f32_32x32x64_f8f6f4; RRR reads B with transposing LDS
-// reads); everything else the register-staged mainloop (16x16x128).
+// K % 16 == 0 with 16-byte rows takes the LDS-DMA mainloops
+// (v_mfma_f32_32x32x64_f8f6f4; RRR reads B with transposing LDS reads);
+// everything else the register-staged mainloop (16x16x128).
 #pragma once
 
 #include <type_traits>
 
 #include "gemm_mfma.hpp"
-#include "gemm_mfma2.hpp"
+#include "gemm_ring.hpp"
 #include "act.hpp"
 
 namespace bk {
@@ -130,33 +130,15 @@ struct F8DmaPolicy { typedef mfma2::PolicyF8<C, FMT> type; };
 template <int FMT, class C>
 struct F8DmaPolicy<FMT, F8_RRR, C> { typedef mfma2::PolicyF8RowB<C, FMT> type; };
 
-// Fast path: 256x256 tiles (edge tiles included), K % 128 == 0, 16-byte rows,
-// N % 4 == 0, vector stores.
-template <int FMT, int LAYOUT, int EPI, int ACT, class C = F8DmaCfg>
-__global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_dma_kernel(F8Args p) {
+// Epilogue of a tile of any policy configuration: the staged stores where D
+// allows them, else 4-column quads.  `scratch`: this wave's part of the LDS
+// that the loop left (see the staged stores).
+template <int FMT, int EPI, int ACT, class P>
+__device__ __forceinline__ void f8_store_tile(const mfma2::AccTile<P> &acc, int8_t *scratch, const F8Args &p, int m_base,
+                                              int n_base) {
     namespace M2 = mfma2;
-    typedef typename F8DmaPolicy<FMT, LAYOUT, C>::type P;
-    __shared__ __attribute__((aligned(1024))) int8_t stage0[2 * C::OPER];
-    __shared__ __attribute__((aligned(1024))) int8_t stage1[2 * C::OPER];
-    // Edge tiles (M or N not a multiple of 256): rows past M / N load as
-    // zeros (past the buffer resources' byte counts; RRR B columns past N
-    // read the next k-row, reaching only output columns that are not stored).
-    int tm, tn;
-    tile_coords(blockIdx.x, (p.M + C::TB - 1) / C::TB, (p.N + C::TB - 1) / C::TB, tm, tn);
-    const int m_base = tm * C::TB, n_base = tn * C::TB;
-    const bool full = m_base + C::TB <= p.M && n_base + C::TB <= p.N;
-    M2::AccTile<P> acc;
-    if constexpr (LAYOUT == F8_RCR) {
-        M2::DmaRows<false, false> d;
-        d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-        d.b = M2::make_dma_interior<C>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb);
-        M2::mainloop<P>(stage0, stage1, d, p.K, acc);
-    } else {
-        M2::DmaRowsRrr d;
-        d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-        d.b = M2::make_dma_row_b<C>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base);
-        M2::mainloop<P>(stage0, stage1, d, p.K, acc);
-    }
+    typedef typename P::Cfg C;
+    const bool full = m_base + C::TB <= p.M && n_base + C::TBN <= p.N;
     if constexpr (EPI == F8_BF16) {
         // bf16 rows staged per wave in LDS (free after the mainloop's last
         // barrier), written as 16-byte units: D = bf16_rne(alpha * acc).
@@ -164,7 +146,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_dma_kern
             const int wave = threadIdx.x >> 6;
             const int wrow = m_base + (wave / C::WAVES_N) * C::WM;
             const int wcol = n_base + (wave % C::WAVES_N) * C::WN;
-            int8_t *scratch = (wave < C::WAVES / 2 ? stage0 : stage1) + (wave % (C::WAVES / 2)) * (C::WM * 128);
             const float alpha = p.alpha;
             M2::store_bf16x4_staged<P>(
                 acc, scratch,
@@ -187,7 +168,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_dma_kern
             const int wave = threadIdx.x >> 6;
             const int wrow = m_base + (wave / C::WAVES_N) * C::WM;
             const int wcol = n_base + (wave % C::WAVES_N) * C::WN;
-            int8_t *scratch = (wave < C::WAVES / 2 ? stage0 : stage1) + (wave % (C::WAVES / 2)) * (C::WM / 2 * 256);
             const float alpha = p.alpha;
             M2::store_x32x4_staged<P>(
                 acc, scratch,
@@ -209,7 +189,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_dma_kern
             const int wave = threadIdx.x >> 6;
             const int wrow = m_base + (wave / C::WAVES_N) * C::WM;
             const int wcol = n_base + (wave % C::WAVES_N) * C::WN;
-            int8_t *scratch = (wave < C::WAVES / 2 ? stage0 : stage1) + (wave % (C::WAVES / 2)) * (C::WM * C::WN);
             // The C term and the M / N bounds decided once per tile, not per element.
             auto staged = [&](auto has_c, auto whole) {
                 M2::store_u8x4_staged<P>(
@@ -247,6 +226,57 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_dma_kern
     M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4f &v) { epi(m_base + ml, n_base + nl, v); });
 }
 
+// Fast path: 256x256 tiles (edge tiles included), K % 16 == 0, 16-byte rows,
+// N % 4 == 0, vector stores.
+template <int FMT, int LAYOUT, int EPI, int ACT>
+__global__ __launch_bounds__(F8DmaCfg::NT, 1) void gemm_fp8_dma_kernel(F8Args p) {
+    namespace M2 = mfma2;
+    typedef F8DmaCfg C;
+    typedef typename F8DmaPolicy<FMT, LAYOUT, C>::type P;
+    __shared__ __attribute__((aligned(1024))) int8_t stage0[2 * C::OPER];
+    __shared__ __attribute__((aligned(1024))) int8_t stage1[2 * C::OPER];
+    // Edge tiles (M or N not a multiple of 256): rows past M / N load as
+    // zeros (past the buffer resources' byte counts; RRR B columns past N
+    // read the next k-row, reaching only output columns that are not stored).
+    int tm, tn;
+    tile_coords(blockIdx.x, (p.M + C::TB - 1) / C::TB, (p.N + C::TB - 1) / C::TB, tm, tn);
+    const int m_base = tm * C::TB, n_base = tn * C::TB;
+    M2::AccTile<P> acc;
+    if constexpr (LAYOUT == F8_RCR) {
+        M2::DmaRows<false, false> d;
+        d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
+        d.b = M2::make_dma_interior<C>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb);
+        M2::mainloop<P>(stage0, stage1, d, p.K, acc);
+    } else {
+        M2::DmaRowsRrr d;
+        d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
+        d.b = M2::make_dma_row_b<C>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base);
+        M2::mainloop<P>(stage0, stage1, d, p.K, acc);
+    }
+    f8_store_tile<FMT, EPI, ACT, P>(acc, M2::wave_scratch<C>(stage0, stage1), p, m_base, n_base);
+}
+
+// RCR on the tiles of gemm_ring.hpp: C's block tile over a ring of DEPTH
+// stages (dynamic LDS of DEPTH * C::STAGE bytes), SPREAD MFMAs per DMA; wave
+// tiles below 64 rows multiply 16 x 16 x 128.
+template <int FMT, int EPI, int ACT, class C, int DEPTH, int SPREAD>
+__global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_ring_kernel(F8Args p) {
+    namespace M2 = mfma2;
+    typedef std::conditional_t<(C::WM < 64), M2::PolicyF8x16<C, FMT>, M2::PolicyF8<C, FMT>> P;
+    constexpr int SCRATCH = DEPTH * C::STAGE / C::WAVES;   // bytes per wave after the loop
+    static_assert(SCRATCH >= C::WM * 128 && SCRATCH >= 16 * 256 && SCRATCH % 1024 == 0, "staged stores");
+    extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+    int tm, tn;
+    tile_coords(blockIdx.x, (p.M + C::TB - 1) / C::TB, (p.N + C::TBN - 1) / C::TBN, tm, tn);
+    const int m_base = tm * C::TB, n_base = tn * C::TBN;
+    M2::DmaRows<false, false> d;
+    d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
+    d.b = M2::make_dma_interior<C, C::ROWS_PER_WAVE_B>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb);
+    M2::AccTile<P> acc;
+    M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    f8_store_tile<FMT, EPI, ACT, P>(acc, lds + (threadIdx.x >> 6) * SCRATCH, p, m_base, n_base);
+}
+
 // RCR last rows (1 to 16 RF of them, m0 = the first): A and B streamed
 // through LDS in K stages of SB bytes, DEPTH stages in flight.  A workgroup
 // of 16 waves owns 16 NB output columns; each stage holds its 16 RF A rows
@@ -260,7 +290,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_dma_kern
 // first operand, so lane l ends with A row l % 16 and columns 4 (l / 16) ..
 // + 3).  The CH chunk partials of a fragment pair are added in chunk order
 // through LDS and the waves run the tiles' epilogue, one fragment pair at a
-// time.  Requirements (checked by the launcher): K % SB == 0, the fast
+// time.  Requirements (checked by the launcher): K % 16 == 0, the fast
 // path's alignment and 2^31 extents, N % (16 NB) == 0; dynamic LDS of
 // DEPTH * (16 RF + 16 NB) * SB bytes.
 //
@@ -309,19 +339,22 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
             const int idx = 64 * j + lane;
             const int r = idx / UPR, slot = idx % UPR;
             const int unit = slot ^ (r & 15);
+            // units at or past K (a partial last stage) land as zeros
+            const bool past = k0 + 16 * unit >= p.K;
             if (r < 16 * RF) {
-                mfma2::dma16(ra, (int)((int64_t)(m0 + r) * p.lda) + 16 * unit, k0, buf + j * 1024);
+                mfma2::dma16(ra, past ? mfma2::kPastExtent : (int)((int64_t)(m0 + r) * p.lda) + 16 * unit, k0, buf + j * 1024);
             } else if constexpr (RowB) {
                 const int ib = idx - 16 * RF * UPR;   // unit of the B region: k-row ib / NB
                 mfma2::dma16(rb, (ib / NB) * (int)p.ldb + n0 + 16 * (ib % NB),
                              __builtin_amdgcn_readfirstlane(k0 * (int)p.ldb), buf + j * 1024);
             } else {
-                mfma2::dma16(rb, (int)((int64_t)(n0 + r - 16 * RF) * p.ldb) + 16 * unit, k0, buf + j * 1024);
+                mfma2::dma16(rb, past ? mfma2::kPastExtent : (int)((int64_t)(n0 + r - 16 * RF) * p.ldb) + 16 * unit, k0,
+                             buf + j * 1024);
             }
         }
     };
     const bool hi = NI % WAVES == 0 || wave < NI % WAVES;
-    const int ns = p.K / SB;
+    const int ns = (p.K + SB - 1) / SB;
     for (int st = 0; st < DEPTH && st < ns; ++st) dma_stage(st, lds + st * STAGE);
     const int c = wave % CH, f0 = wave / CH;
     const bool active = ALL || wave < RF * CH;   // wave-uniform
@@ -391,7 +424,7 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
     }
 }
 
-// One last row (M = 1 decode steps; K % (1024 BT) == 0), no MFMA: a
+// One last row (M = 1 decode steps; K % 16 == 0, % 2048 for BT = 2), no MFMA: a
 // workgroup of 4 waves owns 4 output columns and wave w streams B row
 // n0 + w over all of K, 16 bytes per lane of every kilobyte straight into
 // registers (BT kilobytes requested before their products), beside the same
@@ -416,6 +449,23 @@ __global__ __launch_bounds__(256) void gemm_fp8_rcr_row1_kernel(F8Args p, int m0
     const int8_t *brow = p.b + (int64_t)(n0 + wave) * p.ldb + lane * 16;
     const int8_t *arow = p.a + (int64_t)m0 * p.lda + lane * 16;
     float acc0 = 0.0f, acc1 = 0.0f;
+    auto add16 = [&](const v4i &av, const v4i &bv) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const v2f a0 = fp8x2_to_f32<FMT, false>(av[q]), b0 = fp8x2_to_f32<FMT, false>(bv[q]);
+            const v2f a1 = fp8x2_to_f32<FMT, true>(av[q]), b1 = fp8x2_to_f32<FMT, true>(bv[q]);
+            acc0 = __builtin_fmaf(a0[0], b0[0], acc0);
+            acc1 = __builtin_fmaf(a0[1], b0[1], acc1);
+            acc0 = __builtin_fmaf(a1[0], b1[0], acc0);
+            acc1 = __builtin_fmaf(a1[1], b1[1], acc1);
+        }
+    };
+    if constexpr (BT == 1) {
+        // the part of a kilobyte at the end of K % 1024 != 0
+        if (nch * 1024 + lane * 16 < p.K)
+            add16(*reinterpret_cast<const v4i *>(arow + (int64_t)nch * 1024),
+                  __builtin_nontemporal_load(reinterpret_cast<const v4i *>(brow + (int64_t)nch * 1024)));
+    }
     for (int c0 = 0; c0 < nch; c0 += BT) {
         v4i av[BT], bv[BT];
 #pragma unroll
@@ -426,17 +476,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_rcr_row1_kernel(F8Args p, int m0
             bv[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(brow + (int64_t)(c0 + u) * 1024));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < BT; ++u)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const v2f a0 = fp8x2_to_f32<FMT, false>(av[u][q]), b0 = fp8x2_to_f32<FMT, false>(bv[u][q]);
-                const v2f a1 = fp8x2_to_f32<FMT, true>(av[u][q]), b1 = fp8x2_to_f32<FMT, true>(bv[u][q]);
-                acc0 = __builtin_fmaf(a0[0], b0[0], acc0);
-                acc1 = __builtin_fmaf(a0[1], b0[1], acc1);
-                acc0 = __builtin_fmaf(a1[0], b1[0], acc0);
-                acc1 = __builtin_fmaf(a1[1], b1[1], acc1);
-            }
+        for (int u = 0; u < BT; ++u) add16(av[u], bv[u]);
     }
     float acc = acc0 + acc1;
 #pragma unroll
@@ -459,16 +499,16 @@ __global__ __launch_bounds__(256) void gemm_fp8_rcr_row1_kernel(F8Args p, int m0
 // columns 24.2-25.9).  16 columns (N below 6144): 1 fragment with 2 KiB
 // stages, 2 with 1 KiB stages three deep, 4 and 8 with 512-byte stages.
 template <int FMT, int EPI, int ACT>
-bool launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
+void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
     // one row: the FMA row kernel (K = 4096 over rotated weights, graph
     // replay: N = 14336 13.4 -> 10.4 us, N = 4096 5.2 -> 4.8 us against the
     // staged kernel)
-    if (rem == 1 && p.K % 1024 == 0) {
+    if (rem == 1) {
         if (p.K % 2048 == 0)
             hipLaunchKernelGGL((gemm_fp8_rcr_row1_kernel<FMT, EPI, ACT, 2>), dim3(p.N / 4), dim3(256), 0, stream, p, m0);
         else
             hipLaunchKernelGGL((gemm_fp8_rcr_row1_kernel<FMT, EPI, ACT, 1>), dim3(p.N / 4), dim3(256), 0, stream, p, m0);
-        return true;
+        return;
     }
     if (rem > 32 && mfma2::last_rows_col_frags(p.N) == 1) {
         // 33-128 rows below N = 6144 as row blocks (mfma2::last_rows_blocks);
@@ -480,11 +520,11 @@ bool launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
         int rf, blk, nbb;
         mfma2::last_rows_blocks(rem, p.N, rf, blk, nbb);
 #define BK_F8RB(RF, NB, SB, DEPTH)                                                                        \
-        if (rf == (RF) && nbb == (NB) && p.K % (SB) == 0) {                                                  \
+        if (rf == (RF) && nbb == (NB)) {                                                  \
             hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH>),           \
                                dim3(p.N / (16 * (NB)), blk), dim3(1024), (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), \
                                stream, p, m0);                                                               \
-            return true;                                                                                     \
+            return;                                                                                     \
         }
         BK_F8RB(4, 1, 512, 2) BK_F8RB(4, 2, 512, 2) BK_F8RB(4, 4, 512, 2)
         BK_F8RB(2, 1, 1024, 3) BK_F8RB(2, 2, 1024, 2)
@@ -492,11 +532,11 @@ bool launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
     }
     const int nb = mfma2::last_rows_col_frags(p.N);
 #define BK_F8ROWS(RF, NB, SB, DEPTH)                                                                     \
-    if (rem <= 16 * (RF) && nb == (NB) && p.K % (SB) == 0) {                                              \
+    if (rem <= 16 * (RF) && nb == (NB)) {                                              \
         hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH>),           \
                            dim3(p.N / (16 * (NB))), dim3(1024), (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), \
                            stream, p, m0);                                                               \
-        return true;                                                                                     \
+        return;                                                                                     \
     }
     // up to 16 / 32 rows at 32 or 64 columns: 1 / 2 fragments, 4 / 8 waves
     // with MFMA work (padding A rows cost DMA and LDS time: N = 14336, M = 2
@@ -515,7 +555,88 @@ bool launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
     BK_F8ROWS(4, 1, 512, 2)
     BK_F8ROWS(8, 1, 512, 2)
 #undef BK_F8ROWS
+}
+
+template <int FMT, int EPI, int ACT, class C, int DEPTH, int SPREAD>
+void launch_fp8_ring(const F8Args &p, hipStream_t stream) {
+    const int tiles = ((p.M + C::TB - 1) / C::TB) * ((p.N + C::TBN - 1) / C::TBN);
+    hipLaunchKernelGGL((gemm_fp8_ring_kernel<FMT, EPI, ACT, C, DEPTH, SPREAD>), dim3(tiles), dim3(C::NT),
+                       (size_t)DEPTH * C::STAGE, stream, p);
+}
+
+// All of M as RCR tiles of the cheapest shape (mfma2::ring_tile).
+template <int FMT, int EPI, int ACT>
+void launch_fp8_tiles(const F8Args &p, hipStream_t stream) {
+    using mfma2::Cfg;
+    switch (mfma2::ring_tile(p.M, p.N, p.K)) {
+        case mfma2::RT_64x64: return launch_fp8_ring<FMT, EPI, ACT, Cfg<4, 1, 64, 64>, 4, 0>(p, stream);
+        case mfma2::RT_64x128: return launch_fp8_ring<FMT, EPI, ACT, Cfg<2, 2, 64, 128>, 3, 1>(p, stream);
+        case mfma2::RT_128x128: return launch_fp8_ring<FMT, EPI, ACT, Cfg<4, 2, 128, 128>, 3, 1>(p, stream);
+        case mfma2::RT_128x256: return launch_fp8_ring<FMT, EPI, ACT, Cfg<2, 4, 128, 256>, 3, 1>(p, stream);
+        case mfma2::RT_192x256: return launch_fp8_ring<FMT, EPI, ACT, Cfg<2, 4, 192, 256>, 2, 0>(p, stream);
+        default: break;
+    }
+    const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+    hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, F8_RCR, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT), 0, stream, p);
+}
+
+// Every RCR row as row blocks of the last-rows kernel, 64-row blocks first
+// while they fit one round of workgroups (K = 4096, M = 129 / 256: N = 2048
+// 9.6 / 10.1 -> 7.9 / 8.1 us against 128-row blocks); false when they exceed
+// one round.
+template <int FMT, int EPI, int ACT>
+bool launch_fp8_row_blocks(const F8Args &p, hipStream_t stream) {
+    const int b4 = (p.M + 63) / 64;
+    const int n4 = mfma2::last_rows_col_frags(p.N, b4);
+    if (b4 * (p.N / (16 * n4)) <= 256) {
+#define BK_F8BLK4(NB)                                                                                     \
+        if (n4 == (NB)) {                                                                                 \
+            hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, 4, NB, 512, 2>),            \
+                               dim3(p.N / (16 * (NB)), b4), dim3(1024), (size_t)2 * (64 + 16 * (NB)) * 512, \
+                               stream, p, 0);                                                             \
+            return true;                                                                                  \
+        }
+        BK_F8BLK4(1) BK_F8BLK4(2) BK_F8BLK4(4)
+#undef BK_F8BLK4
+    }
+    const int blocks = (p.M + 127) / 128;
+    const int nb = mfma2::last_rows_col_frags(p.N, blocks);
+    if (blocks * (p.N / (16 * nb)) > 256) return false;
+#define BK_F8BLOCKS(NB, SB)                                                                              \
+    if (nb == (NB)) {                                                                                    \
+        hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, 8, NB, SB, 2>),                \
+                           dim3(p.N / (16 * (NB)), blocks), dim3(1024),                                  \
+                           (size_t)2 * (128 + 16 * (NB)) * (SB), stream, p, 0);                          \
+        return true;                                                                                     \
+    }
+    BK_F8BLOCKS(1, 512)
+    BK_F8BLOCKS(2, 512)
+    BK_F8BLOCKS(4, 256)
+#undef BK_F8BLOCKS
     return false;
+}
+
+// RCR: last rows, row blocks or tiles, by the int8 kernel's rules.
+template <int FMT, int EPI, int ACT>
+void launch_fp8_rcr(const F8Args &p, hipStream_t stream) {
+    const int rem = mfma2::last_rows_pass(p.M, p.N, 128);
+    if (rem == p.M) {
+        if (rem > 32 && !mfma2::few_tiles(p.M, p.N)) launch_fp8_tiles<FMT, EPI, ACT>(p, stream);
+        else launch_fp8_rows<FMT, EPI, ACT>(p, 0, rem, stream);
+        return;
+    }
+    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && mfma2::few_tiles(p.M, p.N) &&
+        launch_fp8_row_blocks<FMT, EPI, ACT>(p, stream))
+        return;
+    if (rem != 0 && mfma2::last_rows_pay(p.M, p.N, p.K, rem)) {
+        F8Args pm = p;
+        pm.M = p.M - rem;
+        const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+        hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, F8_RCR, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT), 0, stream, pm);
+        launch_fp8_rows<FMT, EPI, ACT>(p, pm.M, rem, stream);
+        return;
+    }
+    launch_fp8_tiles<FMT, EPI, ACT>(p, stream);
 }
 
 template <int FMT, int LAYOUT, int EPI, int ACT>
@@ -528,10 +649,10 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
     const int64_t pad_m = (int64_t)((p.M + mfma2::BM - 1) / mfma2::BM) * mfma2::BM;
     const int64_t pad_b = LAYOUT == F8_RCR ? (int64_t)((p.N + mfma2::BN - 1) / mfma2::BN) * mfma2::BN * p.ldb
                                            : b_rows * p.ldb + mfma2::BN;
-    const bool fast = p.K % mfma2::BK == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) &&
+    const bool fast = p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) &&
                       aligned16(p.b) && p.N % 4 == 0 && pad_m * p.lda < (1ll << 31) && pad_b < (1ll << 31) &&
                       p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % (4 * out_elem)) == 0;
-    if (fast && LAYOUT == F8_RRR && p.K % 512 == 0 && (int64_t)p.K * p.ldb + mfma2::BN < (1ll << 31)) {
+    if (fast && LAYOUT == F8_RRR) {
         // RRR last rows: the staged kernel reading row-major B, column groups
         // by the last-rows rule (XCD-major in the kernel)
         const int rem = mfma2::last_rows_pass(p.M, p.N, 128);
@@ -571,7 +692,7 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
                 int rf, blk, nbb;
                 mfma2::last_rows_blocks(rem, p.N, rf, blk, nbb);
 #define BK_F8RRRB(RF, NB, SB, DEPTH)                                                                      \
-                if (rf == (RF) && nbb == (NB) && p.K % (SB) == 0) {                                          \
+                if (rf == (RF) && nbb == (NB)) {                                                             \
                     hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH, true>), \
                                        dim3(p.N / (16 * (NB)), blk), dim3(1024),                             \
                                        (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), stream, p, pm.M);   \
@@ -608,71 +729,14 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
 #undef BK_F8RRRROWS
         }
     }
-    if (fast && LAYOUT == F8_RCR && p.M > 128 && p.M <= 512 && p.K % 512 == 0 && p.N % 16 == 0 &&
-        mfma2::last_rows_pass(p.M, p.N, 128) == 0) {
-        // small problems whose 128-row blocks of the last-rows kernel fit one
-        // round of workgroups: all rows that way instead of tiles.  K = 4096,
-        // M = 129 / 256 / 512: N = 4096 12.6 / 13.2 / 18.6 us against 23.9 /
-        // 24.2 / 24.3 on 128x128 tiles; N = 8192, M = 129 / 256: 17.5 / 18.6
-        // against 28.2 / 28.6
-        // 64-row blocks first while they fit one round (K = 4096, M = 129 /
-        // 256: N = 4096 12.3 / 12.8 -> 11.2 / 11.7 us, N = 2048 9.6 / 10.1
-        // -> 7.9 / 8.1 us; N = 8192 level), else 128-row blocks
-        const int b4 = (p.M + 63) / 64;
-        const int n4 = mfma2::last_rows_col_frags(p.N, b4);
-        if (b4 * (p.N / (16 * n4)) <= 256) {
-#define BK_F8BLK4(NB)                                                                                     \
-            if (n4 == (NB)) {                                                                             \
-                hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, 4, NB, 512, 2>),        \
-                                   dim3(p.N / (16 * (NB)), b4), dim3(1024), (size_t)2 * (64 + 16 * (NB)) * 512, \
-                                   stream, p, 0);                                                         \
-                return launch_status();                                                                   \
-            }
-            BK_F8BLK4(1) BK_F8BLK4(2) BK_F8BLK4(4)
-#undef BK_F8BLK4
-        }
-        const int blocks = (p.M + 127) / 128;
-        const int nb = mfma2::last_rows_col_frags(p.N, blocks);
-        if (blocks * (p.N / (16 * nb)) <= 256) {
-#define BK_F8BLOCKS(NB, SB)                                                                              \
-            if (nb == (NB)) {                                                                            \
-                hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, 8, NB, SB, 2>),        \
-                                   dim3(p.N / (16 * (NB)), blocks), dim3(1024),                          \
-                                   (size_t)2 * (128 + 16 * (NB)) * (SB), stream, p, 0);                  \
-                return launch_status();                                                                  \
-            }
-            BK_F8BLOCKS(1, 512)
-            BK_F8BLOCKS(2, 512)
-            BK_F8BLOCKS(4, 256)
-#undef BK_F8BLOCKS
-        }
-    }
-    if (fast && LAYOUT == F8_RCR) {
-        // the last rows as their own pass when a row of tiles would start
-        // another round (decode-sized M: all of it)
-        const int rem = mfma2::last_rows_pass(p.M, p.N, 128);
-        if (rem != 0 && p.K % 512 == 0) {
-            F8Args pm = p;
-            pm.M = p.M - rem;
-            const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-            if (tiles > 0)
-                hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, LAYOUT, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT),
-                                   0, stream, pm);
-            if (launch_fp8_rows<FMT, EPI, ACT>(p, pm.M, rem, stream)) return launch_status();
-            // K % 512 == 0 always finds a stage shape
+    if constexpr (LAYOUT == F8_RCR) {
+        if (fast) {
+            launch_fp8_rcr<FMT, EPI, ACT>(p, stream);
+            return launch_status();
         }
     }
     if (fast) {
         const int tiles = (int)(pad_m / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-        if (LAYOUT == F8_RCR && tiles <= 128) {
-            // at most half a round of 256x256 tiles: 128x128 tiles of 4 waves
-            // (two workgroups per CU), as the int8 kernel
-            typedef mfma2::Cfg<2, 2, 128> SmallCfg;
-            const int tiles128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
-            hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, F8_RCR, EPI, ACT, SmallCfg>), dim3(tiles128),
-                               dim3(SmallCfg::NT), 0, stream, p);
-            return launch_status();
-        }
         hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, LAYOUT, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT),
                            0, stream, p);
     } else {

@@ -89,6 +89,7 @@ struct PolicyI8 {
     template <class F> __device__ static void fixup(F &, Sums &) {}
     __device__ static void stage_hook(const int8_t *, Sums &) {}
 
+    static constexpr int SUBS = 2;           // sub-steps (fragment sets) per 128-byte stage
     static constexpr int TI = C::WM / 16;    // 16x16 tiles per wave along M
     static constexpr int TJ = C::WN / 16;    // ... along N
     typedef v4i Acc;
@@ -181,6 +182,7 @@ struct PolicyF8 {
     template <class F> __device__ static void fixup(F &, Sums &) {}
     __device__ static void stage_hook(const int8_t *, Sums &) {}
 
+    static constexpr int SUBS = 2;
     static constexpr int TI = C::WM / 32;
     static constexpr int TJ = C::WN / 32;
     typedef v16f Acc;
@@ -208,6 +210,34 @@ struct PolicyF8 {
         for (int g = 0; g < 4; ++g)
             f(i * 32 + (lane & 31), j * 32 + g * 8 + (lane >> 5) * 4,
               v4f{c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]});
+    }
+};
+
+// fp8: v_mfma_f32_16x16x128_f8f6f4 for wave tiles of fewer than 64 rows, one
+// instruction per 128-byte stage and pair of 16-row fragments: lane l
+// supplies row l % 16, bytes 32 (l / 16) .. + 31 of the stage.
+template <class C, int FMT = 0>
+struct PolicyF8x16 : PolicyI8<C> {
+    static constexpr int SUBS = 1;
+    typedef v4f Acc;
+    typedef v8i Frag;
+    __device__ static Frag load(const int8_t *op, int row0, int t, int, int lane) {
+        const int row = row0 + t * 16 + (lane & 15);
+        const int u = (lane >> 4) * 2;
+        const v4i lo = *reinterpret_cast<const v4i *>(op + lds_off(row, u));
+        const v4i hi = *reinterpret_cast<const v4i *>(op + lds_off(row, u + 1));
+        return Frag{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+    __device__ static Frag load_b(const int8_t *op, int row0, int t, int s, int lane) {
+        return load(op, row0, t, s, lane);
+    }
+    __device__ static void mma(Acc &c, const Frag &b, const Frag &a, int) {
+        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, a, c, FMT, FMT, 0, 0, 0, 0);
+    }
+    __device__ static Acc zero() { return Acc{0.0f, 0.0f, 0.0f, 0.0f}; }
+    template <class F>
+    __device__ static void visit(const Acc &c, int i, int j, int lane, F &&f) {
+        f(i * 16 + (lane & 15), j * 16 + (lane >> 4) * 4, c);
     }
 };
 

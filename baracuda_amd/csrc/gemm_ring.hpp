@@ -44,12 +44,12 @@ __device__ __forceinline__ void dma_pieces(int8_t *stage, const D &d, int kbyte)
     }
 }
 
-// MFMA t of a stage's two sub-steps, then the DMA pieces due after it.
+// MFMA t of a stage's sub-steps, then the DMA pieces due after it.
 template <class P, int T, int SPREAD, class D>
 __device__ __forceinline__ void ring_mma(AccTile<P> &acc, const Frags<P> &f0, const Frags<P> &f1, int8_t *nxt, const D &d,
                                          int kbyte) {
     typedef typename P::Cfg C;
-    constexpr int SUB = P::H * P::TI * P::TJ, TOT = 2 * SUB, NI = C::DMA_PER_STAGE;
+    constexpr int SUB = P::H * P::TI * P::TJ, TOT = P::SUBS * SUB, NI = C::DMA_PER_STAGE;
     if constexpr (T < TOT) {
         constexpr int r = T % SUB, h = r / (P::TI * P::TJ), j = r / P::TI % P::TJ, i = r % P::TI;
         const Frags<P> &f = T < SUB ? f0 : f1;
@@ -107,13 +107,13 @@ __device__ __forceinline__ void mainloop_ring(int8_t *lds, D d, int K, AccTile<P
         __syncthreads();
         const int8_t *st = lds + cur;
         load_frags<P>(f0, st, 0, wave_m, wave_n, lane);
-        load_frags<P>(f1, st, 1, wave_m, wave_n, lane);
+        if constexpr (P::SUBS == 2) load_frags<P>(f1, st, 1, wave_m, wave_n, lane);
         if constexpr (SPREAD == 0) {
             __builtin_amdgcn_sched_barrier(0);
             dma_pieces<C, 0, NI>(lds + nxt, d, (kt + DEPTH - 1) * BK);
             __builtin_amdgcn_sched_barrier(0);
             mma_block<P, 0, P::TJ>(acc, f0);
-            mma_block<P, 0, P::TJ>(acc, f1);
+            if constexpr (P::SUBS == 2) mma_block<P, 0, P::TJ>(acc, f1);
         } else {
             ring_mma<P, 0, SPREAD>(acc, f0, f1, lds + nxt, d, (kt + DEPTH - 1) * BK);
         }
@@ -169,6 +169,24 @@ inline RingTile ring_tile(int M, int N, int kbytes, float *cost = nullptr) {
     }
     if (cost) *cost = us;
     return (RingTile)best;
+}
+
+// Row blocks of the staged last-rows kernels instead of tiles (33-512 rows)
+// where 64 x 64 tiles would leave half of the CUs idle: they split K over
+// their waves, which a tile does not.  us, int8, blocks against the best
+// tile: 200 x 1024 x 4096 7.0 / 9.8, 128 x 4096 x 4096 8.5 / 10.0, 512 x 1024
+// x 4096 8.3 / 10.1, 128 x 4096 x 14336 25.9 / 33; past the line 200 x 4096 x
+// 4096 11.5 / 10.2, 384 x 2048 x 1024 5.7 / 4.9, 128 x 8192 x 4096 14.9 /
+// 11.7, 64 x 14336 x 4096 17.8 / 15.7.
+inline bool few_tiles(int M, int N) { return (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 128; }
+
+// Whole 256-row tiles and a last-rows pass for more than 512 rows, against
+// the cheapest tile over all rows: the pass reads the weights once more, at
+// about 3.6 TB/s behind the tiles, and takes at least a launch.
+inline bool last_rows_pay(int M, int N, int kbytes, int rem) {
+    float all;
+    ring_tile(M, N, kbytes, &all);
+    return ring_cost(kRingCost[RT_256x256], M - rem, N, kbytes) + 3.0f + (float)N * (float)kbytes / 3.6e6f < all;
 }
 
 }  // namespace mfma2

@@ -1633,24 +1633,6 @@ void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
 #undef BK_S8ROWS
 }
 
-// Row blocks of the staged last-rows kernel instead of tiles (33-512 rows)
-// where 64 x 64 tiles would leave half of the CUs idle: they split K over
-// their waves, which a tile does not.  us, blocks against the best tile: 200 x
-// 1024 x 4096 7.0 / 9.8, 128 x 4096 x 4096 8.5 / 10.0, 512 x 1024 x 4096 8.3 /
-// 10.1, 128 x 4096 x 14336 25.9 / 33; past the line 200 x 4096 x 4096 11.5 /
-// 10.2, 384 x 2048 x 1024 5.7 / 4.9, 128 x 8192 x 4096 14.9 / 11.7, 64 x
-// 14336 x 4096 17.8 / 15.7.
-inline bool few_tiles(int M, int N) { return (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 128; }
-
-// Whole 256-row tiles and a last-rows pass for more than 512 rows, against
-// the cheapest tile over all rows: the pass reads the weights once more, at
-// about 3.6 TB/s behind the tiles, and takes at least a launch.
-inline bool last_rows_pay(int M, int N, int K, int rem) {
-    float all;
-    mfma2::ring_tile(M, N, K, &all);
-    return mfma2::ring_cost(mfma2::kRingCost[mfma2::RT_256x256], M - rem, N, K) + 3.0f + (float)N * (float)K / 3.6e6f < all;
-}
-
 template <int EPI, bool VecOut, int ACT, typename BiasT>
 void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *workspace, size_t workspace_bytes) {
     if (!fast_k) {
@@ -1671,14 +1653,14 @@ void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *works
     }
     const int rem = rows_path_rows(p.M, p.N);
     if (rem == p.M) {
-        if (VecOut && rem > 32 && !few_tiles(p.M, p.N)) launch_tiles<EPI, VecOut, ACT, BiasT>(p, stream);
+        if (VecOut && rem > 32 && !mfma2::few_tiles(p.M, p.N)) launch_tiles<EPI, VecOut, ACT, BiasT>(p, stream);
         else launch_last_rows<EPI, VecOut, ACT, BiasT>(p, 0, rem, stream);
         return;
     }
-    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && (!VecOut || few_tiles(p.M, p.N)) &&
+    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && (!VecOut || mfma2::few_tiles(p.M, p.N)) &&
         launch_row_blocks<EPI, VecOut, ACT, BiasT>(p, stream))
         return;
-    if (rem != 0 && (!VecOut || last_rows_pay(p.M, p.N, p.K, rem))) {
+    if (rem != 0 && (!VecOut || mfma2::last_rows_pay(p.M, p.N, p.K, rem))) {
         S8Args pm = p;
         pm.M = p.M - rem;
         const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);

@@ -12,7 +12,8 @@ import torch
 from baracuda_amd import plans as P
 from baracuda_amd.ffi import lib
 from oracle.inputs import int8_uniform, rng
-from tests.gpu_util import dev, host_bits16, sync
+from tests import test_gpu_sweep as S
+from tests.gpu_util import FP8_FLOOR, dev, host_bits16, sync
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +83,39 @@ def test_int8_depth_tail_reads_stay_in_the_row(gpu, shape):
         dev(pa)[:, :k], dev(pb)[:, :k], d)
     sync()
     assert np.array_equal(d.cpu().numpy(), _acc(np.ascontiguousarray(pa[:, :k]), np.ascontiguousarray(pb[:, :k])))
+
+
+@pytest.mark.parametrize("shape", TILE_SHAPES + ROW_SHAPES)
+def test_fp8_tiles_and_depth_tails(gpu, shape):
+    """e4m3 RCR: f32 out within the FP8 tolerance, bf16 out its rounding; what
+    lies past K in a row (NaN codes here) stays out."""
+    m, n, k = shape
+    print(f"case: fp8 tiles {shape}", flush=True)
+    g = rng(m + 5 * n + 3 * k)
+
+    def operand(rows, pad):
+        x = torch.from_numpy(g.standard_normal((rows, k)).astype(np.float32) * 100)
+        x = x.clamp(-448, 448).to(torch.float8_e4m3fn)      # past 464 torch casts to NaN
+        t = torch.full((rows, k + pad), 0x7f, dtype=torch.uint8)
+        t[:, :k] = x.view(torch.uint8)
+        return x.double(), t.to("cuda:0")[:, :k]
+
+    xa, ta = operand(m, 112)
+    xb, tb = operand(n, 48)
+    d = torch.zeros((m, n), dtype=torch.float32, device="cuda:0")
+    P.Fp8GemmPlan.select(P.Fp8GemmDescriptor(m, n, k, output=P.ElementKind.F32)).run(ta, tb, d, alpha=0.5)
+    db = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda:0")
+    P.Fp8GemmPlan.select(P.Fp8GemmDescriptor(m, n, k, output=P.ElementKind.Bf16)).run(
+        ta, tb, db, scale_a=0.5, scale_b=1.0)
+    sync()
+    got, exact = d.cpu().double(), 0.5 * (xa @ xb.T)
+    bound = 1e-3 * exact.abs() + FP8_FLOOR * 0.5 * (xa.abs() @ xb.abs().T)
+    assert bool(((got - exact).abs() <= bound).all())
+    assert torch.equal(db.cpu(), d.cpu().to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("shape", [(300, 1696, 208), (900, 2064, 400), (13, 6160, 1552), (100, 272, 656),
+                                   (200, 1024, 1072), (4160, 4096, 144)])
+@pytest.mark.parametrize("fmt,layout", [("e4m3", P.LayoutSku.Rrr), ("e5m2", P.LayoutSku.Rcr)])
+def test_fp8_out_depth_tails(gpu, shape, fmt, layout):
+    S.test_fp8_out_with_c_sweep(gpu, shape, fmt, layout)
