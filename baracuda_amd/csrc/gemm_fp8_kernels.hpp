@@ -226,7 +226,7 @@ __device__ __forceinline__ void f8_store_tile(const mfma2::AccTile<P> &acc, int8
     M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4f &v) { epi(m_base + ml, n_base + nl, v); });
 }
 
-// Fast path: 256x256 tiles (edge tiles included), K % 16 == 0, 16-byte rows,
+// Fast path: 256x256 tiles (edge tiles included), K % 128 == 0, 16-byte rows,
 // N % 4 == 0, vector stores.
 template <int FMT, int LAYOUT, int EPI, int ACT>
 __global__ __launch_bounds__(F8DmaCfg::NT, 1) void gemm_fp8_dma_kernel(F8Args p) {
@@ -256,24 +256,36 @@ __global__ __launch_bounds__(F8DmaCfg::NT, 1) void gemm_fp8_dma_kernel(F8Args p)
     f8_store_tile<FMT, EPI, ACT, P>(acc, M2::wave_scratch<C>(stage0, stage1), p, m_base, n_base);
 }
 
-// RCR on the tiles of gemm_ring.hpp: C's block tile over a ring of DEPTH
-// stages (dynamic LDS of DEPTH * C::STAGE bytes), SPREAD MFMAs per DMA; wave
-// tiles below 64 rows multiply 16 x 16 x 128.
-template <int FMT, int EPI, int ACT, class C, int DEPTH, int SPREAD>
+template <int FMT, int LAYOUT, class C>
+struct F8RingPolicy {
+    typedef std::conditional_t<(C::WM < 64), mfma2::PolicyF8x16<C, FMT>, mfma2::PolicyF8<C, FMT>> type;
+};
+template <int FMT, class C>
+struct F8RingPolicy<FMT, F8_RRR, C> { typedef mfma2::PolicyF8RowB<C, FMT> type; };
+
+// The tiles of gemm_ring.hpp: C's block tile over a ring of DEPTH stages
+// (dynamic LDS of DEPTH * C::STAGE bytes), SPREAD MFMAs per DMA; RCR wave
+// tiles below 64 rows multiply 16 x 16 x 128, RRR tiles are 256 columns wide.
+template <int FMT, int LAYOUT, int EPI, int ACT, class C, int DEPTH, int SPREAD>
 __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_ring_kernel(F8Args p) {
     namespace M2 = mfma2;
-    typedef std::conditional_t<(C::WM < 64), M2::PolicyF8x16<C, FMT>, M2::PolicyF8<C, FMT>> P;
+    typedef typename F8RingPolicy<FMT, LAYOUT, C>::type P;
     constexpr int SCRATCH = DEPTH * C::STAGE / C::WAVES;   // bytes per wave after the loop
     static_assert(SCRATCH >= C::WM * 128 && SCRATCH >= 16 * 256 && SCRATCH % 1024 == 0, "staged stores");
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
     int tm, tn;
     tile_coords(blockIdx.x, (p.M + C::TB - 1) / C::TB, (p.N + C::TBN - 1) / C::TBN, tm, tn);
     const int m_base = tm * C::TB, n_base = tn * C::TBN;
-    M2::DmaRows<false, false> d;
-    d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-    d.b = M2::make_dma_interior<C, C::ROWS_PER_WAVE_B>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb);
     M2::AccTile<P> acc;
-    M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    const auto a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
+    if constexpr (LAYOUT == F8_RRR) {
+        const M2::DmaRowsRrr d{a, M2::make_dma_row_b<C>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base)};
+        M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    } else {
+        const M2::DmaRows<false, false> d{
+            a, M2::make_dma_interior<C, C::ROWS_PER_WAVE_B>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb)};
+        M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    }
     f8_store_tile<FMT, EPI, ACT, P>(acc, lds + (threadIdx.x >> 6) * SCRATCH, p, m_base, n_base);
 }
 
@@ -313,8 +325,6 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
     constexpr int ROWS = 16 * RF + 16 * NB;              // A then B rows of a stage
     constexpr int STAGE = ROWS * SB;
     constexpr int UPR = SB / 16;                         // 16-byte units per row
-    constexpr int NI = ROWS * UPR / 64;                  // 1 KiB DMA instructions per stage
-    constexpr int HI = (NI + WAVES - 1) / WAVES, LO = NI / WAVES;
     static_assert((!ALL || RF * CH % WAVES == 0) && UPR >= 16 && (ROWS * UPR) % 64 == 0 && DEPTH >= 2 &&
                       DEPTH <= 4 && RF * NB * CH * 1024 <= DEPTH * STAGE,
                   "stage split");
@@ -329,33 +339,14 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
     // one XCD's L2) and each line is fetched once (FETCH_SIZE 2.0x -> 1.0x of B)
     const int cgroup = RowB && gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
     const int n0 = cgroup * 16 * NB;
-    const v4i ra = mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda));
-    const v4i rb = mfma2::make_rsrc(p.b, (uint32_t)(RowB ? (int64_t)p.K * p.ldb : (int64_t)p.N * p.ldb));
-    // DMA instruction j of a stage: units 64 j .. 64 j + 63 of the row-major
-    // stage, lane L fetching unit (64 j + L) % UPR of row (64 j + L) / UPR
-    auto dma_stage = [&](int st, int8_t *buf) {
-        const int k0 = st * SB;
-        for (int j = wave; j < NI; j += WAVES) {
-            const int idx = 64 * j + lane;
-            const int r = idx / UPR, slot = idx % UPR;
-            const int unit = slot ^ (r & 15);
-            // units at or past K (a partial last stage) land as zeros
-            const bool past = k0 + 16 * unit >= p.K;
-            if (r < 16 * RF) {
-                mfma2::dma16(ra, past ? mfma2::kPastExtent : (int)((int64_t)(m0 + r) * p.lda) + 16 * unit, k0, buf + j * 1024);
-            } else if constexpr (RowB) {
-                const int ib = idx - 16 * RF * UPR;   // unit of the B region: k-row ib / NB
-                mfma2::dma16(rb, (ib / NB) * (int)p.ldb + n0 + 16 * (ib % NB),
-                             __builtin_amdgcn_readfirstlane(k0 * (int)p.ldb), buf + j * 1024);
-            } else {
-                mfma2::dma16(rb, past ? mfma2::kPastExtent : (int)((int64_t)(n0 + r - 16 * RF) * p.ldb) + 16 * unit, k0,
-                             buf + j * 1024);
-            }
-        }
-    };
-    const bool hi = NI % WAVES == 0 || wave < NI % WAVES;
+    mfma2::RowsDma<16 * RF, 16 * NB, SB, RowB> dma;
+    dma.init(mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda)),
+             mfma2::make_rsrc(p.b, (uint32_t)(RowB ? (int64_t)p.K * p.ldb : (int64_t)p.N * p.ldb)),
+             [&](int r) { return (int)((int64_t)(m0 + r) * p.lda); }, n0, (int)p.ldb);
+    constexpr int HI = dma.HI, LO = dma.LO;
+    const bool hi = dma.hi();
     const int ns = (p.K + SB - 1) / SB;
-    for (int st = 0; st < DEPTH && st < ns; ++st) dma_stage(st, lds + st * STAGE);
+    for (int st = 0; st < DEPTH && st < ns; ++st) dma.issue(st, p.K, lds + st * STAGE);
     const int c = wave % CH, f0 = wave / CH;
     const bool active = ALL || wave < RF * CH;   // wave-uniform
     v4f acc[FPW][NB];
@@ -400,7 +391,7 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
         }
         }
         __syncthreads();   // every wave is done with this buffer
-        if (st + DEPTH < ns) dma_stage(st + DEPTH, buf);
+        if (st + DEPTH < ns) dma.issue(st + DEPTH, p.K, buf);
     }
     // partial sums of (A fragment f, B fragment nb), chunk c: part[f][nb][c][lane]
     v4f *part = reinterpret_cast<v4f *>(lds);
@@ -557,27 +548,35 @@ void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
 #undef BK_F8ROWS
 }
 
-template <int FMT, int EPI, int ACT, class C, int DEPTH, int SPREAD>
+template <int FMT, int LAYOUT, int EPI, int ACT, class C, int DEPTH, int SPREAD>
 void launch_fp8_ring(const F8Args &p, hipStream_t stream) {
     const int tiles = ((p.M + C::TB - 1) / C::TB) * ((p.N + C::TBN - 1) / C::TBN);
-    hipLaunchKernelGGL((gemm_fp8_ring_kernel<FMT, EPI, ACT, C, DEPTH, SPREAD>), dim3(tiles), dim3(C::NT),
+    hipLaunchKernelGGL((gemm_fp8_ring_kernel<FMT, LAYOUT, EPI, ACT, C, DEPTH, SPREAD>), dim3(tiles), dim3(C::NT),
                        (size_t)DEPTH * C::STAGE, stream, p);
 }
 
-// All of M as RCR tiles of the cheapest shape (mfma2::ring_tile).
-template <int FMT, int EPI, int ACT>
+// 256 x 256 tiles: the two-stage kernel for whole stages of K, else the ring.
+template <int FMT, int LAYOUT, int EPI, int ACT>
+void launch_fp8_tiles_256(const F8Args &p, hipStream_t stream) {
+    if (p.K % mfma2::BK != 0) return launch_fp8_ring<FMT, LAYOUT, EPI, ACT, F8DmaCfg, 2, 0>(p, stream);
+    const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+    hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, LAYOUT, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT), 0, stream, p);
+}
+
+// All of M as tiles of the cheapest shape (mfma2::ring_tile).
+template <int FMT, int LAYOUT, int EPI, int ACT>
 void launch_fp8_tiles(const F8Args &p, hipStream_t stream) {
     using mfma2::Cfg;
-    switch (mfma2::ring_tile(p.M, p.N, p.K)) {
-        case mfma2::RT_64x64: return launch_fp8_ring<FMT, EPI, ACT, Cfg<4, 1, 64, 64>, 4, 0>(p, stream);
-        case mfma2::RT_64x128: return launch_fp8_ring<FMT, EPI, ACT, Cfg<2, 2, 64, 128>, 3, 1>(p, stream);
-        case mfma2::RT_128x128: return launch_fp8_ring<FMT, EPI, ACT, Cfg<4, 2, 128, 128>, 3, 1>(p, stream);
-        case mfma2::RT_128x256: return launch_fp8_ring<FMT, EPI, ACT, Cfg<2, 4, 128, 256>, 3, 1>(p, stream);
-        case mfma2::RT_192x256: return launch_fp8_ring<FMT, EPI, ACT, Cfg<2, 4, 192, 256>, 2, 0>(p, stream);
-        default: break;
+    constexpr bool kRcr = LAYOUT == F8_RCR;
+    const mfma2::RingTile t = mfma2::ring_tile(p.M, p.N, p.K, nullptr, kRcr ? mfma2::RT_64x64 : mfma2::RT_128x256);
+    if constexpr (kRcr) {
+        if (t == mfma2::RT_64x64) return launch_fp8_ring<FMT, LAYOUT, EPI, ACT, Cfg<4, 1, 64, 64>, 4, 0>(p, stream);
+        if (t == mfma2::RT_64x128) return launch_fp8_ring<FMT, LAYOUT, EPI, ACT, Cfg<2, 2, 64, 128>, 3, 1>(p, stream);
+        if (t == mfma2::RT_128x128) return launch_fp8_ring<FMT, LAYOUT, EPI, ACT, Cfg<4, 2, 128, 128>, 3, 1>(p, stream);
     }
-    const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-    hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, F8_RCR, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT), 0, stream, p);
+    if (t == mfma2::RT_128x256) return launch_fp8_ring<FMT, LAYOUT, EPI, ACT, Cfg<2, 4, 128, 256>, 3, 1>(p, stream);
+    if (t == mfma2::RT_192x256) return launch_fp8_ring<FMT, LAYOUT, EPI, ACT, Cfg<2, 4, 192, 256>, 2, 0>(p, stream);
+    launch_fp8_tiles_256<FMT, LAYOUT, EPI, ACT>(p, stream);
 }
 
 // Every RCR row as row blocks of the last-rows kernel, 64-row blocks first
@@ -621,7 +620,7 @@ template <int FMT, int EPI, int ACT>
 void launch_fp8_rcr(const F8Args &p, hipStream_t stream) {
     const int rem = mfma2::last_rows_pass(p.M, p.N, 128);
     if (rem == p.M) {
-        if (rem > 32 && !mfma2::few_tiles(p.M, p.N)) launch_fp8_tiles<FMT, EPI, ACT>(p, stream);
+        if (rem > 32 && !mfma2::few_tiles(p.M, p.N)) launch_fp8_tiles<FMT, F8_RCR, EPI, ACT>(p, stream);
         else launch_fp8_rows<FMT, EPI, ACT>(p, 0, rem, stream);
         return;
     }
@@ -631,12 +630,11 @@ void launch_fp8_rcr(const F8Args &p, hipStream_t stream) {
     if (rem != 0 && mfma2::last_rows_pay(p.M, p.N, p.K, rem)) {
         F8Args pm = p;
         pm.M = p.M - rem;
-        const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-        hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, F8_RCR, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT), 0, stream, pm);
+        launch_fp8_tiles_256<FMT, F8_RCR, EPI, ACT>(pm, stream);
         launch_fp8_rows<FMT, EPI, ACT>(p, pm.M, rem, stream);
         return;
     }
-    launch_fp8_tiles<FMT, EPI, ACT>(p, stream);
+    launch_fp8_tiles<FMT, F8_RCR, EPI, ACT>(p, stream);
 }
 
 template <int FMT, int LAYOUT, int EPI, int ACT>
@@ -648,11 +646,11 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
     // needs whole 4-column groups (N % 4 == 0).
     const int64_t pad_m = (int64_t)((p.M + mfma2::BM - 1) / mfma2::BM) * mfma2::BM;
     const int64_t pad_b = LAYOUT == F8_RCR ? (int64_t)((p.N + mfma2::BN - 1) / mfma2::BN) * mfma2::BN * p.ldb
-                                           : b_rows * p.ldb + mfma2::BN;
+                                           : ((b_rows + mfma2::BK - 1) / mfma2::BK) * mfma2::BK * p.ldb + mfma2::BN;
     const bool fast = p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) &&
                       aligned16(p.b) && p.N % 4 == 0 && pad_m * p.lda < (1ll << 31) && pad_b < (1ll << 31) &&
                       p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % (4 * out_elem)) == 0;
-    if (fast && LAYOUT == F8_RRR) {
+    if (fast && LAYOUT == F8_RRR && mfma2::row_b_extent_ok(p.K, p.ldb, 1024)) {
         // RRR last rows: the staged kernel reading row-major B, column groups
         // by the last-rows rule (XCD-major in the kernel)
         const int rem = mfma2::last_rows_pass(p.M, p.N, 128);
@@ -682,10 +680,7 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
         if (rem != 0) {
             F8Args pm = p;
             pm.M = p.M - rem;
-            const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-            if (tiles > 0)
-                hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, LAYOUT, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT),
-                                   0, stream, pm);
+            if (pm.M > 0) launch_fp8_tiles_256<FMT, LAYOUT, EPI, ACT>(pm, stream);
             if (rem > 32 && mfma2::last_rows_col_frags(p.N) == 1) {
                 // row blocks as the RCR pass (K = 4096, M = 100: N = 4096
                 // 13.8 -> 11.7 us, N = 2048 12.8 -> 9.8 us)
@@ -736,9 +731,7 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
         }
     }
     if (fast) {
-        const int tiles = (int)(pad_m / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-        hipLaunchKernelGGL((gemm_fp8_dma_kernel<FMT, LAYOUT, EPI, ACT>), dim3(tiles), dim3(F8DmaCfg::NT),
-                           0, stream, p);
+        launch_fp8_tiles<FMT, LAYOUT, EPI, ACT>(p, stream);
     } else {
         const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
         hipLaunchKernelGGL((gemm_fp8_kernel<FMT, LAYOUT, EPI, ACT>), dim3(tiles), dim3(NT), 0, stream, p);

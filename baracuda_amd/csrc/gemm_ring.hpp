@@ -36,6 +36,22 @@ __device__ __forceinline__ void dma_piece(int8_t *stage, const DmaRows<false, fa
     }
 }
 
+// Row-major B (TBN = 256 columns, 8 waves): B pieces of four k-rows.
+template <class C, int I>
+__device__ __forceinline__ void dma_piece(int8_t *stage, const DmaRowsRrr &d, int kbyte) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int NA = C::ROWS_PER_WAVE / 8;
+    static_assert(C::TBN == BN && C::WAVES == 8, "row-major B tiles are 256 columns wide");
+    if constexpr (I < NA) {
+        const int soff = __builtin_amdgcn_readfirstlane(kbyte + I * d.a.row_stride);
+        dma16(d.a.rsrc, (I & 1) ? d.a.odd : d.a.even, soff, stage + (wave * C::ROWS_PER_WAVE + I * 8) * BK);
+    } else {
+        constexpr int J = I - NA;
+        const int soff = __builtin_amdgcn_readfirstlane((kbyte + 4 * J) * d.b.ld);
+        dma16(d.b.rsrc, (J & 1) ? d.b.odd : d.b.even, soff, stage + C::OPER + (wave * 16 + 4 * J) * BN);
+    }
+}
+
 template <class C, int I0, int I1, class D>
 __device__ __forceinline__ void dma_pieces(int8_t *stage, const D &d, int kbyte) {
     if constexpr (I0 < I1) {
@@ -157,12 +173,14 @@ inline float ring_cost(const RingCost &c, int M, int N, int kbytes) {
     return (float)pairs * (c.fixed + kt * c.paired) + (float)(per_cu % 2) * (c.fixed + kt * c.stage);
 }
 
-inline RingTile ring_tile(int M, int N, int kbytes, float *cost = nullptr) {
-    int best = 0;
+// `first`: the smallest shape the caller has (row-major B tiles are 256
+// columns wide, so they start at 128 x 256).
+inline RingTile ring_tile(int M, int N, int kbytes, float *cost = nullptr, RingTile first = RT_64x64) {
+    int best = first;
     float us = 0.0f;
-    for (int i = 0; i <= RT_256x256; ++i) {
+    for (int i = first; i <= RT_256x256; ++i) {
         const float t = ring_cost(kRingCost[i], M, N, kbytes);
-        if (i == 0 || t < us) {
+        if (i == first || t < us) {
             best = i;
             us = t;
         }

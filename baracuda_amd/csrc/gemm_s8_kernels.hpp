@@ -269,8 +269,8 @@ inline bool dma_extent_ok(int rows, int64_t ld) {
     return ((int64_t)(rows + 255) / 256) * 256 * ld < (1ll << 31);
 }
 
-// Fast path: 256x256 tiles (edge tiles read zeros past M / N, a partial last
-// stage past K), K % 16 == 0, 16-byte aligned rows ->
+// Fast path: 256x256 tiles (edge tiles read zeros past M / N), K % 128 == 0,
+// 16-byte aligned rows ->
 // LDS-DMA mainloop, 8 waves (2 x 4) of 128 x 64, v_mfma_i32_16x16x64_i8.
 typedef mfma2::Cfg<2, 4> DmaCfg;
 
@@ -486,23 +486,34 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_s8_rcr_dma_kernel(S8Args p
     s8_store_tile<EPI, VecOut, ACT, BiasT, P>(acc, M2::wave_scratch<C>(stage0, stage1), p, m_base, n_base);
 }
 
+template <class C, bool RowB>
+struct S8RingPolicy { typedef mfma2::PolicyI8<C> type; };
+template <class C>
+struct S8RingPolicy<C, true> { typedef mfma2::PolicyI8RowB<C> type; };
+
 // The same GEMM on the tiles of gemm_ring.hpp: C's block tile over a ring of
 // DEPTH stages (dynamic LDS of DEPTH * C::STAGE bytes), SPREAD MFMAs per DMA.
-template <int EPI, bool VecOut, int ACT, typename BiasT, class C, int DEPTH, int SPREAD>
-__global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_rcr_ring_kernel(S8Args p) {
+// RowB: B row-major [K, N] (the RRR SKUs; 256-column tiles).
+template <int EPI, bool VecOut, int ACT, typename BiasT, class C, int DEPTH, int SPREAD, bool RowB = false>
+__global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_ring_kernel(S8Args p) {
     namespace M2 = mfma2;
-    typedef M2::PolicyI8<C> P;
+    typedef typename S8RingPolicy<C, RowB>::type P;
     constexpr int SCRATCH = DEPTH * C::STAGE / C::WAVES;   // bytes per wave after the loop
     static_assert(SCRATCH >= C::WM * 128 && SCRATCH >= 16 * 512 && SCRATCH % 1024 == 0, "staged stores");
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
     int tm, tn;
     tile_coords(blockIdx.x, (p.M + C::TB - 1) / C::TB, (p.N + C::TBN - 1) / C::TBN, tm, tn);
     const int m_base = tm * C::TB, n_base = tn * C::TBN;
-    M2::DmaRows<false, false> d;
-    d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-    d.b = M2::make_dma_interior<C, C::ROWS_PER_WAVE_B>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb);
     M2::AccTile<P> acc;
-    M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    const auto a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
+    if constexpr (RowB) {
+        const M2::DmaRowsRrr d{a, M2::make_dma_row_b<C>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base)};
+        M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    } else {
+        const M2::DmaRows<false, false> d{
+            a, M2::make_dma_interior<C, C::ROWS_PER_WAVE_B>(p.b, (uint32_t)(p.N * p.ldb), (int)p.ldb, n_base * (int)p.ldb)};
+        M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
+    }
     s8_store_tile<EPI, VecOut, ACT, BiasT, P>(acc, lds + (threadIdx.x >> 6) * SCRATCH, p, m_base, n_base);
 }
 
@@ -741,8 +752,6 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_staged_kernel(S8Args p,
     constexpr int ROWS = 16 * RF + 16 * NB;                   // A then B rows of a stage
     constexpr int STAGE = ROWS * SB;                          // bytes
     constexpr int UPR = SB / 16;                              // 16-byte units per row
-    constexpr int NI = ROWS * UPR / 64;                       // 1 KiB DMA instructions per stage
-    constexpr int HI = (NI + WAVES - 1) / WAVES, LO = NI / WAVES;
     static_assert((!ALL || RF * CH % WAVES == 0) && UPR >= 16 && (ROWS * UPR) % 64 == 0 && DEPTH >= 2 &&
                       DEPTH <= 4 && RF * NB * CH * 1024 <= 160 * 1024 && DEPTH * STAGE <= 160 * 1024,
                   "stage split");
@@ -756,36 +765,14 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_staged_kernel(S8Args p,
     // one XCD's L2) and each line is fetched once (FETCH_SIZE 2.0x -> 1.0x of B)
     const int cgroup = RowB && gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
     const int n0 = cgroup * 16 * NB;
-    const v4i ra = mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda));
-    const v4i rb = mfma2::make_rsrc(p.b, (uint32_t)(RowB ? (int64_t)p.K * p.ldb : (int64_t)p.N * p.ldb));
-    // this wave's DMA instructions j = wave, wave + 16, ...: units 64 j ..
-    // 64 j + 63 of the row-major stage (A rows first), lane L fetching unit
-    // (64 j + L) % UPR of row (64 j + L) / UPR
-    auto dma_stage = [&](int st, int8_t *buf) {
-        const int k0 = st * SB;
-        for (int j = wave; j < NI; j += WAVES) {
-            const int idx = 64 * j + lane;
-            const int r = idx / UPR, slot = idx % UPR;
-            const int unit = slot ^ (r & 15);
-            // units at or past K (a partial last stage) land as zeros
-            const bool past = k0 + 16 * unit >= p.K;
-            if (r < 16 * RF) {
-                mfma2::dma16(ra, past ? mfma2::kPastExtent : (int)((int64_t)(m0 + r) * p.lda) + 16 * unit, k0, buf + j * 1024);
-            } else if constexpr (RowB) {
-                // unit ib of the B region: k-row ib / NB, 16 columns ib % NB
-                const int ib = idx - 16 * RF * UPR;
-                mfma2::dma16(rb, (ib / NB) * (int)p.ldb + n0 + 16 * (ib % NB),
-                             __builtin_amdgcn_readfirstlane(k0 * (int)p.ldb), buf + j * 1024);
-            } else {
-                mfma2::dma16(rb, past ? mfma2::kPastExtent : (int)((int64_t)(n0 + r - 16 * RF) * p.ldb) + 16 * unit, k0,
-                             buf + j * 1024);
-            }
-        }
-    };
-    // waves below NI % 16 issue HI instructions per stage, the others LO
-    const bool hi = NI % WAVES == 0 || wave < NI % WAVES;
+    mfma2::RowsDma<16 * RF, 16 * NB, SB, RowB> dma;
+    dma.init(mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda)),
+             mfma2::make_rsrc(p.b, (uint32_t)(RowB ? (int64_t)p.K * p.ldb : (int64_t)p.N * p.ldb)),
+             [&](int r) { return (int)((int64_t)(m0 + r) * p.lda); }, n0, (int)p.ldb);
+    constexpr int HI = dma.HI, LO = dma.LO;
+    const bool hi = dma.hi();
     const int ns = (p.K + SB - 1) / SB;
-    for (int st = 0; st < DEPTH && st < ns; ++st) dma_stage(st, lds + st * STAGE);
+    for (int st = 0; st < DEPTH && st < ns; ++st) dma.issue(st, p.K, lds + st * STAGE);
     const int c = wave % CH, f0 = wave / CH;
     const bool active = ALL || wave < RF * CH;   // wave-uniform
     v4i acc[FPW][NB];
@@ -835,7 +822,7 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_staged_kernel(S8Args p,
         }
         }
         __syncthreads();   // every wave is done with this buffer
-        if (st + DEPTH < ns) dma_stage(st + DEPTH, buf);
+        if (st + DEPTH < ns) dma.issue(st + DEPTH, p.K, buf);
     }
     // partial sums of (A fragment f, B fragment nb), chunk c: part[f][nb][c][lane]
     v4i *part = reinterpret_cast<v4i *>(lds);
@@ -884,15 +871,7 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_s8_rrr_dma_kernel(S8Args p
     d.b = M2::make_dma_row_b<DmaCfg>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base);
     M2::AccTile<P> acc;
     M2::mainloop<P>(stage0, stage1, d, p.K, acc);
-    const S8Epilogue<EPI_S8, VecOut, ACT, BiasT> epi{p};
-    const bool full = m_base + M2::BM <= p.M && n_base + M2::BN <= p.N;
-    if constexpr (VecOut) {
-        if (p.ldd % 16 == 0 && (reinterpret_cast<uintptr_t>(p.d) & 15u) == 0 && (full || p.N % 16 == 0)) {
-            store_s8_tile_staged<P>(acc, mfma2::wave_scratch<DmaCfg>(stage0, stage1), p, m_base, n_base, epi);
-            return;
-        }
-    }
-    M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4i &v) { epi(m_base + ml, n_base + nl, v); });
+    s8_store_tile<EPI_S8, VecOut, ACT, BiasT, P>(acc, M2::wave_scratch<DmaCfg>(stage0, stage1), p, m_base, n_base);
 }
 
 // ---- u8 x u8 RRR (B row-major [K,N]) ----------------------------------------
@@ -973,10 +952,10 @@ __device__ __forceinline__ void park_row_sums(uint32_t v, int *dst) {
 }
 
 // u8 outputs of a whole tile: staged 16-byte row stores when D allows them.
-template <bool VecOut, class P, class Epi>
+template <bool Staged, class P, class Epi>
 __device__ __forceinline__ void store_u8_tile(const mfma2::AccTile<P> &acc, int8_t *stage0, int8_t *stage1,
                                               const S8Args &p, int m_base, int n_base, const Epi &epi) {
-    if constexpr (VecOut) {
+    if constexpr (Staged) {
         if (p.ldd % 16 == 0 && (reinterpret_cast<uintptr_t>(p.d) & 15u) == 0) {
             const int wave = threadIdx.x >> 6;
             const int wrow = (wave / DmaCfg::WAVES_N) * DmaCfg::WM;
@@ -1008,13 +987,15 @@ __device__ __forceinline__ void store_u8_tile(const mfma2::AccTile<P> &acc, int8
     mfma2::for_each_quad<P>(acc, [&](int ml, int nl, const v4i &v) { epi(ml, nl, v, m_base, n_base); });
 }
 
-template <bool VecOut, int ACT, typename BiasT>
+template <bool VecOut, int ACT, typename BiasT, bool Edge = false>
 __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_u8_rrr_dma_kernel(S8Args p) {
     namespace M2 = mfma2;
     typedef M2::PolicyU8RowB<DmaCfg> P;
     __shared__ __attribute__((aligned(1024))) int8_t stage0[2 * M2::OPER];
     __shared__ __attribute__((aligned(1024))) int8_t stage1[2 * M2::OPER];
-    const int tiles_m = p.M / M2::BM, tiles_n = p.N / M2::BN;
+    // Edge: M, N or K off the tile.  Rows past M are zeros (and the other rows'
+    // sums their own), columns past N are not stored; 4-byte stores.
+    const int tiles_m = (p.M + M2::BM - 1) / M2::BM, tiles_n = (p.N + M2::BN - 1) / M2::BN;
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m_base = tm * M2::BM, n_base = tn * M2::BN;
@@ -1026,7 +1007,7 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_u8_rrr_dma_kernel(S8Args p
     sums.ra = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) sums.cb[q] = 0;
-    M2::mainloop<P>(stage0, stage1, d, p.K, acc, sums);
+    M2::mainloop<P, Edge>(stage0, stage1, d, p.K, acc, sums);
     // Park: row sums directly; column partials per wave in [8][256], then
     // summed; above the staged-store scratch of waves 4..7 (stage1's first 32 KiB).
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1044,8 +1025,8 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_u8_rrr_dma_kernel(S8Args p
         sc[256 + threadIdx.x] = t;
     }
     __syncthreads();
-    const U8Epilogue<VecOut, ACT, BiasT> epi{p, sc, sc + 256, 16384u * (uint32_t)p.K};
-    store_u8_tile<VecOut, P>(acc, stage0, stage1, p, m_base, n_base, epi);
+    const U8Epilogue<VecOut, ACT, BiasT> epi{p, sc, sc + 256, 16384u * (uint32_t)((p.K + M2::BK - 1) / M2::BK * M2::BK)};
+    store_u8_tile<VecOut && !Edge, P>(acc, stage0, stage1, p, m_base, n_base, epi);
 }
 
 // ---- u8 pre-pass (when the caller gives a workspace) ------------------------
@@ -1183,14 +1164,35 @@ __global__ __launch_bounds__(NT, 1) void gemm_u8_rrr_kernel(S8Args p) {
 
 // Whole-tile problems the LDS-DMA u8 RRR kernels take.
 inline bool u8_rrr_dma_eligible(const S8Args &p) {
-    return p.K % mfma2::BK == 0 && p.M % mfma2::BM == 0 && p.N % mfma2::BN == 0 && p.lda % 16 == 0 &&
-           p.ldb % 16 == 0 && aligned16(p.a) && aligned16(p.b) && (int64_t)p.M * p.lda < (1ll << 31) &&
-           (int64_t)p.K * p.ldb < (1ll << 31);
+    return p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) && aligned16(p.b) &&
+           dma_extent_ok(p.M, p.lda) && mfma2::row_b_extent_ok(p.K, p.ldb, mfma2::BK);
 }
 
-// ... of which those whose operands the pre-pass can rewrite into a workspace.
+// Problems of whole tiles whose operands the pre-pass can rewrite into a
+// workspace.
 inline bool u8_rrr_prepass_eligible(const S8Args &p) {
-    return u8_rrr_dma_eligible(p) && (int64_t)p.K * p.N < (1ll << 31);
+    return p.K % mfma2::BK == 0 && p.M % mfma2::BM == 0 && p.N % mfma2::BN == 0 && p.lda % 16 == 0 &&
+           p.ldb % 16 == 0 && aligned16(p.a) && aligned16(p.b) && (int64_t)p.M * p.lda < (1ll << 31) &&
+           (int64_t)p.K * p.ldb < (1ll << 31) && (int64_t)p.K * p.N < (1ll << 31);
+}
+
+// Launches the in-loop u8 RRR tiles.
+template <int ACT, typename BiasT>
+void launch_u8_rrr_dma(const S8Args &p, hipStream_t stream) {
+    const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+    const bool vec = p.N % 4 == 0 && p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % 4) == 0;
+    const bool edge = p.M % mfma2::BM != 0 || p.N % mfma2::BN != 0 || p.K % mfma2::BK != 0;
+    auto go = [&](auto v, auto e) {
+        hipLaunchKernelGGL((gemm_u8_rrr_dma_kernel<decltype(v)::value, ACT, BiasT, decltype(e)::value>), dim3(tiles),
+                           dim3(DmaCfg::NT), 0, stream, p);
+    };
+    if (edge) {
+        if (vec) go(std::true_type{}, std::true_type{});
+        else go(std::false_type{}, std::true_type{});
+    } else {
+        if (vec) go(std::true_type{}, std::false_type{});
+        else go(std::false_type{}, std::false_type{});
+    }
 }
 
 // u8 RRR last rows (decode-sized M; M % 256 in [1, 128] when a row of tiles
@@ -1250,20 +1252,14 @@ bool launch_u8_rrr_rows(const S8Args &p, hipStream_t stream) {
         blocks = (p.M + 127) / 128;
         whole = true;
     }
-    if (rem == 0 || p.K % 512 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.a) || !aligned16(p.b) ||
-        !dma_extent_ok(p.M, p.lda) || (int64_t)p.K * p.ldb + mfma2::BN >= (1ll << 31))
+    if (rem == 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.a) || !aligned16(p.b) ||
+        !dma_extent_ok(p.M, p.lda) || !mfma2::row_b_extent_ok(p.K, p.ldb, 512))
         return false;
     S8Args pm = p;
     pm.M = whole ? 0 : p.M - rem;
     if (pm.M > 0 && !u8_rrr_dma_eligible(pm)) return false;
     const bool vec = p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % 4) == 0;
-    if (pm.M > 0) {
-        const int tiles = (pm.M / mfma2::BM) * (p.N / mfma2::BN);
-        if (vec)
-            hipLaunchKernelGGL((gemm_u8_rrr_dma_kernel<true, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, pm);
-        else
-            hipLaunchKernelGGL((gemm_u8_rrr_dma_kernel<false, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, pm);
-    }
+    if (pm.M > 0) launch_u8_rrr_dma<ACT, BiasT>(pm, stream);
     int rf, nb;   // as the s8 RRR pass
     rows_blocks_plan(p.M, p.N, rem, whole, rf, blocks, nb);
 #define BK_U8RRRROWS(RF, NB, SB, DEPTH)                                                                        \
@@ -1323,14 +1319,7 @@ int32_t launch_u8_rrr(const S8Args &p, hipStream_t stream, void *workspace = nul
         return launch_status();
     }
     if (dma) {
-        const int tiles = (p.M / mfma2::BM) * (p.N / mfma2::BN);
-        const bool vec = p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % 4) == 0;
-        if (vec)
-            hipLaunchKernelGGL((gemm_u8_rrr_dma_kernel<true, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0,
-                               stream, p);
-        else
-            hipLaunchKernelGGL((gemm_u8_rrr_dma_kernel<false, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0,
-                               stream, p);
+        launch_u8_rrr_dma<ACT, BiasT>(p, stream);
         return launch_status();
     }
     const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
@@ -1346,13 +1335,13 @@ int32_t launch_u8_rrr(const S8Args &p, hipStream_t stream, void *workspace = nul
 // ---- u8 x u8 RCR (B [N, K]) ---------------------------------------------------
 // Same correction as the RRR kernels; both operands are K-contiguous rows, so
 // the column sums are B row sums, gathered exactly like the A row sums.
-template <bool VecOut, int ACT, typename BiasT>
+template <bool VecOut, int ACT, typename BiasT, bool Edge = false>
 __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_u8_rcr_dma_kernel(S8Args p) {
     namespace M2 = mfma2;
     typedef M2::PolicyU8<DmaCfg> P;
     __shared__ __attribute__((aligned(1024))) int8_t stage0[2 * M2::OPER];
     __shared__ __attribute__((aligned(1024))) int8_t stage1[2 * M2::OPER];
-    const int tiles_m = p.M / M2::BM, tiles_n = p.N / M2::BN;
+    const int tiles_m = (p.M + M2::BM - 1) / M2::BM, tiles_n = (p.N + M2::BN - 1) / M2::BN;   // edge tiles included
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m_base = tm * M2::BM, n_base = tn * M2::BN;
@@ -1362,15 +1351,15 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_u8_rcr_dma_kernel(S8Args p
     M2::AccTile<P> acc;
     typename P::Sums sums;
     sums.ra = sums.rb = 0;
-    M2::mainloop<P>(stage0, stage1, d, p.K, acc, sums);
+    M2::mainloop<P, Edge>(stage0, stage1, d, p.K, acc, sums);
     // Row sums of A and of B into LDS (free after the loop's last barrier),
     // above the staged-store scratch of waves 4..7 (stage1's first 32 KiB).
     int *sc = reinterpret_cast<int *>(stage1 + 40 * 1024);   // rs[256] | cs[256]
     park_row_sums(sums.ra, sc);
     park_row_sums(sums.rb, sc + 256);
     __syncthreads();
-    const U8Epilogue<VecOut, ACT, BiasT> epi{p, sc, sc + 256, 16384u * (uint32_t)p.K};
-    store_u8_tile<VecOut, P>(acc, stage0, stage1, p, m_base, n_base, epi);
+    const U8Epilogue<VecOut, ACT, BiasT> epi{p, sc, sc + 256, 16384u * (uint32_t)((p.K + M2::BK - 1) / M2::BK * M2::BK)};
+    store_u8_tile<VecOut && !Edge, P>(acc, stage0, stage1, p, m_base, n_base, epi);
 }
 
 // General u8 RCR path: register-staged mainloop, clamped rows, byte-exact K
@@ -1403,6 +1392,25 @@ __global__ __launch_bounds__(NT, 1) void gemm_u8_rcr_kernel(S8Args p) {
     for_each_fragment(acc, [&](int ml, int nl, const v4i &v) { epi(ml, nl, v, m_base, n_base); });
 }
 
+// Launches the in-loop u8 RCR tiles.
+template <int ACT, typename BiasT>
+void launch_u8_rcr_dma(const S8Args &p, hipStream_t stream) {
+    const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+    const bool vec = p.N % 4 == 0 && p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % 4) == 0;
+    const bool edge = p.M % mfma2::BM != 0 || p.N % mfma2::BN != 0 || p.K % mfma2::BK != 0;
+    auto go = [&](auto v, auto e) {
+        hipLaunchKernelGGL((gemm_u8_rcr_dma_kernel<decltype(v)::value, ACT, BiasT, decltype(e)::value>), dim3(tiles),
+                           dim3(DmaCfg::NT), 0, stream, p);
+    };
+    if (edge) {
+        if (vec) go(std::true_type{}, std::true_type{});
+        else go(std::false_type{}, std::true_type{});
+    } else {
+        if (vec) go(std::true_type{}, std::false_type{});
+        else go(std::false_type{}, std::false_type{});
+    }
+}
+
 // u8 RCR last rows (decode-sized M; M % 256 in [1, 128] when a row of tiles
 // would start another round) through the staged last-rows kernel; false
 // when the shape does not fit it.  N = K = 4096: M = 1 / 16 / 128 on the
@@ -1419,21 +1427,14 @@ bool launch_u8_rcr_rows(const S8Args &p, hipStream_t stream) {
         blocks = (p.M + 127) / 128;
         whole = true;
     }
-    if (rem == 0 || p.K % 512 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.a) || !aligned16(p.b) ||
+    if (rem == 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.a) || !aligned16(p.b) ||
         !dma_extent_ok(p.M, p.lda) || !dma_extent_ok(p.N, p.ldb))
         return false;
     S8Args pm = p;
     pm.M = whole ? 0 : p.M - rem;
-    if (pm.M > 0 && p.N % mfma2::BN != 0) return false;
     const bool vec = p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % 4) == 0;
-    if (pm.M > 0) {
-        const int tiles = (pm.M / mfma2::BM) * (p.N / mfma2::BN);
-        if (vec)
-            hipLaunchKernelGGL((gemm_u8_rcr_dma_kernel<true, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, pm);
-        else
-            hipLaunchKernelGGL((gemm_u8_rcr_dma_kernel<false, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, pm);
-    }
-    if (rem == 1 && !whole && p.K % 1024 == 0) {
+    if (pm.M > 0) launch_u8_rcr_dma<ACT, BiasT>(pm, stream);
+    if (rem == 1 && !whole) {
         // one row: the dot4 row kernel (N = K = 4096: 7.6 us on the staged kernel)
         if (p.K % 2048 == 0) {
             if (vec) hipLaunchKernelGGL((gemm_s8_rcr_row1_kernel<0, true, ACT, BiasT, 2, true>), dim3(p.N / 4), dim3(256), 0, stream, p, pm.M);
@@ -1476,18 +1477,9 @@ bool launch_u8_rcr_rows(const S8Args &p, hipStream_t stream) {
 template <int ACT, typename BiasT>
 int32_t launch_u8_rcr(const S8Args &p, hipStream_t stream) {
     if (launch_u8_rcr_rows<ACT, BiasT>(p, stream)) return launch_status();
-    const bool dma = p.K % mfma2::BK == 0 && p.M % mfma2::BM == 0 && p.N % mfma2::BN == 0 &&
-                     p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) && aligned16(p.b) &&
-                     (int64_t)p.M * p.lda < (1ll << 31) && (int64_t)p.N * p.ldb < (1ll << 31);
-    if (dma) {
-        const int tiles = (p.M / mfma2::BM) * (p.N / mfma2::BN);
-        const bool vec = p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % 4) == 0;
-        if (vec)
-            hipLaunchKernelGGL((gemm_u8_rcr_dma_kernel<true, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0,
-                               stream, p);
-        else
-            hipLaunchKernelGGL((gemm_u8_rcr_dma_kernel<false, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0,
-                               stream, p);
+    if (p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) && aligned16(p.b) &&
+        dma_extent_ok(p.M, p.lda) && dma_extent_ok(p.N, p.ldb)) {
+        launch_u8_rcr_dma<ACT, BiasT>(p, stream);
         return launch_status();
     }
     const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
@@ -1500,11 +1492,26 @@ int32_t launch_u8_rcr(const S8Args &p, hipStream_t stream) {
     return launch_status();
 }
 
-template <int EPI, bool VecOut, int ACT, typename BiasT, class C, int DEPTH, int SPREAD>
+template <int EPI, bool VecOut, int ACT, typename BiasT, class C, int DEPTH, int SPREAD, bool RowB = false>
 void launch_ring(const S8Args &p, hipStream_t stream) {
     const int tiles = ((p.M + C::TB - 1) / C::TB) * ((p.N + C::TBN - 1) / C::TBN);
-    hipLaunchKernelGGL((gemm_s8_rcr_ring_kernel<EPI, VecOut, ACT, BiasT, C, DEPTH, SPREAD>), dim3(tiles), dim3(C::NT),
+    hipLaunchKernelGGL((gemm_s8_ring_kernel<EPI, VecOut, ACT, BiasT, C, DEPTH, SPREAD, RowB>), dim3(tiles), dim3(C::NT),
                        (size_t)DEPTH * C::STAGE, stream, p);
+}
+
+// 256 x 256 tiles: the two-stage kernel for whole stages of K, the ring with
+// two stages otherwise (128 x 128 for outputs without 4-column stores).
+template <int EPI, bool VecOut, int ACT, typename BiasT>
+void launch_tiles_256(const S8Args &p, hipStream_t stream) {
+    if (p.K % BK == 0) {
+        const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
+        hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, p,
+                           TailSplit{0, 0, 1}, (int32_t *)nullptr);
+    } else if constexpr (VecOut) {
+        launch_ring<EPI, VecOut, ACT, BiasT, DmaCfg, 2, 0>(p, stream);
+    } else {
+        launch_ring<EPI, VecOut, ACT, BiasT, mfma2::Cfg<4, 2, 128, 128>, 3, 2>(p, stream);
+    }
 }
 
 // All of M as tiles of the cheapest shape (mfma2::ring_tile); outputs
@@ -1522,8 +1529,7 @@ void launch_tiles(const S8Args &p, hipStream_t stream) {
         if (t == mfma2::RT_192x256) return launch_ring<EPI, VecOut, ACT, BiasT, Cfg<2, 4, 192, 256>, 2, 0>(p, stream);
     }
     if (t == mfma2::RT_128x128) return launch_ring<EPI, VecOut, ACT, BiasT, Cfg<4, 2, 128, 128>, 3, 2>(p, stream);
-    hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, p,
-                       TailSplit{0, 0, 1}, (int32_t *)nullptr);
+    launch_tiles_256<EPI, VecOut, ACT, BiasT>(p, stream);
 }
 
 // Every row of the problem as `blocks` row blocks of 16 rf rows on the
@@ -1663,9 +1669,7 @@ void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *works
     if (rem != 0 && (!VecOut || mfma2::last_rows_pay(p.M, p.N, p.K, rem))) {
         S8Args pm = p;
         pm.M = p.M - rem;
-        const int tiles = (pm.M / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
-        hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT),
-                           0, stream, pm, TailSplit{0, 0, 1}, (int32_t *)nullptr);
+        launch_tiles_256<EPI, VecOut, ACT, BiasT>(pm, stream);
         launch_last_rows<EPI, VecOut, ACT, BiasT>(p, pm.M, rem, stream);
         return;
     }
@@ -1695,17 +1699,35 @@ int32_t launch(const S8Args &p, hipStream_t stream, void *workspace = nullptr, s
     return launch_status();
 }
 
-// Launches the RRR DMA kernel when the problem fits it (whole 256x256 tiles,
-// K % 128 == 0, 16-byte A / B rows and bases, buffer offsets below 2^31);
-// returns kOk if launched, kUnsupported to let the caller take the general
-// kernel.
+// Launches RRR tiles when the problem fits the DMA path (K % 16 == 0, 16-byte
+// A / B rows and bases, buffer offsets below 2^31): 128 x 256, 192 x 256 or
+// 256 x 256 by the least modelled time (s8, 1000 x 4096 x 4096: 45.8 us on
+// 256 x 256, 26.9 on 128 x 256); returns kOk if launched, kUnsupported to let
+// the caller take the general kernel.
 template <int ACT, typename BiasT>
 int32_t launch_rrr_dma(const S8Args &p, hipStream_t stream) {
-    const bool fits = p.K % mfma2::BK == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) &&
-                      aligned16(p.b) && dma_extent_ok(p.M, p.lda) && (int64_t)p.K * p.ldb + mfma2::BN < (1ll << 31);
+    const bool fits = p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) &&
+                      aligned16(p.b) && dma_extent_ok(p.M, p.lda) && mfma2::row_b_extent_ok(p.K, p.ldb, mfma2::BK);
     if (!fits) return kUnsupported;
     const int tiles = ((p.M + mfma2::BM - 1) / mfma2::BM) * ((p.N + mfma2::BN - 1) / mfma2::BN);
     const bool vec = p.N % 4 == 0 && p.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(p.d) % 4) == 0;
+    if (vec) {
+        using mfma2::Cfg;
+        const mfma2::RingTile t = mfma2::ring_tile(p.M, p.N, p.K, nullptr, mfma2::RT_128x256);
+        if (t == mfma2::RT_128x256) {
+            launch_ring<EPI_S8, true, ACT, BiasT, Cfg<2, 4, 128, 256>, 3, 4, true>(p, stream);
+            return kOk;
+        }
+        if (t == mfma2::RT_192x256) {
+            launch_ring<EPI_S8, true, ACT, BiasT, Cfg<2, 4, 192, 256>, 2, 0, true>(p, stream);
+            return kOk;
+        }
+        if (p.K % mfma2::BK != 0) {
+            launch_ring<EPI_S8, true, ACT, BiasT, DmaCfg, 2, 0, true>(p, stream);
+            return kOk;
+        }
+    }
+    if (p.K % mfma2::BK != 0) return kUnsupported;
     if (vec)
         hipLaunchKernelGGL((gemm_s8_rrr_dma_kernel<true, ACT, BiasT>), dim3(tiles), dim3(DmaCfg::NT), 0, stream, p);
     else
@@ -1729,8 +1751,8 @@ bool launch_rrr_rows(const S8Args &p, hipStream_t stream) {
         blocks = (p.M + 127) / 128;
         whole = true;
     }
-    if (rem == 0 || p.K % 512 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.a) || !aligned16(p.b) ||
-        !dma_extent_ok(p.M, p.lda) || (int64_t)p.K * p.ldb + mfma2::BN >= (1ll << 31))
+    if (rem == 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.a) || !aligned16(p.b) ||
+        !dma_extent_ok(p.M, p.lda) || !mfma2::row_b_extent_ok(p.K, p.ldb, 512))
         return false;
     // column groups by the last-rows rule (16 / 32 / 64 columns, at least 192
     // workgroups), numbered XCD-major in the kernel so the groups sharing a
@@ -1740,6 +1762,9 @@ bool launch_rrr_rows(const S8Args &p, hipStream_t stream) {
     // tiles 40.5 / 37.7)
     int rf, nb;
     rows_blocks_plan(p.M, p.N, rem, whole, rf, blocks, nb);
+    // more than a round of workgroups: tiles (512 x 14336 x 4096: 128 x 256
+    // tiles 28 us, four rounds of row blocks 69)
+    if (whole && blocks * (p.N / (16 * nb)) > 256) return false;
     S8Args pm = p;
     pm.M = whole ? 0 : p.M - rem;
     if (pm.M > 0 && launch_rrr_dma<ACT, BiasT>(pm, stream) != kOk) return false;

@@ -119,3 +119,13 @@ def test_fp8_tiles_and_depth_tails(gpu, shape):
 @pytest.mark.parametrize("fmt,layout", [("e4m3", P.LayoutSku.Rrr), ("e5m2", P.LayoutSku.Rcr)])
 def test_fp8_out_depth_tails(gpu, shape, fmt, layout):
     S.test_fp8_out_with_c_sweep(gpu, shape, fmt, layout)
+
+
+@pytest.mark.parametrize("shape", [(300, 520, 208), (700, 1000, 336), (900, 2064, 400), (2300, 5008, 400), (257, 262, 48),
+                                   (13, 6160, 304), (1, 272, 48), (100, 272, 656), (200, 1024, 1072), (428, 1440, 2752)])
+def test_rrr_and_u8_depth_tails(gpu, shape):
+    """s8 RRR tiles (128x256 to 256x256) and last rows, u8 RCR / RRR on edge
+    tiles and partial last stages."""
+    S.test_int8_rrr_bias_relu_sweep(gpu, shape)
+    S.test_u8_rcr_sweep(gpu, shape)
+    S.test_u8_rrr_sweep(gpu, shape, False)
