@@ -521,11 +521,11 @@ void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
         BK_F8RB(2, 1, 1024, 3) BK_F8RB(2, 2, 1024, 2)
 #undef BK_F8RB
     }
-    const int nb = mfma2::last_rows_col_frags(p.N);
+    const int nb = rem <= 32 ? mfma2::last_rows_width(p.N) : mfma2::last_rows_col_frags(p.N);
 #define BK_F8ROWS(RF, NB, SB, DEPTH)                                                                     \
     if (rem <= 16 * (RF) && nb == (NB)) {                                              \
         hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH>),           \
-                           dim3(p.N / (16 * (NB))), dim3(1024), (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), \
+                           dim3((p.N + 16 * (NB) - 1) / (16 * (NB))), dim3(1024), (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), \
                            stream, p, m0);                                                               \
         return;                                                                                     \
     }
@@ -533,10 +533,16 @@ void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
     // with MFMA work (padding A rows cost DMA and LDS time: N = 14336, M = 2
     // / 8 / 16 / 32 14.7 / 14.0 / 13.3 / 13.6 -> 13.4 / 12.8 / 12.3 / 12.9 us
     // against 4 fragments; N = 8192, M = 2-16 8.9 -> 8.35 us)
-    BK_F8ROWS(1, 4, 512, 2)
-    BK_F8ROWS(2, 4, 512, 2)
     BK_F8ROWS(1, 2, 512, 2)
+    BK_F8ROWS(1, 3, 512, 2)
+    BK_F8ROWS(1, 4, 512, 2)
+    BK_F8ROWS(1, 6, 512, 2)
+    BK_F8ROWS(1, 7, 512, 2)
     BK_F8ROWS(2, 2, 512, 2)
+    BK_F8ROWS(2, 3, 512, 2)
+    BK_F8ROWS(2, 4, 512, 2)
+    BK_F8ROWS(2, 6, 512, 2)
+    BK_F8ROWS(2, 7, 512, 2)
     BK_F8ROWS(4, 4, 512, 2)
     BK_F8ROWS(8, 4, 256, 2)
     BK_F8ROWS(4, 2, 512, 2)

@@ -531,6 +531,28 @@ inline int last_rows_col_frags(int N, int blocks = 1) {
     return 1;
 }
 
+// Column fragments per workgroup of an RCR last-rows pass of at most 32 rows,
+// any number of them (the columns past N of the last group are neither read
+// nor stored): the width with the fewest columns per CU, counting whole
+// rounds of 256 workgroups, the wider of two alike.  With one round the pass
+// streams its weights at about 4.6 TB/s; 344 workgroups in a round and a third
+// take two.  int8, 20 rows, K = 4096, rotated weights (us by 1 / 2 / 3 / 4 / 6 /
+// 7 fragments): N = 5120 8.8 / 7.8 / 9.1, N = 11008 13.9 / 13.1 / 11.7 / 12.3,
+// N = 14336 17.5 / 14.3 / 17.0 / 14.1, N = 22016 24.6 / 21.0 / 19.1 / 24.4 /
+// 19.6, N = 28672 30.1 / 27.3 / 27.0 / 28.2 / 32.8 / 25.7.
+inline int last_rows_width(int N) {
+    int best = 1, cols = 0;
+    for (const int nb : {1, 2, 3, 4, 6, 7}) {
+        const int groups = (N + 16 * nb - 1) / (16 * nb);
+        const int c = (groups + 255) / 256 * nb;
+        if (nb == 1 || c <= cols) {
+            best = nb;
+            cols = c;
+        }
+    }
+    return best;
+}
+
 // Row blocks of a last-rows pass of 33-128 rows when the rule above gives
 // 16-column workgroups (N below 6144), which would each stage all the rows:
 // blocks of 32 rows, or of 64 rows for more than 64 rows when N > 2048, the

@@ -1575,7 +1575,7 @@ bool launch_row_blocks(const S8Args &p, hipStream_t stream) {
 // The last `rem` (<= kRowsPathMax) rows, from row m0 (N % 16 == 0).
 template <int EPI, bool VecOut, int ACT, typename BiasT>
 void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
-    const int nb = mfma2::last_rows_col_frags(p.N);
+    const int nb = rem <= 32 ? mfma2::last_rows_width(p.N) : mfma2::last_rows_col_frags(p.N);
     if (nb == 1 && rem > 32) {
         // 33-128 rows where 16-column workgroups would each read all
         // of them: 2-4 row blocks (last_rows_blocks).  K = 4096,
@@ -1609,7 +1609,7 @@ void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
     // 4096 6.55 / 6.93 -> 6.37 / 6.42 us, N = 2048 4.95 / 5.27 -> 4.87 / 4.90;
     // it stays ahead up to 8 rows), 8 at 32 columns, 5 at 64 (N = 14336 /
     // 12288, M = 8 14.2 / 11.6 -> 13.2 / 10.8 us staged, level at 2-5 rows).
-    if (rem <= (nb == 1 ? 10 : nb == 2 ? 8 : 5) && p.K % 1024 == 0 && p.K <= kRowsDmaMaxK) {
+    if (rem <= (nb == 1 ? 10 : nb == 2 ? 8 : nb == 4 ? 5 : 1) && p.K % 1024 == 0 && p.K <= kRowsDmaMaxK) {
         // B rows; the 16 waves' partial sums reuse the same LDS
         const size_t lds = std::max((size_t)16 * p.K, (size_t)kRowsDmaWaves * 1024);
         hipLaunchKernelGGL((gemm_s8_rcr_rows_dma_kernel<EPI, VecOut, ACT, BiasT, 1>), dim3(p.N / 16),
@@ -1619,7 +1619,7 @@ void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
 #define BK_S8ROWS(RF, NB, SB, DEPTH)                                                                        \
     if (rem <= 16 * (RF) && nb == (NB)) {                                                                    \
         hipLaunchKernelGGL((gemm_s8_rcr_rows_staged_kernel<EPI, VecOut, ACT, BiasT, RF, NB, SB, DEPTH>),     \
-                           dim3(p.N / (16 * (NB))), dim3(1024),                                             \
+                           dim3((p.N + 16 * (NB) - 1) / (16 * (NB))), dim3(1024),                           \
                            std::max((size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), (size_t)(RF) * (NB) * ((SB) / 64) * 1024), \
                            stream, p, m0);                                                                  \
         return;                                                                                             \
@@ -1627,13 +1627,19 @@ void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
     // up to 16 rows: one fragment, 8 of the 16 waves multiplying (N = 14336 /
     // 8192, M = 12-16: 13.85 / 8.6-8.7 -> 13.3 / 8.5 us against two)
     BK_S8ROWS(1, 1, 512, 3)
-    BK_S8ROWS(2, 1, 512, 3)
     BK_S8ROWS(1, 2, 512, 2)
+    BK_S8ROWS(1, 3, 512, 2)
     BK_S8ROWS(1, 4, 512, 2)
+    BK_S8ROWS(1, 6, 512, 2)
+    BK_S8ROWS(1, 7, 512, 2)
+    BK_S8ROWS(2, 1, 512, 3)
     BK_S8ROWS(2, 2, 512, 3)
+    BK_S8ROWS(2, 3, 512, 2)
+    BK_S8ROWS(2, 4, 512, 2)
+    BK_S8ROWS(2, 6, 512, 2)
+    BK_S8ROWS(2, 7, 512, 2)
     BK_S8ROWS(4, 2, 512, 2)
     BK_S8ROWS(8, 2, 512, 2)
-    BK_S8ROWS(2, 4, 512, 3)
     BK_S8ROWS(4, 4, 512, 2)
     BK_S8ROWS(8, 4, 256, 2)
 #undef BK_S8ROWS

@@ -23,7 +23,9 @@ TILE_SHAPES = [(300, 1700, 208), (450, 2896, 1040), (1000, 2500, 1136), (1500, 5
 # width, row blocks, whole tiles with last rows
 ROW_SHAPES = [(1, 4096, 4080), (1, 272, 48), (5, 512, 1040), (9, 12288, 304), (13, 6160, 1552), (24, 4096, 2752),
               (60, 12288, 304), (100, 272, 656), (120, 6144, 176), (200, 1024, 1072), (400, 1024, 208),
-              (4160, 4096, 144)]
+              (4160, 4096, 144),
+              # 48-, 96- and 112-column workgroups, the last one partly past N
+              (20, 11008, 304), (12, 22016, 144), (30, 28656, 144)]
 
 
 def _acc(a, b):
