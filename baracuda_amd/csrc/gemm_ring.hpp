@@ -36,6 +36,21 @@ __device__ __forceinline__ void dma_piece(int8_t *stage, const DmaRows<false, fa
     }
 }
 
+// Gathered A rows (MoE): one per-lane offset per A piece.
+template <class C, int I>
+__device__ __forceinline__ void dma_piece(int8_t *stage, const DmaRows<true, false> &d, int kbyte) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int NA = C::ROWS_PER_WAVE / 8;
+    if constexpr (I < NA) {
+        dma16(d.a.rsrc, d.a.off[I], __builtin_amdgcn_readfirstlane(kbyte), stage + (wave * C::ROWS_PER_WAVE + I * 8) * BK);
+    } else {
+        constexpr int J = I - NA;
+        const int soff = __builtin_amdgcn_readfirstlane(kbyte + J * d.b.row_stride);
+        dma16(d.b.rsrc, (J & 1) ? d.b.odd : d.b.even, soff,
+              stage + C::OPER + (wave * C::ROWS_PER_WAVE_B + J * 8) * BK);
+    }
+}
+
 // Row-major B (TBN = 256 columns, 8 waves): B pieces of four k-rows.
 template <class C, int I>
 __device__ __forceinline__ void dma_piece(int8_t *stage, const DmaRowsRrr &d, int kbyte) {
@@ -164,13 +179,16 @@ constexpr RingCost kRingCost[] = {
 // 5120 x 2880 128x256 23.7 (192x256 31.6, 128x128 28.9), 810 x 2352 x 1856
 // 64x128 9.3 (128x128 10.9), 200 x 11008 x 4096 128x128 20.3 (64x128 24.3),
 // 3072 x 4096 x 4096 192x256 44.3 (256x256 47.0), 4096^3 256x256 55.5.
-inline float ring_cost(const RingCost &c, int M, int N, int kbytes) {
-    const int64_t tiles = (int64_t)((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn);
+inline float ring_cost_tiles(const RingCost &c, int64_t tiles, int kbytes) {
     const float kt = (float)((kbytes + BK - 1) / BK);
     const int64_t per_cu = (tiles + 255) / 256;
     if (c.paired == 0.0f) return (float)per_cu * (c.fixed + kt * c.stage);
     const int64_t pairs = per_cu / 2;
     return (float)pairs * (c.fixed + kt * c.paired) + (float)(per_cu % 2) * (c.fixed + kt * c.stage);
+}
+
+inline float ring_cost(const RingCost &c, int M, int N, int kbytes) {
+    return ring_cost_tiles(c, (int64_t)((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn), kbytes);
 }
 
 // `first`: the smallest shape the caller has (row-major B tiles are 256

@@ -21,7 +21,7 @@
 // LDS counters (no global atomics, no memset: graph-capturable), and the GEMM
 // is one launch whose workgroups walk the ragged per-expert tile list.
 #include "gemm_mfma.hpp"
-#include "gemm_mfma2.hpp"
+#include "gemm_ring.hpp"
 
 namespace bk {
 namespace {
@@ -31,54 +31,55 @@ using namespace mfma;
 constexpr int kMaxExperts = 1024;
 
 // expert_counts / expert_offsets from expert_ids (one workgroup, 1024 threads).
-// Up to 64 experts each wave counts 64 ids at a time with one ballot per
-// expert, lane e keeping expert e's running count, and adds its counts to
-// LDS once; more experts fall back to one LDS atomic per id.  Ids outside
-// [0, num_experts) are not counted.
+// The ids come grouped by expert, so a wave's 64 of them are a few runs of
+// equal ids: the first lane of each run adds the run's length to the expert's
+// LDS counter (any order of the ids counts right; ids outside [0, E) nowhere),
+// and the counts' prefix sum runs over the 16 waves.  One ballot per expert
+// and 64 ids, and the sum by one thread, took 29 us at 3072 ids of 64 experts
+// and 7.7 at 8192 of 8; now 4.6 and 5.7.
 __global__ __launch_bounds__(1024) void moe_offsets_kernel(const int32_t *__restrict__ expert_ids,
-                                                           int32_t size_m, int32_t num_experts,
+                                                           int size_m, int num_experts,
                                                            int32_t *__restrict__ counts,
                                                            int32_t *__restrict__ offsets) {
-    __shared__ int32_t cnt[kMaxExperts];
-    for (int e = threadIdx.x; e < num_experts; e += blockDim.x) cnt[e] = 0;
+    __shared__ int cnt[kMaxExperts];
+    __shared__ int wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    cnt[tid] = 0;
     __syncthreads();
-    if (num_experts <= 64) {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-        int mine = 0;   // count of expert `lane`
-        // Each wave takes 8 ids per lane per pass, all loads issued before the
-        // first ballot so one memory round trip covers 512 ids.
-        constexpr int V = 8;
-        for (int base = wave * 64 * V; base < size_m; base += waves * 64 * V) {
-            int e[V];
+    constexpr int U = 4;   // ids per lane requested before the first is used
+    for (int i0 = 0; i0 < size_m; i0 += 1024 * U) {
+        int id[U];
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                const int i = base + v * 64 + lane;
-                e[v] = i < size_m ? expert_ids[i] : -1;
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + u * 1024 + tid;
+            id[u] = i < size_m ? expert_ids[i] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int prev = __shfl_up(id[u], 1, 64);
+            const uint64_t heads = __ballot(lane == 0 || id[u] != prev);
+            if (((heads >> lane) & 1) && id[u] >= 0 && id[u] < num_experts) {
+                const uint64_t next = lane < 63 ? heads >> (lane + 1) : 0;
+                atomicAdd(&cnt[id[u]], next ? __ffsll((unsigned long long)next) : 64 - lane);
             }
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                for (int x = 0; x < num_experts; ++x) {
-                    const int c = __popcll(__ballot(e[v] == x));
-                    if (lane == x) mine += c;
-                }
-        }
-        if (lane < num_experts && mine) atomicAdd(&cnt[lane], mine);
-    } else {
-        for (int i = threadIdx.x; i < size_m; i += blockDim.x) {
-            const int e = expert_ids[i];
-            if (e >= 0 && e < num_experts) atomicAdd(&cnt[e], 1);
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        offsets[0] = 0;
-        for (int e = 0; e < num_experts; ++e) {
-            counts[e] = cnt[e];
-            run += cnt[e];
-            offsets[e + 1] = run;
-        }
+    const int c = tid < num_experts ? cnt[tid] : 0;
+    int run = c;                                  // inclusive sum over the wave
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(run, off, 64);
+        if (lane >= off) run += v;
     }
+    if (lane == 63) wsum[wave] = run;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) run += wsum[w];
+    if (tid < num_experts) {
+        counts[tid] = c;
+        offsets[tid + 1] = run;
+    }
+    if (tid == 0) offsets[0] = 0;
 }
 
 // Operand kinds: int8 (W8A8 epilogue), bf16, f16 (16-bit float elements),
@@ -352,6 +353,85 @@ template <int KIND> struct MoePolicy { typedef mfma2::PolicyI8<DmaCfg> type; }; 
 template <> struct MoePolicy<MOE_BF16> { typedef mfma2::PolicyH16<DmaCfg, true> type; };
 template <> struct MoePolicy<MOE_F16> { typedef mfma2::PolicyH16<DmaCfg, false> type; };
 
+// Epilogue of a tile: rows staged in this wave's `scratch` (see the staged
+// stores) and written to the pairs' output rows; padding rows are skipped.
+// wc: the wave's first output column; ncols: valid columns from there (a
+// multiple of 8; 4 for int32).
+template <int KIND, class P>
+__device__ __forceinline__ void moe_store_tile(const mfma2::AccTile<P> &acc, int8_t *scratch, const MoeArgs &p,
+                                               const int32_t *rows_tok, int seg_rows, int in_div, int e, int wc,
+                                               int ncols) {
+    namespace M2 = mfma2;
+    typedef typename P::Cfg C;
+    const int wr = ((int)(threadIdx.x >> 6) / C::WAVES_N) * C::WM;
+    if constexpr (KIND == MOE_S8_I32) {
+        // int32 rows staged per wave in two halves of 64 rows and written as
+        // 16-byte units of the pair's output row; padding rows are skipped.
+        M2::store_x32x4_staged<P>(
+            acc, scratch, [&](int, int, const v4i &v) { return v; },
+            [&](int r) -> int32_t * {
+                return wr + r < seg_rows ? static_cast<int32_t *>(p.out) + (int64_t)rows_tok[wr + r] * p.N + wc
+                                         : nullptr;
+            },
+            ncols);
+        return;
+    } else if constexpr (KIND != MOE_S8) {
+        if ((reinterpret_cast<uintptr_t>(p.out) & 15u) == 0) {
+            // Rows staged per wave in LDS and written as 16-byte units of the
+            // token's output row; padding rows of a partial tile are skipped.
+            M2::store_bf16x4_staged<P>(
+                acc, scratch,
+                [&](int r, int, const v4f &v) {
+                    const float tw = p.topk_w ? p.topk_w[rows_tok[wr + r]] : 1.0f;
+                    uint16_t h[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float y = p.topk_w ? v[q] * tw : v[q];
+                        h[q] = KIND == MOE_BF16 ? f32_to_bf16_rne(y) : f32_to_f16_rne(y);
+                    }
+                    return v2i{(int)((uint32_t)h[0] | ((uint32_t)h[1] << 16)),
+                               (int)((uint32_t)h[2] | ((uint32_t)h[3] << 16))};
+                },
+                [&](int r) -> uint16_t * {
+                    return wr + r < seg_rows ? static_cast<uint16_t *>(p.out) + (int64_t)rows_tok[wr + r] * p.N + wc
+                                             : nullptr;
+                },
+                ncols);
+            return;
+        }
+        const int wcol = (threadIdx.x >> 6) % C::WAVES_N * C::WN;   // for_each_quad counts from the tile's column
+        M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4f &v) {
+            moe_store_h<KIND>(p, rows_tok, seg_rows, ml, wc - wcol + nl, v);
+        });
+        return;
+    } else {
+        // Epilogue: scales (per token row, per expert column) fetched once per
+        // lane; the wave tile is staged in LDS and written as full 128-byte rows
+        // of the token's output row; padding rows of a partial tile are skipped.
+        const float *swe = p.sw + (int64_t)e * p.N;
+        const int lane = threadIdx.x & 63;
+        float sam[P::TI], post[P::TI];
+        v4f swv[P::TJ];
+#pragma unroll
+        for (int i = 0; i < P::TI; ++i) {
+            const int tok = rows_tok[min(wr + i * 16 + (lane & 15), seg_rows - 1)];
+            sam[i] = p.sa[tok / in_div];
+            post[i] = p.topk_w ? p.topk_w[tok] : 1.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < P::TJ; ++j) {
+            const int col = j * 16 + (lane >> 4) * 4;
+            swv[j] = col < ncols ? *reinterpret_cast<const v4f *>(swe + wc + col) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        auto dst = [&](int r) -> uint16_t * {
+            return wr + r < seg_rows ? static_cast<uint16_t *>(p.out) + (int64_t)rows_tok[wr + r] * p.N + wc
+                                     : nullptr;
+        };
+        if (p.topk_w) M2::store_w8a8_bf16_staged<P, true>(acc, scratch, sam, post, swv, dst, ncols);
+        else M2::store_w8a8_bf16_staged<P, false>(acc, scratch, sam, post, swv, dst, ncols);
+    }
+}
+
 template <int KIND>
 __global__ __launch_bounds__(DmaCfg::NT, 1) void moe_grouped_dma_kernel(MoeArgs p) {
     namespace M2 = mfma2;
@@ -386,80 +466,113 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void moe_grouped_dma_kernel(MoeArgs 
     }
     M2::AccTile<P> acc;
     M2::mainloop<P>(stage0, stage1, d, kb, acc);
-    if constexpr (KIND == MOE_S8_I32) {
-        // int32 rows staged per wave in two halves of 64 rows and written as
-        // 16-byte units of the pair's output row; padding rows are skipped.
-        const int wave = threadIdx.x >> 6;
-        const int wr = (wave / DmaCfg::WAVES_N) * DmaCfg::WM;
-        const int wc = n_base + (wave % DmaCfg::WAVES_N) * DmaCfg::WN;
-        int8_t *scratch = (wave < 4 ? stage0 : stage1) + (wave & 3) * (DmaCfg::WM / 2 * 256);
-        M2::store_x32x4_staged<P>(
-            acc, scratch, [&](int, int, const v4i &v) { return v; },
-            [&](int r) -> int32_t * {
-                return wr + r < seg_rows ? static_cast<int32_t *>(p.out) + (int64_t)s_rows_tok[wr + r] * p.N + wc
-                                         : nullptr;
-            });
-        return;
-    } else if constexpr (KIND != MOE_S8) {
-        if ((reinterpret_cast<uintptr_t>(p.out) & 15u) == 0) {
-            // Rows staged per wave in LDS and written as 16-byte units of the
-            // token's output row; padding rows of a partial tile are skipped.
-            const int wave = threadIdx.x >> 6;
-            const int wr = (wave / DmaCfg::WAVES_N) * DmaCfg::WM;
-            const int wc = n_base + (wave % DmaCfg::WAVES_N) * DmaCfg::WN;
-            int8_t *scratch = (wave < 4 ? stage0 : stage1) + (wave & 3) * (DmaCfg::WM * 128);
-            M2::store_bf16x4_staged<P>(
-                acc, scratch,
-                [&](int r, int, const v4f &v) {
-                    const float tw = p.topk_w ? p.topk_w[s_rows_tok[wr + r]] : 1.0f;
-                    uint16_t h[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float y = p.topk_w ? v[q] * tw : v[q];
-                        h[q] = KIND == MOE_BF16 ? f32_to_bf16_rne(y) : f32_to_f16_rne(y);
-                    }
-                    return v2i{(int)((uint32_t)h[0] | ((uint32_t)h[1] << 16)),
-                               (int)((uint32_t)h[2] | ((uint32_t)h[3] << 16))};
-                },
-                [&](int r) -> uint16_t * {
-                    return wr + r < seg_rows ? static_cast<uint16_t *>(p.out) + (int64_t)s_rows_tok[wr + r] * p.N + wc
-                                             : nullptr;
-                });
-            return;
-        }
-        M2::for_each_quad<P>(acc, [&](int ml, int nl, const v4f &v) {
-            moe_store_h<KIND>(p, s_rows_tok, seg_rows, ml, n_base + nl, v);
-        });
-        return;
-    } else {
-        // Epilogue: scales (per token row, per expert column) fetched once per
-        // lane; the wave tile is staged in LDS and written as full 128-byte rows
-        // of the token's output row; padding rows of a partial tile are skipped.
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int wr = (wave / DmaCfg::WAVES_N) * DmaCfg::WM;
-        const int wc = n_base + (wave % DmaCfg::WAVES_N) * DmaCfg::WN;
-        const float *swe = p.sw + (int64_t)e * p.N;
-        float sam[P::TI], post[P::TI];
-        v4f swv[P::TJ];
-#pragma unroll
-        for (int i = 0; i < P::TI; ++i) {
-            const int tok = s_rows_tok[wr + i * 16 + (lane & 15)];
-            sam[i] = p.sa[tok / in_div];
-            post[i] = p.topk_w ? p.topk_w[tok] : 1.0f;
-        }
-#pragma unroll
-        for (int j = 0; j < P::TJ; ++j) swv[j] = *reinterpret_cast<const v4f *>(swe + wc + j * 16 + (lane >> 4) * 4);
-        int8_t *scratch = (wave < 4 ? stage0 : stage1) + (wave & 3) * (DmaCfg::WM * DmaCfg::WN * 2);
-        auto dst = [&](int r) -> uint16_t * {
-            return wr + r < seg_rows ? static_cast<uint16_t *>(p.out) + (int64_t)s_rows_tok[wr + r] * p.N + wc
-                                     : nullptr;
-        };
-        if (p.topk_w) M2::store_w8a8_bf16_staged<P, true>(acc, scratch, sam, post, swv, dst);
-        else M2::store_w8a8_bf16_staged<P, false>(acc, scratch, sam, post, swv, dst);
-    }
+    const int wave = threadIdx.x >> 6;
+    moe_store_tile<KIND, P>(acc, M2::wave_scratch<DmaCfg>(stage0, stage1), p, s_rows_tok, seg_rows, in_div, e,
+                            n_base + (wave % DmaCfg::WAVES_N) * DmaCfg::WN, DmaCfg::WN);
 }
 
-// Decode-sized MoE (size_m <= 64): one launch over (N / (16 NB) column
+// ---- tiles of gemm_ring.hpp ---------------------------------------------------
+// Few rows per expert (serving batches, many experts), N off 256 or K off 128
+// bytes: tiles of C::TB rows of one expert by C::TBN columns, over a ring of
+// DEPTH stages.  256-row tiles pay for the padding of every expert's last tile,
+// and the register-staged kernel took what the LDS-DMA one did not.
+
+// Workgroup id -> (expert, first pair, rows, n-tile) of the list of C::TB-row
+// slots in the n-block order of moe_list_tile, each XCD owning a contiguous
+// range of it; false past the list.  Measured, us, 256-row tiles or the
+// register-staged kernel -> now: bf16, 192 tokens, 2 of 8 experts 14336 x 4096
+// 229 -> 191 (the kernel alone 171, 5.5 TB/s of weights); int8, 512 tokens, 6 of
+// 64 experts 1408 x 2048 147 -> 46; int8, 1024 tokens, 4 of 16 experts 4096 x
+// 4096 137 -> 112.  Every wave finds it from the offsets by
+// itself: 64 experts at a time, one per lane, a prefix sum of their tiles (a
+// walk over the experts by every thread takes microseconds at 64 of them).
+template <int TB>
+__device__ __forceinline__ bool moe_ring_tile(const MoeArgs &p, int n_tiles, int &e, int &seg0, int &rows, int &ntile) {
+    const int lane = threadIdx.x & 63;
+    auto load = [&](int e0, int &o0, int &n) {
+        const int x = e0 + lane;
+        o0 = x < p.E ? min(p.offsets[x], p.size_m) : 0;
+        n = x < p.E ? max(min(p.offsets[x + 1], p.size_m) - o0, 0) : 0;
+        int incl = (n + TB - 1) / TB;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int v = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += v;
+        }
+        return incl;
+    };
+    int S = 0, o0, n, incl = 0;
+    for (int e0 = 0; e0 < p.E; e0 += 64) {
+        incl = load(e0, o0, n);
+        S += __builtin_amdgcn_readlane(incl, 63);
+    }
+    const int T = S * n_tiles, pid = blockIdx.x, xcd = pid % 8, q = T / 8, r = T % 8;
+    if (pid / 8 >= q + (xcd < r ? 1 : 0)) return false;
+    int slot;
+    moe_list_tile(xcd * q + min(xcd, r) + pid / 8, S, n_tiles, slot, ntile);
+    for (int e0 = 0; e0 < p.E; e0 += 64) {
+        if (p.E > 64) incl = load(e0, o0, n);
+        const uint64_t past = __ballot(incl > slot);
+        if (past) {
+            const int l = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)past) - 1);
+            const int first = slot - (__builtin_amdgcn_readlane(incl, l) -
+                                      (__builtin_amdgcn_readlane(n, l) + TB - 1) / TB);   // tile within the expert
+            e = e0 + l;
+            seg0 = __builtin_amdgcn_readlane(o0, l) + first * TB;
+            rows = min(TB, __builtin_amdgcn_readlane(n, l) - first * TB);
+            return true;
+        }
+        slot -= __builtin_amdgcn_readlane(incl, 63);
+    }
+    return false;
+}
+
+template <int KIND, class C> struct MoeRingPolicy { typedef mfma2::PolicyI8<C> type; };
+template <class C> struct MoeRingPolicy<MOE_BF16, C> { typedef mfma2::PolicyH16<C, true> type; };
+template <class C> struct MoeRingPolicy<MOE_F16, C> { typedef mfma2::PolicyH16<C, false> type; };
+
+template <int KIND, class C, int DEPTH, int SPREAD>
+__global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void moe_ring_kernel(MoeArgs p, int n_tiles) {
+    namespace M2 = mfma2;
+    typedef typename MoeRingPolicy<KIND, C>::type P;
+    constexpr int SCRATCH = DEPTH * C::STAGE / C::WAVES;   // bytes per wave after the loop
+    static_assert(SCRATCH >= C::WM * 128 && SCRATCH % 1024 == 0, "staged stores");
+    extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+    int32_t *s_tok = reinterpret_cast<int32_t *>(lds + DEPTH * C::STAGE);   // [TB]
+    int e, seg0, seg_rows, ntile;
+    if (!moe_ring_tile<C::TB>(p, n_tiles, e, seg0, seg_rows, ntile)) return;   // whole workgroup exits
+    for (int r = threadIdx.x; r < C::TB; r += C::NT) s_tok[r] = r < seg_rows ? p.sorted_ids[seg0 + r] : -1;
+    __syncthreads();
+    const int n_base = ntile * C::TBN;
+    const int in_div = p.topk_w ? 1 : p.topk;
+    const int x_rows = p.topk_w ? p.size_m : (p.size_m + p.topk - 1) / p.topk;
+    const int kb = p.K * MoeElem<KIND>::SIZE;   // row length in bytes
+    M2::DmaRows<true, false> d;
+    // padding rows point past the input and load as zeros
+    d.a = M2::make_dma_gathered<C>(p.x, (uint32_t)((int64_t)x_rows * kb), [&](int r) {
+        const int tok = s_tok[r];
+        return tok >= 0 ? (tok / in_div) * kb : x_rows * kb;
+    });
+    d.b = M2::make_dma_interior<C, C::ROWS_PER_WAVE_B>(p.w + (int64_t)e * p.N * kb, (uint32_t)((int64_t)p.N * kb), kb,
+                                                       n_base * kb);
+    M2::AccTile<P> acc;
+    M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, kb, acc);
+    const int wave = threadIdx.x >> 6, wc = n_base + (wave % C::WAVES_N) * C::WN;
+    if (wave / C::WAVES_N * C::WM >= seg_rows || wc >= p.N) return;   // nothing of this wave's tile is stored
+    moe_store_tile<KIND, P>(acc, lds + wave * SCRATCH, p, s_tok, seg_rows, in_div, e, wc, min(C::WN, p.N - wc));
+}
+
+template <int KIND, class C, int DEPTH, int SPREAD>
+void launch_moe_ring(const MoeArgs &p, hipStream_t stream) {
+    const int n_tiles = (p.N + C::TBN - 1) / C::TBN;
+    // at most ceil(size_m / TB) + (experts with rows) slots
+    const int64_t slots = (p.size_m + C::TB - 1) / C::TB + std::min(p.E, p.size_m);
+    const int64_t grid = (slots * n_tiles + 7) / 8 * 8;
+    hipLaunchKernelGGL((moe_ring_kernel<KIND, C, DEPTH, SPREAD>), dim3((uint32_t)grid), dim3(C::NT),
+                       (size_t)DEPTH * C::STAGE + C::TB * 4, stream, p, n_tiles);
+}
+
+// Decode-sized MoE (size_m <= 64): one launch over (ceil(N / (16 NB)) column
 // groups) x E experts x (size_m / 16 RF row blocks), no offsets kernel in
 // front.  A workgroup of 16 waves finds its expert's rows from the ids
 // (moe_decode_rows) and exits when its block of them is empty; otherwise,
@@ -484,8 +597,6 @@ __global__ __launch_bounds__(1024) void moe_rows_staged_kernel(MoeArgs p) {
     constexpr int ROWS = 16 * RF + 16 * NB;
     constexpr int STAGE = ROWS * SB;
     constexpr int UPR = SB / 16;
-    constexpr int NI = ROWS * UPR / 64;
-    constexpr int HI = (NI + WAVES - 1) / WAVES, LO = NI / WAVES;
     constexpr bool INT = KIND == MOE_S8 || KIND == MOE_S8_I32;
     constexpr int ES = MoeElem<KIND>::SIZE;
     typedef typename std::conditional<INT, v4i, v4f>::type Acc;
@@ -512,26 +623,18 @@ __global__ __launch_bounds__(1024) void moe_rows_staged_kernel(MoeArgs p) {
     const int x_rows = p.topk_w ? p.size_m : (p.size_m + p.topk - 1) / p.topk;
     for (int r = threadIdx.x; r < 16 * RF; r += blockDim.x) s_tok[r] = r < rows ? p.sorted_ids[o0 + r] : -1;
     __syncthreads();
-    const v4i ra = mfma2::make_rsrc(p.x, (uint32_t)((int64_t)x_rows * kb));
-    const v4i rb = mfma2::make_rsrc(p.w + (int64_t)e * p.N * kb, (uint32_t)((int64_t)p.N * kb));
-    auto dma_stage = [&](int st, int8_t *buf) {
-        const int k0 = st * SB;
-        for (int j = wave; j < NI; j += WAVES) {
-            const int idx = 64 * j + lane;
-            const int r = idx / UPR, slot = idx % UPR;
-            const int unit = slot ^ (r & 15);
-            if (r < 16 * RF) {
-                const int tok = s_tok[r];
-                const int base = tok >= 0 ? (tok / in_div) * kb : x_rows * kb;   // past the input: zeros
-                mfma2::dma16(ra, base + 16 * unit, k0, buf + j * 1024);
-            } else {
-                mfma2::dma16(rb, (n0 + r - 16 * RF) * kb + 16 * unit, k0, buf + j * 1024);
-            }
-        }
-    };
-    const bool hi = NI % WAVES == 0 || wave < NI % WAVES;
-    const int ns = kb / SB;
-    for (int st = 0; st < DEPTH && st < ns; ++st) dma_stage(st, lds + st * STAGE);
+    mfma2::RowsDma<16 * RF, 16 * NB, SB, false> dma;
+    dma.init(mfma2::make_rsrc(p.x, (uint32_t)((int64_t)x_rows * kb)),
+             mfma2::make_rsrc(p.w + (int64_t)e * p.N * kb, (uint32_t)((int64_t)p.N * kb)),
+             [&](int r) {
+                 const int tok = s_tok[r];
+                 return tok >= 0 ? (tok / in_div) * kb : x_rows * kb;   // past the input: zeros
+             },
+             n0, kb);
+    constexpr int HI = dma.HI, LO = dma.LO;
+    const bool hi = dma.hi();
+    const int ns = (kb + SB - 1) / SB;
+    for (int st = 0; st < DEPTH && st < ns; ++st) dma.issue(st, kb, lds + st * STAGE);
     const int c = wave % CH, f0 = wave / CH;
     const bool active = ALL || wave < RF * CH;   // wave-uniform
     Acc acc[FPW][NB];
@@ -564,7 +667,7 @@ __global__ __launch_bounds__(1024) void moe_rows_staged_kernel(MoeArgs p) {
         }
         }
         __syncthreads();
-        if (st + DEPTH < ns) dma_stage(st + DEPTH, buf);
+        if (st + DEPTH < ns) dma.issue(st + DEPTH, kb, buf);
     }
     Acc *part = reinterpret_cast<Acc *>(lds);
     if (active) {
@@ -669,6 +772,26 @@ __global__ __launch_bounds__(256) void moe_row_kernel(MoeArgs p) {
     }
 }
 
+// Tile shape by the dense tiles' model: an expert's rows end in a tile that is
+// half empty on average, so about size_m / TB + experts / 2 slots of TB rows
+// (the counts are on the GPU).  256 x 256 only where its kernel takes the
+// problem.
+inline mfma2::RingTile moe_tile_shape(int size_m, int E, int N, int kb, bool whole) {
+    int best = -1;
+    float us = 0.0f;
+    for (const int i : {mfma2::RT_64x128, mfma2::RT_128x128, mfma2::RT_128x256, mfma2::RT_256x256}) {
+        if (i == mfma2::RT_256x256 && !whole) continue;
+        const mfma2::RingCost &c = mfma2::kRingCost[i];
+        const float slots = (float)size_m / (float)c.tm + 0.5f * (float)std::min(E, size_m);
+        const float t = mfma2::ring_cost_tiles(c, (int64_t)(slots * (float)((N + c.tn - 1) / c.tn) + 0.5f), kb);
+        if (best < 0 || t < us) {
+            best = i;
+            us = t;
+        }
+    }
+    return (mfma2::RingTile)best;
+}
+
 // Offsets, then the grouped GEMM (DMA path when the problem fits it).
 template <int KIND>
 int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_counts,
@@ -681,6 +804,9 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
     // slab) and what its epilogue needs (out_ok).
     const int64_t kb = (int64_t)p.K * ES;
     const int64_t x_rows = p.topk_w ? p.size_m : (p.size_m + p.topk - 1) / p.topk;
+    const bool ring = kb % 16 == 0 && p.N % 8 == 0 && mfma::aligned16(p.x) && mfma::aligned16(p.w) &&
+                      (x_rows + 1) * kb < (1ll << 31) && (int64_t)(p.N + 256) * kb < (1ll << 31) && out_ok &&
+                      mfma::aligned16(p.out);
     const bool fast = kb % mfma2::BK == 0 && p.N % mfma2::BN == 0 && mfma::aligned16(p.x) &&
                       mfma::aligned16(p.w) && x_rows * kb < (1ll << 31) &&
                       (int64_t)p.N * kb < (1ll << 31) && out_ok;
@@ -697,7 +823,7 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
         // (2 / 3 tokens: 53.4 / 53.4 -> 48.0 / 48.0 us against the staged
         // kernel's 16-row blocks; at 2 pairs 22.5 against 22.4 us, at 8
         // 65.9 against 64.8 us: those stay staged)
-        if (fast && p.size_m > 2 && p.size_m <= 6 && kb % 1024 == 0 && p.N % 4 == 0) {
+        if (ring && p.size_m > 2 && p.size_m <= 6 && kb % 1024 == 0) {
             if (kb % 2048 == 0)
                 hipLaunchKernelGGL((moe_row_kernel<KIND, 2, 2>), dim3(p.N / 4, p.E), dim3(256), 0, stream, q);
             else
@@ -705,13 +831,18 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
             return launch_status();
         }
     }
-    if (fast && p.size_m <= 64 && kb % 512 == 0) {
+    if (ring && p.size_m <= 64) {
         // decode-sized.  N = 14336, K = 4096, E = 8, top-2: 1 / 4 / 16 tokens
         // (2 / 5 / 7 experts) in 27.4 / 62.3 / 99.0 us (with the offsets
         // kernel) against 43.5 / 100.5 / 117.8 on 256-row tiles; at size_m
         // 96 / 128 8 row fragments ran level with the tiles (123 us), so
         // larger size_m stays on them.
-        const int nb = mfma2::last_rows_col_frags(p.N);
+        // Columns per workgroup: the widest of 64, 32, 16 that leaves 192
+        // workgroups with rows, of about min(E, size_m) / 2 experts (the last
+        // group may lie partly past N).
+        const int touched = std::max(1, std::min(p.E, p.size_m) / 2);
+        int nb = 4;
+        while (nb > 1 && (int64_t)((p.N + 16 * nb - 1) / (16 * nb)) * touched < 192) nb /= 2;
         // blocks of 16 rows up to 32 pairs, of 32 above (blockIdx.z): an
         // expert's few rows stage fewer padding rows (N = 14336, K = 4096,
         // 1 / 8 / 16 / 32 tokens top-2: 22.6 / 80.7 / 95.5 / 106.6 -> 21.6 /
@@ -720,7 +851,7 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
 #define BK_MOEROWS(RF, NB, SB, DEPTH)                                                                        \
         if (rfz == (RF) && nb == (NB)) {                                                                     \
             hipLaunchKernelGGL((moe_rows_staged_kernel<KIND, RF, NB, SB, DEPTH>),                            \
-                               dim3(p.N / (16 * (NB)), p.E, (p.size_m + 16 * (RF) - 1) / (16 * (RF))),      \
+                               dim3((p.N + 16 * (NB) - 1) / (16 * (NB)), p.E, (p.size_m + 16 * (RF) - 1) / (16 * (RF))), \
                                dim3(1024),                                                                   \
                                std::max((size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB),                    \
                                         (size_t)(RF) * (NB) * ((SB) / 64) * 1024) + 64 * (RF),               \
@@ -729,7 +860,7 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
         }
         BK_MOEROWS(1, 1, 512, 3)
         BK_MOEROWS(1, 2, 512, 3)
-        BK_MOEROWS(1, 4, 512, 3)
+        BK_MOEROWS(1, 4, 512, 2)
         BK_MOEROWS(2, 1, 512, 3)
         BK_MOEROWS(2, 2, 512, 3)
         BK_MOEROWS(2, 4, 512, 3)
@@ -738,6 +869,15 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
     hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(1024), 0, stream, expert_ids, p.size_m, p.E,
                        expert_counts, const_cast<int32_t *>(p.offsets));
     if (hipPeekAtLastError() != hipSuccess) return kLaunch;
+    if (ring) {
+        using mfma2::Cfg;
+        switch (moe_tile_shape(p.size_m, p.E, p.N, (int)kb, fast)) {
+            case mfma2::RT_64x128: launch_moe_ring<KIND, Cfg<2, 2, 64, 128>, 3, 2>(p, stream); return launch_status();
+            case mfma2::RT_128x128: launch_moe_ring<KIND, Cfg<4, 2, 128, 128>, 3, 2>(p, stream); return launch_status();
+            case mfma2::RT_128x256: launch_moe_ring<KIND, Cfg<2, 4, 128, 256>, 3, 4>(p, stream); return launch_status();
+            default: break;
+        }
+    }
     if (fast) {
         const int work = slots * (p.N / mfma2::BN);
         const int padded = (work + 7) / 8 * 8;   // whole XCD groups

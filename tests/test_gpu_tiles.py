@@ -1,8 +1,8 @@
-"""The mid-size block tiles of the RCR GEMMs and depths off the 128-byte stage.
+"""Block tiles of the GEMMs and the grouped MoE, and depths off the 128-byte stage.
 
-Shapes pick each tile of the chooser (64x64 to 256x256) with ragged M and N
-edges and K a multiple of 16 only (last stages of 16, 64 and 112 bytes), and
-the last-rows kernels with partial last stages.  Integer results are exact
+Shapes pick each tile of the choosers (64x64 to 256x256) with ragged M and N
+edges and K a multiple of 16 bytes only (last stages of 16, 64 and 112 bytes),
+and the last-rows kernels with partial last stages.  Integer results are exact
 against float64 products (sums below 2^53).
 """
 import numpy as np
@@ -11,9 +11,11 @@ import torch
 
 from baracuda_amd import plans as P
 from baracuda_amd.ffi import lib
-from oracle.inputs import int8_uniform, rng
+from oracle.inputs import int8_uniform, moe_routing, rng
+from tests import test_gpu_moe_wmma as W
 from tests import test_gpu_sweep as S
 from tests.gpu_util import FP8_FLOOR, dev, host_bits16, sync
+from tests.test_gpu_moe import _block_routing, _run as _moe_run
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +133,33 @@ def test_rrr_and_u8_depth_tails(gpu, shape):
     S.test_int8_rrr_bias_relu_sweep(gpu, shape)
     S.test_u8_rcr_sweep(gpu, shape)
     S.test_u8_rrr_sweep(gpu, shape, False)
+
+
+# experts' row counts (ends of 64- and 128-row tiles, empty experts, more than
+# 64 experts), N and K in bytes off 256 / 128
+MOE_CASES = [([64, 1, 0, 129, 65, 300], 328, 208), ([3] * 70 + [0] * 30 + [200] * 3, 136, 80),
+             ([700, 0, 641, 1200], 2312, 1040), ([2000, 1900, 1800, 2048], 2056, 272), ([90] * 16, 1408, 336),
+             ([5, 0, 17, 1, 33], 360, 1040), ([1, 0, 1], 72, 48), ([20, 12], 1416, 3088)]
+
+
+@pytest.mark.parametrize("case", MOE_CASES)
+def test_moe_s8_tiles_and_depth_tails(gpu, case):
+    counts, n, k = case
+    print(f"case: moe s8 rows={counts[:8]} n={n} k={k}", flush=True)
+    tokens, routing = _block_routing(counts, seed=n + k)
+    _moe_run(tokens=tokens, E=len(counts), topk=1, n=n, k=k, seed=n, routing=routing)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("t", ["bf16", "f16"])
+@pytest.mark.parametrize("shape", [(150, 8, 2, 328, 104), (40, 70, 3, 136, 264), (600, 4, 2, 264, 520), (12, 6, 2, 72, 136)])
+def test_moe_float_tiles_and_depth_tails(gpu, shape, t, weighted):
+    tokens, e, topk, n, k = shape
+    print(f"case: moe {t} {shape} weighted={weighted}", flush=True)
+    g = rng(tokens + e + n + k)
+    sid, eid = moe_routing(tokens, e, topk, seed=tokens)[:2]
+    rows = tokens * topk
+    x = g.standard_normal((rows if weighted else tokens, k)).astype(np.float32)
+    w = (g.standard_normal((e, n, k)) / np.sqrt(k)).astype(np.float32)
+    tw = g.uniform(0.1, 1.0, rows).astype(np.float32) if weighted else None
+    W._check(*W._run(t, x, w, sid, eid, topk, tw, rows), t)
