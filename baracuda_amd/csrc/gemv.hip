@@ -18,6 +18,8 @@
 //    the 16 partials are summed in LDS in slice order.  Fixed order => the
 //    result does not depend on grid shape and replays bit-identically.
 //    beta == 0 never reads D (write-only, gemv_dense.cu:163-169).
+#include <type_traits>
+
 #include "bk_common.hpp"
 
 namespace bk {
@@ -128,6 +130,63 @@ __global__ __launch_bounds__(64) void gemv_s8w_m1_kernel(
     for (int r = 0; r < ROWS; ++r) o[r] = f32_to_bf16_rne(wave_sum_lane63(acc[r]) * sc[r]);
     if (lane == 63) {
         if (ROWS == 2 && (EVEN || (row0 + 1 < N && (reinterpret_cast<uintptr_t>(d + row0) & 3u) == 0))) {
+            *reinterpret_cast<uint32_t *>(d + row0) = (uint32_t)o[0] | ((uint32_t)o[ROWS - 1] << 16);
+        } else {
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r)
+                if (row0 + r < N) d[row0 + r] = o[r];
+        }
+    }
+}
+
+// K % 16 == 0 off the kilobyte, with the same rows per wave and loads as above:
+// weights and x through buffer resources of K and 2 K bytes, so the units past
+// K of the last kilobyte read as zeros (and move nothing) without a branch.
+// One byte per lane and load, 21156 x 4672 from HBM took 97 us, now 18.7 (5.3 TB/s);
+// 30000 x 11008 309 -> 63.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+template <int ROWS, int B>
+__global__ __launch_bounds__(64) void gemv_s8w_m1_any_kernel(
+    int N, int K, const uint16_t *__restrict__ x, const int8_t *__restrict__ w, int64_t ldw,
+    const float *__restrict__ scale, uint16_t *__restrict__ d) {
+    constexpr int kRaw = 0x00020000, kNt = 2;   // raw buffer format word; non-temporal
+    const int lane = threadIdx.x & 63;
+    const int row0 = blockIdx.x * ROWS;
+    float sc[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) sc[r] = scale[min(row0 + r, N - 1)];
+    const rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(x), 0, 2 * K, kRaw);
+    rsrc_t rw[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+        rw[r] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(w) + (int64_t)min(row0 + r, N - 1) * ldw, 0, K, kRaw);
+    float acc[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) acc[r] = 0.0f;
+    for (int k0 = 0; k0 < K; k0 += 1024 * B) {
+        v4i wv[B][ROWS], xlo[B], xhi[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            xlo[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rx, 32 * lane, 2 * (k0 + 1024 * u), 0));
+            xhi[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rx, 32 * lane + 16, 2 * (k0 + 1024 * u), 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r)
+                wv[u][r] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw[r], 16 * lane, k0 + 1024 * u, kNt));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) acc[r] = dot16_s8_bf16(wv[u][r], xlo[u], xhi[u], acc[r]);
+    }
+    uint16_t o[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) o[r] = f32_to_bf16_rne(wave_sum_lane63(acc[r]) * sc[r]);
+    if (lane == 63) {
+        if (ROWS == 2 && row0 + 1 < N && (reinterpret_cast<uintptr_t>(d + row0) & 3u) == 0) {
             *reinterpret_cast<uint32_t *>(d + row0) = (uint32_t)o[0] | ((uint32_t)o[ROWS - 1] << 16);
         } else {
 #pragma unroll
@@ -304,8 +363,8 @@ __global__ __launch_bounds__(1024) void gemv_dense_m1_vec_kernel(
 // read-only probe of it moves the 32 MiB of a bf16 K = N = 4096 B in 16 us,
 // the same bytes read contiguously take 6 us.
 //   pass 1: workgroup (slice s, column group g): 256 threads x 16 bytes of
-//           columns over the split_rows<Tag>() rows of slice s (16 for 16-bit
-//           elements, 8 for f32); partial[s][col] =
+//           columns over the rows of slice s (16 for 16-bit elements, 8 for
+//           f32, more in large problems, see split_rows_for); partial[s][col] =
 //           sum over the slice's k (ascending) of a[k] * B[k, col]
 //   pass 2: total = sum over s of partial[s][col] (16 ascending runs of
 //           slices, added in run order); D = alpha * total (+ beta * D)
@@ -321,21 +380,34 @@ template <typename Tag>
 constexpr int split_rows() { return sizeof(typename Codec<Tag>::S) == 4 ? 8 : 16; }
 constexpr int kSplitThreads = 256;
 
+// Rows per slice of a problem: `split_rows` times as many as leave about 4096
+// workgroups (at most 16 times), since the float partials of every slice are
+// written and read back: a quarter of B's bytes.  f32, four 5198 x 19552
+// matrices 379 -> 284 us (5.7 TB/s), bf16, 8192 x 32000 117 -> 108.
 template <typename Tag>
+inline int split_rows_for(int64_t n, int64_t k, int64_t batch) {
+    constexpr int EPL = 16 / (int)sizeof(typename Codec<Tag>::S);
+    const int64_t slices = (k + split_rows<Tag>() - 1) / split_rows<Tag>();
+    const int64_t wgs = slices * ((n / EPL + kSplitThreads - 1) / kSplitThreads) * batch;
+    int mult = 1;
+    while (mult < 16 && wgs / (2 * mult) >= 4096) mult *= 2;
+    return split_rows<Tag>() * mult;
+}
+
+template <typename Tag, bool Tall>
 __global__ __launch_bounds__(kSplitThreads) void gemv_dense_split_partial_kernel(
-    int n, int k, const typename Codec<Tag>::S *__restrict__ a, int64_t stride_a,
+    int n, int k, int rows, const typename Codec<Tag>::S *__restrict__ a, int64_t stride_a,
     const typename Codec<Tag>::S *__restrict__ b, int64_t ldb, int64_t stride_b, float *__restrict__ part) {
     typedef Codec<Tag> C;
     typedef typename C::S S;
     constexpr int EPL = 16 / (int)sizeof(S);
     constexpr int kSplitRows = split_rows<Tag>();
-    const int slices = (k + kSplitRows - 1) / kSplitRows;
+    const int slices = Tall ? gridDim.x : (k + kSplitRows - 1) / kSplitRows;
     const int s = blockIdx.x, slot = blockIdx.z;
     const int col = (blockIdx.y * kSplitThreads + threadIdx.x) * EPL;
     if (col >= n) return;
     const S *arow = a + (int64_t)slot * stride_a;
     const S *bcol = b + (int64_t)slot * stride_b + col;
-    const int k0 = s * kSplitRows, k1 = min(k, k0 + kSplitRows);
     float acc[EPL];
 #pragma unroll
     for (int e = 0; e < EPL; ++e) acc[e] = 0.0f;
@@ -352,21 +424,43 @@ __global__ __launch_bounds__(kSplitThreads) void gemv_dense_split_partial_kernel
             }
         }
     };
-    if (k1 - k0 == kSplitRows) {
-        // whole slice (uniform branch): every row load issued before the first FMA
-        v4i w[kSplitRows];
-        float av[kSplitRows];
+    auto add_rows = [&](int k0, int k1) {
+        if (k1 - k0 == kSplitRows) {
+            // whole group (uniform branch): every row load issued before the first FMA
+            v4i w[kSplitRows];
+            float av[kSplitRows];
 #pragma unroll
-        for (int r = 0; r < kSplitRows; ++r)
-            w[r] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(bcol + (int64_t)(k0 + r) * ldb));
+            for (int r = 0; r < kSplitRows; ++r)
+                w[r] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(bcol + (int64_t)(k0 + r) * ldb));
 #pragma unroll
-        for (int r = 0; r < kSplitRows; ++r) av[r] = C::ld(arow[k0 + r]);
+            for (int r = 0; r < kSplitRows; ++r) av[r] = C::ld(arow[k0 + r]);
 #pragma unroll
-        for (int r = 0; r < kSplitRows; ++r) fma_row(w[r], av[r]);
+            for (int r = 0; r < kSplitRows; ++r) fma_row(w[r], av[r]);
+        } else {
+            for (int kk = k0; kk < k1; ++kk)
+                fma_row(__builtin_nontemporal_load(reinterpret_cast<const v4i *>(bcol + (int64_t)kk * ldb)),
+                        C::ld(arow[kk]));
+        }
+    };
+    if constexpr (Tall) {
+        // each group's sum by itself, then the groups in order: chains no longer
+        // than the short slices' (one chain over a slice measured 1.7e-7 from
+        // the f64 result at 5198 x 19552 f32, short slices 1.5e-7)
+        float sum[EPL];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) sum[e] = 0.0f;
+        for (int k0 = s * rows, end = min(k, k0 + rows); k0 < end; k0 += kSplitRows) {
+            add_rows(k0, min(end, k0 + kSplitRows));
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+                sum[e] += acc[e];
+                acc[e] = 0.0f;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[e] = sum[e];
     } else {
-        for (int kk = k0; kk < k1; ++kk)
-            fma_row(__builtin_nontemporal_load(reinterpret_cast<const v4i *>(bcol + (int64_t)kk * ldb)),
-                    C::ld(arow[kk]));
+        add_rows(s * kSplitRows, min(k, (s + 1) * kSplitRows));
     }
     float *dst = part + ((int64_t)slot * slices + s) * n + col;
 #pragma unroll
@@ -377,14 +471,14 @@ __global__ __launch_bounds__(kSplitThreads) void gemv_dense_split_partial_kernel
 // Pass 2: workgroup of 16 waves per 64 columns; wave w sums the slices
 // [w*per, (w+1)*per) of its lane's column in ascending order, then the 16
 // wave sums are added in wave order.
-template <typename Tag>
+template <typename Tag, bool Tall>
 __global__ __launch_bounds__(1024) void gemv_dense_split_reduce_kernel(
-    int n, int k, float alpha, float beta, const float *__restrict__ part, typename Codec<Tag>::S *__restrict__ d,
+    int n, int k, int rows, float alpha, float beta, const float *__restrict__ part, typename Codec<Tag>::S *__restrict__ d,
     int64_t stride_d) {
     typedef Codec<Tag> C;
     __shared__ float ws[16][64];
     constexpr int kSplitRows = split_rows<Tag>();
-    const int slices = (k + kSplitRows - 1) / kSplitRows;
+    const int slices = Tall ? (k + rows - 1) / rows : (k + kSplitRows - 1) / kSplitRows;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = blockIdx.x * 64 + lane, slot = blockIdx.y;
     const int per = (slices + 15) / 16;
@@ -465,12 +559,19 @@ int32_t launch_dense(int32_t m, int32_t n, int32_t k, int32_t batch, int32_t lay
         ((int64_t)ldb * (int64_t)sizeof(S)) % 16 == 0 && ((int64_t)stride_b * (int64_t)sizeof(S)) % 16 == 0 &&
         (reinterpret_cast<uintptr_t>(b) & 15u) == 0) {
         constexpr int EPL = 16 / (int)sizeof(S);
-        const int slices = (k + split_rows<Tag>() - 1) / split_rows<Tag>();
+        const int rows = split_rows_for<Tag>(n, k, batch);
+        const int slices = (k + rows - 1) / rows;
         const int groups = (n / EPL + kSplitThreads - 1) / kSplitThreads;
-        hipLaunchKernelGGL((gemv_dense_split_partial_kernel<Tag>), dim3(slices, groups, batch), dim3(kSplitThreads),
-                           0, stream, n, k, (const S *)a, stride_a, (const S *)b, ldb, stride_b, (float *)workspace);
-        hipLaunchKernelGGL((gemv_dense_split_reduce_kernel<Tag>), dim3((n + 63) / 64, batch), dim3(1024), 0, stream,
-                           n, k, alpha, beta, (const float *)workspace, (S *)d, stride_d);
+        auto go = [&](auto tall) {
+            constexpr bool kTall = decltype(tall)::value;
+            hipLaunchKernelGGL((gemv_dense_split_partial_kernel<Tag, kTall>), dim3(slices, groups, batch),
+                               dim3(kSplitThreads), 0, stream, n, k, rows, (const S *)a, stride_a, (const S *)b, ldb,
+                               stride_b, (float *)workspace);
+            hipLaunchKernelGGL((gemv_dense_split_reduce_kernel<Tag, kTall>), dim3((n + 63) / 64, batch), dim3(1024), 0,
+                               stream, n, k, rows, alpha, beta, (const float *)workspace, (S *)d, stride_d);
+        };
+        if (rows == split_rows<Tag>()) go(std::false_type{});
+        else go(std::true_type{});
         return launch_status();
     }
     if (vec) {
@@ -513,14 +614,24 @@ int32_t baracuda_kernels_gemv_s8w_m1_bf16_gfx950_run(int32_t n, int32_t k, const
     if (n == 0) return kOk;
     if (!x || !w || !scale || !d) return kInvalid;
     hipStream_t stream = (hipStream_t)stream_ptr;
-    const bool fast = k > 0 && k % 1024 == 0 && ldw % 16 == 0 &&
+    const bool fast = k > 0 && k % 16 == 0 && k < (1 << 29) && ldw % 16 == 0 &&
                       (reinterpret_cast<uintptr_t>(w) & 15u) == 0 &&
                       (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
     if (fast) {
         const int waves = (n + kGemvRows - 1) / kGemvRows;
         const int chunks = k / 1024;
         const bool even = n % kGemvRows == 0 && (reinterpret_cast<uintptr_t>(d) & 3u) == 0;
-        if (chunks == 4 && even)
+        if (k % 1024 != 0) {
+            // batches that divide the kilobytes, the partial one counted
+            const int c = chunks + 1;
+            auto go = [&](auto b) {
+                hipLaunchKernelGGL((gemv_s8w_m1_any_kernel<kGemvRows, decltype(b)::value>), dim3(waves), dim3(64), 0, stream,
+                                   n, k, (const uint16_t *)x, (const int8_t *)w, ldw, (const float *)scale, (uint16_t *)d);
+            };
+            if (c % 4 == 0) go(std::integral_constant<int, 4>{});
+            else if (c % 2 == 0) go(std::integral_constant<int, 2>{});
+            else go(std::integral_constant<int, 1>{});
+        } else if (chunks == 4 && even)
             hipLaunchKernelGGL((gemv_s8w_m1_kernel<kGemvRows, 4, 4, true>), dim3(waves), dim3(64), 0, stream, n, k,
                                (const uint16_t *)x, (const int8_t *)w, ldw, (const float *)scale, (uint16_t *)d);
         else if (chunks == 4)

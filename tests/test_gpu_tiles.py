@@ -15,6 +15,7 @@ from oracle.inputs import int8_uniform, moe_routing, rng
 from tests import test_gpu_moe_wmma as W
 from tests import test_gpu_sweep as S
 from tests.gpu_util import FP8_FLOOR, dev, host_bits16, sync
+from tests.test_gpu_decode import _gemv_check, _gemv_inputs, _gemv_run
 from tests.test_gpu_moe import _block_routing, _run as _moe_run
 
 pytestmark = pytest.mark.gpu
@@ -163,3 +164,31 @@ def test_moe_float_tiles_and_depth_tails(gpu, shape, t, weighted):
     w = (g.standard_normal((e, n, k)) / np.sqrt(k)).astype(np.float32)
     tw = g.uniform(0.1, 1.0, rows).astype(np.float32) if weighted else None
     W._check(*W._run(t, x, w, sid, eid, topk, tw, rows), t)
+
+
+@pytest.mark.parametrize("shape", [(1, 16), (5, 1040), (4097, 4672), (300, 3072), (130, 8176), (64, 11008), (7, 4080)])
+def test_gemv_s8w_depth_tails(gpu, shape):
+    print(f"case: gemv_s8w depth tail {shape}", flush=True)
+    w, scale, xb = _gemv_inputs(*shape, seed=shape[0] + shape[1])
+    _gemv_check(_gemv_run(w, scale, xb), w, scale, xb)
+
+
+@pytest.mark.parametrize("dtype,n,k,batch", [(torch.bfloat16, 4096, 8199, 8), (torch.float32, 4100, 4099, 8)])
+def test_gemv_dense_tall_slices(gpu, dtype, n, k, batch):
+    """Split-K slices of several row groups, the last one short (f32 sums)."""
+    print(f"case: gemv_dense {dtype} {batch}x{k}x{n}", flush=True)
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(n + k)
+    a = torch.empty((batch, k), dtype=dtype, device="cuda:0").normal_(generator=g)
+    b = torch.empty((batch, k, n), dtype=dtype, device="cuda:0").normal_(0.0, k ** -0.5, generator=g)
+    d = torch.empty((batch, n), dtype=dtype, device="cuda:0")
+    plan = P.GemvDensePlan.select(P.GemvDenseDescriptor(n, k, batch), dtype)
+    ws = torch.empty(plan.workspace_size(), dtype=torch.uint8, device="cuda:0")
+    plan.run(a, b, d, lda=k, stride_a=k, ldb=n, stride_b=k * n, ldd=n, stride_d=n, workspace=ws)
+    sync()
+    for i in range(batch):
+        x, w = a[i].double(), b[i].double()
+        exact, mag = x @ w, x.abs() @ w.abs()
+        # f32 sums of k products in chains of at most 128 + 64 + 16 additions, one output rounding
+        bound = 208 * 2.0 ** -24 * mag + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * exact.abs()
+        assert bool(((d[i].double() - exact).abs() <= bound).all())
