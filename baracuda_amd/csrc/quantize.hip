@@ -18,7 +18,9 @@
 // of x, one write of q (8-byte stores on the bf16 path).  Longer rows
 // take a two-pass loop over global memory.  Max is exact
 // in any order, so the result is bit-identical to the reference's.
-#include "bk_common.hpp"
+#include <type_traits>
+
+#include "quant.hpp"
 
 namespace bk {
 namespace {
@@ -34,28 +36,9 @@ template <> struct QIn<float> {
 template <> struct QIn<double> {
     __device__ static float ld(const double *p) { return (float)*p; }
 };
-struct Bf16In { uint16_t bits; };   // element type: pointer steps of 2 bytes
 template <> struct QIn<Bf16In> {
     __device__ static float ld(const Bf16In *p) { return bf16_to_f32(p->bits); }
 };
-
-__device__ __forceinline__ float block_max(float v, float *red) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) red[wave] = v;
-    __syncthreads();
-    float m = red[0];
-#pragma unroll
-    for (int w = 1; w < kQBlock / 64; ++w) m = fmaxf(m, red[w]);
-    return m;
-}
-
-// clamp(round_half_even(v * inv), qmin, qmax), the clamp in float before the
-// conversion (rne_clamp: NaN -> 0, no out-of-range conversion).
-__device__ __forceinline__ int8_t quant1(float v, float inv, float qmin, float qmax) {
-    return (int8_t)(int)rne_clamp(v * inv, qmin, qmax);
-}
 
 // T: element type of x; S: type of the scale output.
 template <typename T, typename S>
@@ -82,7 +65,7 @@ __global__ __launch_bounds__(kQBlock) void quantize_per_token_kernel(
         } else {
             for (int e = threadIdx.x; e < D; e += kQBlock) m = fmaxf(m, fabsf(QIn<T>::ld(row + e)));
         }
-        const float max_abs = block_max(m, red);
+        const float max_abs = block_max<kQBlock / 64>(m, red);
         const float s = max_abs > 0.0f ? max_abs / fqmax : 1.0f;
         const float inv = s != 0.0f ? 1.0f / s : 0.0f;
         if (threadIdx.x == 0) scale[n] = (S)s;
@@ -100,55 +83,55 @@ __global__ __launch_bounds__(kQBlock) void quantize_per_token_kernel(
     }
 }
 
-// Vector path for 2-byte inputs (bf16): 16-byte non-temporal loads of 8
-// elements, 8-byte non-temporal int8 stores; chunk c = tid + kQBlock * i, kChunks chunks
-// (8 * kChunks values) per thread held in registers (D <= 2048 * kChunks,
-// D % 8 == 0, 16-byte aligned rows).  The launcher picks the smallest of
-// 1, 2, 4, 8 chunks that holds the row: fewer registers keep more rows in
-// flight (4096 x 4096: 14.3 us with 8 chunks, 10.9 us with 2).
-template <typename S, int kChunks>
-__global__ __launch_bounds__(kQBlock) void quantize_per_token_bf16v_kernel(
-    const uint16_t *__restrict__ x, S *__restrict__ scale, int8_t *__restrict__ q, int N, int D,
+// Codes that the caches can hold stay in them for the GEMM that reads them
+// next; larger streams go past them.  Quantizer and GEMM, us, non-temporal ->
+// kept: bf16 4096 x 4096 to 4096 columns 69.7 -> 65.7, 4096 x 14336 to 4096 226
+// -> 221, 2000 x 11008 to 1024 52.8 -> 44.8, f32 777 x 4096 to 11008 55.1 ->
+// 47.8.  (The quantizer alone, its output not read, prefers non-temporal
+// stores: bf16 4096 x 4096 10.9 us against 11.6.)
+constexpr int64_t kQKeepBytes = 64ll << 20;
+template <bool Keep>
+__device__ __forceinline__ void store_codes(const v2i &v, int8_t *dst) {
+    if constexpr (Keep) *reinterpret_cast<v2i *>(dst) = v;
+    else __builtin_nontemporal_store(v, reinterpret_cast<v2i *>(dst));
+}
+
+// Vector path (bf16, f32): 16-byte non-temporal loads, 8-byte non-temporal
+// int8 stores; chunk of 8 values c = tid + BLOCK * i, kChunks of them per thread
+// held in registers (D <= 8 * BLOCK * kChunks, D % 8 == 0, 16-byte aligned
+// rows).  The launcher picks the smallest of 1, 2, 4, 8 chunks that holds the
+// row: fewer registers keep more rows in flight (bf16, 4096 x 4096: 14.3 us
+// with 8 chunks, 10.9 us with 2).  f32 rows read 4 bytes per lane and load
+// before: 777 x 4096 10.3 -> 5.3 us.
+template <typename T, typename S, int BLOCK, int kChunks, bool kKeep>
+__global__ __launch_bounds__(BLOCK) void quantize_per_token_vec_kernel(
+    const T *__restrict__ x, S *__restrict__ scale, int8_t *__restrict__ q, int N, int D,
     int qmin, int qmax) {
-    __shared__ float red[kQBlock / 64];
+    __shared__ float red[BLOCK / 64];
     const float fqmax = (float)qmax;
     const float fqmin = (float)qmin;
     const int nch = D >> 3;
     for (int n = blockIdx.x; n < N; n += gridDim.x) {
-        const v4i *row = reinterpret_cast<const v4i *>(x + (int64_t)n * D);
-        v4i w[kChunks];
-        float m = 0.0f;
+        const T *row = x + (int64_t)n * D;
+        QChunk<T> w[kChunks];
 #pragma unroll
         for (int i = 0; i < kChunks; ++i) {
-            const int c = threadIdx.x + kQBlock * i;
-            w[i] = c < nch ? __builtin_nontemporal_load(row + c) : v4i{0, 0, 0, 0};
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                const uint32_t u = (uint32_t)w[i][h];
-                m = fmaxf(m, fabsf(__uint_as_float(u << 16)));
-                m = fmaxf(m, fabsf(__uint_as_float(u & 0xffff0000u)));
-            }
+            const int c = threadIdx.x + BLOCK * i;
+            if (c < nch) w[i].load(row, c);
+            else w[i].clear();
         }
-        const float max_abs = block_max(m, red);
-        const float s = max_abs > 0.0f ? max_abs / fqmax : 1.0f;
-        const float inv = s != 0.0f ? 1.0f / s : 0.0f;
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kChunks; ++i) m = chunk_max(w[i], m);
+        float s, inv;
+        quant_scale(block_max<BLOCK / 64>(m, red), fqmax, s, inv);
         if (threadIdx.x == 0) scale[n] = (S)s;
         int8_t *qrow = q + (int64_t)n * D;
 #pragma unroll
         for (int i = 0; i < kChunks; ++i) {
-            const int c = threadIdx.x + kQBlock * i;
+            const int c = threadIdx.x + BLOCK * i;
             if (c >= nch) break;
-            uint32_t lo = 0, hi = 0;
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                const uint32_t u = (uint32_t)w[i][h];
-                const uint32_t q0 = (uint8_t)quant1(__uint_as_float(u << 16), inv, fqmin, fqmax);
-                const uint32_t q1 = (uint8_t)quant1(__uint_as_float(u & 0xffff0000u), inv, fqmin, fqmax);
-                const uint32_t pair = q0 | (q1 << 8);
-                if (h < 2) lo |= pair << (16 * h);
-                else hi |= pair << (16 * (h - 2));
-            }
-            __builtin_nontemporal_store(v2i{(int)lo, (int)hi}, reinterpret_cast<v2i *>(qrow + 8 * c));
+            store_codes<kKeep>(chunk_codes(w[i], inv, fqmin, fqmax), qrow + 8 * c);
         }
         __syncthreads();   // `red` is reused by the next row
     }
@@ -160,10 +143,11 @@ __global__ __launch_bounds__(kQBlock) void quantize_per_token_bf16v_kernel(
 // barrier), 8-byte non-temporal int8 stores.  kEven: D == 512 kChunks, no
 // per-chunk guards (they cost 0.7 us at 4096 x 4096).  4096 x 4096 over 24
 // rotated input / output pairs: 10.05 us against 10.7-10.9 for
-// quantize_per_token_bf16v_kernel and 9.45 us for a copy with the same
+// quantize_per_token_vec_kernel and 9.45 us for a copy with the same
 // loads and stores and no arithmetic (bit-identical).
 constexpr int kQRowsPerBlock = 4;
-template <typename S, int kChunks, bool kEven>
+constexpr int kQFewRows = 256;   // a workgroup per row up to here (one per CU)
+template <typename S, int kChunks, bool kEven, bool kKeep>
 __global__ __launch_bounds__(64 * kQRowsPerBlock) void quantize_per_token_bf16w_kernel(
     const uint16_t *__restrict__ x, S *__restrict__ scale, int8_t *__restrict__ q, int N, int D,
     int qmin, int qmax) {
@@ -207,7 +191,7 @@ __global__ __launch_bounds__(64 * kQRowsPerBlock) void quantize_per_token_bf16w_
                 if (h < 2) lo |= pair << (16 * h);
                 else hi |= pair << (16 * (h - 2));
             }
-            __builtin_nontemporal_store(v2i{(int)lo, (int)hi}, reinterpret_cast<v2i *>(qrow + 8 * c));
+            store_codes<kKeep>(v2i{(int)lo, (int)hi}, qrow + 8 * c);
         }
     }
 }
@@ -227,46 +211,54 @@ int32_t launch_quant(int32_t N, int32_t D, int32_t qmin, int32_t qmax, const voi
     if ((int64_t)N * D == 0) return kOk;
     if (!input || !scale || !output) return kInvalid;
     const int grid = N < 65535 ? N : 65535;
-    if constexpr (sizeof(T) == 2) {
+    if constexpr (sizeof(T) <= 4) {
         const bool vec = D % 8 == 0 && D <= kQBlock * kQMaxPerThread &&
                          (reinterpret_cast<uintptr_t>(input) & 15u) == 0 &&
                          (reinterpret_cast<uintptr_t>(output) & 7u) == 0;
-        if (vec) {
-            const uint16_t *xi = (const uint16_t *)input;
-            S *sc = (S *)scale;
-            int8_t *qo = (int8_t *)output;
-            const int nch = D / 8;
-            if (nch <= 64 * 8) {
+        const int nch = D / 8;
+        const bool keep = (int64_t)N * D <= kQKeepBytes;
+        // Rows of up to 4096 bf16 values, one wave each, from kQFewRows on: below
+        // that the chip is idle and a row's 64 values per lane are the time (1 x
+        // 4096 bf16 3.1 -> 2.6 us, 24 x 4096 4.7 -> 3.2 in a kernel trace).
+        if (vec && sizeof(T) == 2 && N > kQFewRows && nch <= 64 * 8) {
+            if constexpr (sizeof(T) == 2) {
+                const uint16_t *xi = (const uint16_t *)input;
+                S *sc = (S *)scale;
+                int8_t *qo = (int8_t *)output;
                 const int wgrid = (N + kQRowsPerBlock - 1) / kQRowsPerBlock < 65535
                                       ? (N + kQRowsPerBlock - 1) / kQRowsPerBlock : 65535;
                 const dim3 wb(64 * kQRowsPerBlock);
 #define BK_QW(CH)                                                                                          \
-    if (nch == 64 * (CH))                                                                                  \
-        hipLaunchKernelGGL((quantize_per_token_bf16w_kernel<S, CH, true>), dim3(wgrid), wb, 0, stream, xi, \
-                           sc, qo, N, D, qmin, qmax);                                                      \
-    else                                                                                                   \
-        hipLaunchKernelGGL((quantize_per_token_bf16w_kernel<S, CH, false>), dim3(wgrid), wb, 0, stream, xi, \
-                           sc, qo, N, D, qmin, qmax);
+    auto go = [&](auto even, auto keep) {                                                                  \
+        hipLaunchKernelGGL((quantize_per_token_bf16w_kernel<S, CH, decltype(even)::value, decltype(keep)::value>), \
+                           dim3(wgrid), wb, 0, stream, xi, sc, qo, N, D, qmin, qmax);                      \
+    };                                                                                                     \
+    if (nch == 64 * (CH)) keep ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{}); \
+    else keep ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
                 if (nch <= 64) { BK_QW(1) }
                 else if (nch <= 128) { BK_QW(2) }
                 else if (nch <= 256) { BK_QW(4) }
                 else { BK_QW(8) }
 #undef BK_QW
-                return launch_status();
             }
-            if (nch <= kQBlock)
-                hipLaunchKernelGGL((quantize_per_token_bf16v_kernel<S, 1>), dim3(grid), dim3(kQBlock), 0, stream,
-                                   xi, sc, qo, N, D, qmin, qmax);
-            else if (nch <= 2 * kQBlock)
-                hipLaunchKernelGGL((quantize_per_token_bf16v_kernel<S, 2>), dim3(grid), dim3(kQBlock), 0, stream,
-                                   xi, sc, qo, N, D, qmin, qmax);
-            else if (nch <= 4 * kQBlock)
-                hipLaunchKernelGGL((quantize_per_token_bf16v_kernel<S, 4>), dim3(grid), dim3(kQBlock), 0, stream,
-                                   xi, sc, qo, N, D, qmin, qmax);
-            else
-                hipLaunchKernelGGL((quantize_per_token_bf16v_kernel<S, 8>), dim3(grid), dim3(kQBlock), 0, stream,
-                                   xi, sc, qo, N, D, qmin, qmax);
             return launch_status();
+        }
+        if (vec) {
+#define BK_QV(BLOCK, CH)                                                                                   \
+    if (nch <= (BLOCK) * (CH)) {                                                                           \
+        auto go = [&](auto k) {                                                                            \
+            hipLaunchKernelGGL((quantize_per_token_vec_kernel<T, S, BLOCK, CH, decltype(k)::value>), dim3(grid), \
+                               dim3(BLOCK), 0, stream, (const T *)input, (S *)scale, (int8_t *)output, N, D, qmin, qmax); \
+        };                                                                                                 \
+        keep ? go(std::true_type{}) : go(std::false_type{});                                               \
+        return launch_status();                                                                            \
+    }
+            if (N <= kQFewRows) {
+                BK_QV(256, 1) BK_QV(512, 1) BK_QV(512, 2) BK_QV(512, 4)
+            } else {
+                BK_QV(256, 1) BK_QV(256, 2) BK_QV(256, 4) BK_QV(256, 8)
+            }
+#undef BK_QV
         }
     }
     hipLaunchKernelGGL((quantize_per_token_kernel<T, S>), dim3(grid), dim3(kQBlock), 0, stream,

@@ -12,6 +12,7 @@ import torch
 from baracuda_amd import plans as P
 from baracuda_amd.ffi import lib
 from oracle.inputs import int8_uniform, moe_routing, rng
+from tests import test_gpu_gemm as G
 from tests import test_gpu_moe_wmma as W
 from tests import test_gpu_sweep as S
 from tests.gpu_util import FP8_FLOOR, dev, host_bits16, sync
@@ -192,3 +193,10 @@ def test_gemv_dense_tall_slices(gpu, dtype, n, k, batch):
         # f32 sums of k products in chains of at most 128 + 64 + 16 additions, one output rounding
         bound = 208 * 2.0 ** -24 * mag + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * exact.abs()
         assert bool(((d[i].double() - exact).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(1, 8), (3, 2056), (256, 4096), (257, 4104), (2, 16384), (1, 16392), (300, 9000)])
+def test_quantize_row_widths(gpu, dtype, shape):
+    """Every chunk count and both workgroup sizes of the vector quantizer."""
+    G.test_quantize_per_token_bit_exact(gpu, dtype, shape)
