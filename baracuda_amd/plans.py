@@ -619,23 +619,26 @@ class MoeS8GroupedPlan:
 
 
 # ---- per-token dynamic quantization + quantized_linear ----------------------
+def _check_quantize(x, scale, q, scale_dtype) -> None:
+    _need(x.dim() == 2 and x.is_contiguous() and q.is_contiguous(), "x, q contiguous [N, D]")
+    _need(tuple(q.shape) == tuple(x.shape) and q.dtype == torch.int8, "q must be int8 [N, D]")
+    _need(scale.dim() == 1 and scale.is_contiguous() and scale.numel() == x.shape[0],
+          "scale must be a contiguous 1-D [N] vector")
+    if x.dtype in (torch.float32, torch.float64, torch.bfloat16):
+        _need(scale.dtype == scale_dtype, f"{x.dtype} input takes a {scale_dtype} scale")
+
+
 def dynamic_range_quantize_per_token_sym(x, scale, q, qmin=-127, qmax=127, stream=None) -> None:
     """DynamicRangeQuantizePlan (baracuda_quantize_compose.cuh:143-203): per row,
     scale = max|x|/qmax (1 for an all-zero row), q = clamp(rne(x/scale))."""
-    _need(x.dim() == 2 and x.is_contiguous() and q.is_contiguous(), "x, q contiguous [N, D]")
+    _check_quantize(x, scale, q, torch.float64 if x.dtype == torch.float64 else torch.float32)
     n, d = x.shape
-    _need(tuple(q.shape) == (n, d) and q.dtype == torch.int8, "q must be int8 [N, D]")
-    _need(scale.dim() == 1 and scale.is_contiguous() and scale.numel() == n,
-          "scale must be a contiguous 1-D [N] vector")
     L = lib()
     if x.dtype == torch.float32:
-        _need(scale.dtype == torch.float32, "f32 input takes an f32 scale")
         fn = L.dynamic_range_quantize_per_token_sym_f32_s8_run
     elif x.dtype == torch.float64:
-        _need(scale.dtype == torch.float64, "f64 input takes an f64 scale")
         fn = L.dynamic_range_quantize_per_token_sym_f64_s8_run
     elif x.dtype == torch.bfloat16:
-        _need(scale.dtype == torch.float32, "bf16 input takes an f32 scale")
         fn = L.dynamic_range_quantize_per_token_sym_bf16_s8_gfx950_run
     else:
         raise Unsupported(f"quantize input dtype {x.dtype}")
@@ -681,26 +684,29 @@ class QuantizedLinearPlan:
         _need(tuple(activation.shape) == (d.m, d.k) and tuple(weight_q.shape) == (d.c_out, d.k),
               "activation [M,K], weight_q [C_out,K]")
         _need(tuple(output.shape) == (d.m, d.c_out), "output [M, C_out]")
-        dynamic_range_quantize_per_token_sym(activation, act_scale_scratch, act_q_scratch,
-                                             d.q_min, d.q_max, stream)
         L, s = lib(), _stream(stream)
-        if activation.dtype == torch.float32:
-            _need(output.dtype == torch.float32 and weight_scale.dtype == torch.float32, "f32 output/scales")
-            st = L.quantized_linear_w8a8_f32_gfx950_run(d.m, d.c_out, d.k, _ptr(weight_q), _ptr(act_q_scratch),
-                                                         _ptr(act_scale_scratch), _ptr(weight_scale),
-                                                         _ptr(output), None, 0, s)
+        if activation.dtype in (torch.float32, torch.bfloat16):
+            # both passes behind one call
+            _check_quantize(activation, act_scale_scratch, act_q_scratch, torch.float32)
+            if activation.dtype == torch.float32:
+                _need(output.dtype == torch.float32 and weight_scale.dtype == torch.float32, "f32 output/scales")
+                st = L.quantized_linear_f32_gfx950_run(d.m, d.c_out, d.k, d.q_min, d.q_max, _ptr(activation),
+                                                       _ptr(weight_q), _ptr(weight_scale), _ptr(output),
+                                                       _ptr(act_q_scratch), _ptr(act_scale_scratch), s)
+            else:
+                _need(output.dtype == torch.bfloat16 and weight_scale.dtype == torch.float32, "bf16 output, f32 scales")
+                st = L.quantized_linear_bf16_gfx950_run(d.m, d.c_out, d.k, d.q_min, d.q_max, _ptr(activation),
+                                                        _ptr(weight_q), _ld(weight_q), _ptr(weight_scale), _ptr(output),
+                                                        _ld(output), _ptr(act_q_scratch), _ptr(act_scale_scratch), s)
         elif activation.dtype == torch.float64:
             # quantized_linear.rs:166-171 f64 arm: f64 activation, scales and output.
+            dynamic_range_quantize_per_token_sym(activation, act_scale_scratch, act_q_scratch,
+                                                 d.q_min, d.q_max, stream)
             _need(output.dtype == torch.float64 and weight_scale.dtype == torch.float64 and
                   act_scale_scratch.dtype == torch.float64, "f64 output / scales")
             st = L.quantized_linear_w8a8_f64_gfx950_run(d.m, d.c_out, d.k, _ptr(weight_q), _ptr(act_q_scratch),
                                                          _ptr(act_scale_scratch), _ptr(weight_scale),
                                                          _ptr(output), None, 0, s)
-        elif activation.dtype == torch.bfloat16:
-            _need(output.dtype == torch.bfloat16 and weight_scale.dtype == torch.float32, "bf16 output, f32 scales")
-            st = L.gemm_w8a8_rcr_gfx950_bf16_run(d.m, d.c_out, d.k, _ptr(act_q_scratch), d.k, _ptr(weight_q),
-                                                 _ld(weight_q), _ptr(act_scale_scratch), _ptr(weight_scale),
-                                                 _ptr(output), _ld(output), None, 0, s)
         else:
             raise Unsupported(f"quantized_linear activation dtype {activation.dtype}")
         check(st, "QuantizedLinearPlan::run")

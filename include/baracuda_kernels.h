@@ -108,6 +108,19 @@ int32_t baracuda_kernels_quantized_linear_w8a8_f64_gfx950_can_implement(
     int32_t M, int32_t C_out, int32_t K, const void *weight_q, const void *act_q,
     const void *scale_a, const void *scale_w, const void *output);
 
+/* New SKUs: both passes of quantized_linear behind one call
+ * (crates/baracuda-kernels/src/quantize/quantized_linear.rs:262-356): act_q [M,K] and
+ * act_scale [M] f32 receive the per-token codes and scales
+ * (dynamic_range_quantize_per_token_sym with q_min / q_max), output [M,C_out] the
+ * dequantized product with weight_q [C_out,K].  bf16: activation and output bf16,
+ * weight and output row pitches in elements; f32: contiguous. */
+int32_t baracuda_kernels_quantized_linear_bf16_gfx950_run(
+    int32_t M, int32_t C_out, int32_t K, int32_t q_min, int32_t q_max, const void *act, const void *weight_q,
+    int64_t ldw, const void *scale_w, void *output, int64_t ldd, void *act_q, void *act_scale, void *stream);
+int32_t baracuda_kernels_quantized_linear_f32_gfx950_run(
+    int32_t M, int32_t C_out, int32_t K, int32_t q_min, int32_t q_max, const void *act, const void *weight_q,
+    const void *scale_w, void *output, void *act_q, void *act_scale, void *stream);
+
 /* int8 RCR with the bias / activation epilogue family.  Same ABI as
  * baracuda_kernels_gemm_{bias,bias_relu,bias_gelu,bias_silu}_{f32bias,i32bias}_s8_rcr_sm80_*
  * (crates/baracuda-cutlass-kernels-sys/kernels/gemm_s8_rcr_sm80_bias.cu:225-275,
