@@ -250,7 +250,7 @@ __global__ __launch_bounds__(F8DmaCfg::NT, 1) void gemm_fp8_dma_kernel(F8Args p)
     } else {
         M2::DmaRowsRrr d;
         d.a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-        d.b = M2::make_dma_row_b<C>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base);
+        d.b = M2::make_dma_row_b<C>(p.b, (uint32_t)M2::row_b_bytes(p.K, p.N, p.ldb), (int)p.ldb, n_base);
         M2::mainloop<P>(stage0, stage1, d, p.K, acc);
     }
     f8_store_tile<FMT, EPI, ACT, P>(acc, M2::wave_scratch<C>(stage0, stage1), p, m_base, n_base);
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_ring_ker
     M2::AccTile<P> acc;
     const auto a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
     if constexpr (LAYOUT == F8_RRR) {
-        const M2::DmaRowsRrr d{a, M2::make_dma_row_b<C>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base)};
+        const M2::DmaRowsRrr d{a, M2::make_dma_row_b<C>(p.b, (uint32_t)M2::row_b_bytes(p.K, p.N, p.ldb), (int)p.ldb, n_base)};
         M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
     } else {
         const M2::DmaRows<false, false> d{
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
     const int n0 = cgroup * 16 * NB;
     mfma2::RowsDma<16 * RF, 16 * NB, SB, RowB> dma;
     dma.init(mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda)),
-             mfma2::make_rsrc(p.b, (uint32_t)(RowB ? (int64_t)p.K * p.ldb : (int64_t)p.N * p.ldb)),
+             mfma2::make_rsrc(p.b, (uint32_t)(RowB ? mfma2::row_b_bytes(p.K, p.N, p.ldb) : (int64_t)p.N * p.ldb)),
              [&](int r) { return (int)((int64_t)(m0 + r) * p.lda); }, n0, (int)p.ldb);
     constexpr int HI = dma.HI, LO = dma.LO;
     const bool hi = dma.hi();

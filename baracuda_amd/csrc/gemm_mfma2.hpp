@@ -638,6 +638,16 @@ struct DmaRowsRrr {
     DmaOperandRowB b;
 };
 
+// Bytes of a row-major B [K, N] of pitch ld from its base to the end of the
+// 16-byte unit that holds column N - 1 of row K - 1: a view of a wider tensor
+// owns no more of its last row.  Units past N of the rows before it belong to
+// the tensor; k-rows at or past K lie past these bytes.  (The range check is
+// per dword, so the last unit counts whole; bases and ld are 16-byte aligned,
+// so a unit never crosses a page.)
+__host__ __device__ constexpr int64_t row_b_bytes(int K, int N, int64_t ld) {
+    return (int64_t)(K - 1) * ld + (N + 15) / 16 * 16;
+}
+
 template <bool GA, bool GB>
 struct DmaRows {
     DmaOperand<GA> a;
@@ -674,7 +684,7 @@ __device__ __forceinline__ void mask_tail(DmaOperand<true> &d, int kbyte, int K)
     }
 }
 
-// Row-major B: k-rows at or past K lie past the extent (K * ld bytes).
+// Row-major B: k-rows at or past K lie past the extent (row_b_bytes).
 template <class C, int>
 __device__ __forceinline__ void mask_tail(DmaOperandRowB &, int, int) {}
 

@@ -507,7 +507,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_s8_ring_kern
     M2::AccTile<P> acc;
     const auto a = M2::make_dma_interior<C>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
     if constexpr (RowB) {
-        const M2::DmaRowsRrr d{a, M2::make_dma_row_b<C>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base)};
+        const M2::DmaRowsRrr d{a, M2::make_dma_row_b<C>(p.b, (uint32_t)M2::row_b_bytes(p.K, p.N, p.ldb), (int)p.ldb, n_base)};
         M2::mainloop_ring<P, DEPTH, SPREAD>(lds, d, p.K, acc);
     } else {
         const M2::DmaRows<false, false> d{
@@ -767,7 +767,7 @@ __global__ __launch_bounds__(1024) void gemm_s8_rcr_rows_staged_kernel(S8Args p,
     const int n0 = cgroup * 16 * NB;
     mfma2::RowsDma<16 * RF, 16 * NB, SB, RowB> dma;
     dma.init(mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda)),
-             mfma2::make_rsrc(p.b, (uint32_t)(RowB ? (int64_t)p.K * p.ldb : (int64_t)p.N * p.ldb)),
+             mfma2::make_rsrc(p.b, (uint32_t)(RowB ? mfma2::row_b_bytes(p.K, p.N, p.ldb) : (int64_t)p.N * p.ldb)),
              [&](int r) { return (int)((int64_t)(m0 + r) * p.lda); }, n0, (int)p.ldb);
     constexpr int HI = dma.HI, LO = dma.LO;
     const bool hi = dma.hi();
@@ -860,15 +860,15 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_s8_rrr_dma_kernel(S8Args p
     __shared__ __attribute__((aligned(1024))) int8_t stage0[2 * M2::OPER];
     __shared__ __attribute__((aligned(1024))) int8_t stage1[2 * M2::OPER];
     // Edge tiles: A rows past M load as zeros (past the buffer's byte count);
-    // B columns past N read bytes of the next k-row (or zeros after the
-    // last), which only reach output columns that are not stored.
+    // B columns past N read bytes of the next k-row (or zeros after the last
+    // row's), which only reach output columns that are not stored.
     const int tiles_m = (p.M + M2::BM - 1) / M2::BM, tiles_n = (p.N + M2::BN - 1) / M2::BN;
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m_base = tm * M2::BM, n_base = tn * M2::BN;
     M2::DmaRowsRrr d;
     d.a = M2::make_dma_interior<DmaCfg>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-    d.b = M2::make_dma_row_b<DmaCfg>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base);
+    d.b = M2::make_dma_row_b<DmaCfg>(p.b, (uint32_t)M2::row_b_bytes(p.K, p.N, p.ldb), (int)p.ldb, n_base);
     M2::AccTile<P> acc;
     M2::mainloop<P>(stage0, stage1, d, p.K, acc);
     s8_store_tile<EPI_S8, VecOut, ACT, BiasT, P>(acc, M2::wave_scratch<DmaCfg>(stage0, stage1), p, m_base, n_base);
@@ -1001,7 +1001,7 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_u8_rrr_dma_kernel(S8Args p
     const int m_base = tm * M2::BM, n_base = tn * M2::BN;
     M2::DmaRowsRrr d;
     d.a = M2::make_dma_interior<DmaCfg>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-    d.b = M2::make_dma_row_b<DmaCfg>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base);
+    d.b = M2::make_dma_row_b<DmaCfg>(p.b, (uint32_t)M2::row_b_bytes(p.K, p.N, p.ldb), (int)p.ldb, n_base);
     M2::AccTile<P> acc;
     typename P::Sums sums;
     sums.ra = 0;
@@ -1116,7 +1116,7 @@ __global__ __launch_bounds__(DmaCfg::NT, 1) void gemm_u8_rrr_ws_kernel(S8Args p,
     const int m_base = tm * M2::BM, n_base = tn * M2::BN;
     M2::DmaRowsRrr d;
     d.a = M2::make_dma_interior<DmaCfg>(p.a, (uint32_t)(p.M * p.lda), (int)p.lda, m_base * (int)p.lda);
-    d.b = M2::make_dma_row_b<DmaCfg>(p.b, (uint32_t)(p.K * p.ldb), (int)p.ldb, n_base);
+    d.b = M2::make_dma_row_b<DmaCfg>(p.b, (uint32_t)M2::row_b_bytes(p.K, p.N, p.ldb), (int)p.ldb, n_base);
     M2::AccTile<P> acc;
     M2::mainloop<P>(stage0, stage1, d, p.K, acc);
     // The tile's 256 row and 256 column sums into LDS (free after the loop),

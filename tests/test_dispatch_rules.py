@@ -1,0 +1,51 @@
+"""Extents and selection rules of the GEMM launchers, as host functions.
+
+The rules are inline functions of the kernel headers; a small library of
+C entry points is compiled from them for the host only, so no GPU is needed.
+"""
+import ctypes
+import subprocess
+
+import numpy as np
+import pytest
+
+from baracuda_amd import build as B
+
+SOURCE = r"""
+#include "gemm_ring.hpp"
+using namespace bk;
+extern "C" {
+int64_t row_b_bytes(int K, int N, int64_t ld) { return mfma2::row_b_bytes(K, N, ld); }
+}
+"""
+
+
+@pytest.fixture(scope="session")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.hip").write_text(SOURCE)
+    cmd = [B.HIPCC, *B.HIP_FLAGS, "--offload-host-only", "-w", "-shared", str(d / "rules.hip"), "-o", str(d / "rules.so")]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    lib = ctypes.CDLL(str(d / "rules.so"))
+    lib.row_b_bytes.restype = ctypes.c_int64
+    lib.row_b_bytes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64]
+    return lib
+
+
+@pytest.mark.parametrize("k,n,ld", [(1, 16, 16), (16, 250, 256), (48, 262, 272), (208, 520, 1040), (144, 4100, 4608),
+                                    (336, 1000, 1008), (512, 256, 256), (400, 2064, 14336)])
+def test_row_major_b_extent(rules, k, n, ld):
+    """Every 16-byte unit of a 256-column tile that the extent admits holds a
+    byte of the view (the last row owns n bytes, the others the pitch), and
+    the units of the k-rows past the last one are not admitted."""
+    extent = rules.row_b_bytes(k, n, ld)
+    own = (k - 1) * ld + n                      # bytes of the strided view
+    assert own <= extent < own + 16 and extent % 16 == 0
+    rows = np.arange((k + 127) // 128 * 128 + 128)[:, None]
+    units = np.arange(0, (n + 255) // 256 * 256, 16)[None, :]
+    off = rows * ld + units
+    admitted = off < extent
+    assert not admitted[k:].any()
+    assert (off[admitted] < own).all()
+    assert admitted[:k, : (n + 15) // 16].all()

@@ -137,6 +137,59 @@ def test_rrr_and_u8_depth_tails(gpu, shape):
     S.test_u8_rrr_sweep(gpu, shape, False)
 
 
+@pytest.mark.parametrize("shape", [(300, 520, 208), (900, 2072, 400), (1500, 3000, 336), (700, 4100, 1040), (13, 6160, 304),
+                                   (100, 272, 656), (40, 8200, 144)])
+@pytest.mark.parametrize("kind", ["s8", "u8", "e4m3", "e5m2"])
+def test_rrr_padded_pitch(gpu, shape, kind):
+    """B as the last columns of a wider tensor with more k-rows behind it: what
+    surrounds the view (127, 255, NaN codes) stays out of the result, which is
+    that of a dense copy on the same kernel, bit for bit."""
+    m, n, k = shape
+    print(f"case: rrr padded pitch {kind} {shape}", flush=True)
+    g = torch.Generator()
+    g.manual_seed(m + n + k)
+    E = P.ElementKind
+    el, fill, code = {"s8": (E.S8, 0x7f, torch.int8), "u8": (E.U8, 0xff, torch.uint8),
+                      "e4m3": (E.Fp8E4M3, 0x7f, torch.float8_e4m3fn), "e5m2": (E.Fp8E5M2, 0x7e, torch.float8_e5m2)}[kind]
+    lead = 48
+    wide = torch.full((k + 128, lead + (n + 15) // 16 * 16), fill, dtype=torch.uint8)
+    # finite FP8 codes below 2 in magnitude
+    wide[:k, lead:lead + n] = torch.randint(0, 256, (k, n), dtype=torch.uint8, generator=g) & (0xff if kind[1] == "8" else 0xbf)
+    wide = wide.to("cuda:0").view(code)
+    a = torch.randint(0, 256, (m, k), dtype=torch.uint8, generator=g) & (0xff if kind[1] == "8" else 0xbf)
+    a = a.to("cuda:0").view(code)
+    if kind[1] == "8":
+        plan = P.IntGemmPlan.select(P.IntGemmDescriptor(m, n, k, layout=P.LayoutSku.Rrr, element=el, output=el))
+        alpha = 2e-4 if kind == "s8" else 1.0 / (128.0 * k)
+    else:
+        plan = P.Fp8GemmPlan.select(P.Fp8GemmDescriptor(m, n, k, layout=P.LayoutSku.Rrr, element=el, output=el))
+        alpha = 0.25
+    ldd = (n + 15) // 16 * 16
+
+    def run(b):
+        d = torch.zeros((m, ldd), dtype=torch.uint8, device="cuda:0").view(code)
+        plan.run(a, b, d[:, :n], alpha=alpha)
+        sync()
+        return d.view(torch.uint8).cpu()
+
+    view = wide[:k, lead:lead + n]
+    dense = torch.zeros((k, ldd), dtype=torch.uint8, device="cuda:0").view(code)[:, :n]   # pitch a multiple of 16
+    dense.view(torch.uint8).copy_(view.view(torch.uint8))
+    got = run(view)
+    assert torch.equal(got, run(dense))
+    if kind[1] != "8":
+        assert not bool(got.view(code).float().isnan().any())
+        exact = alpha * (a.double().cpu() @ view.double().cpu())
+        big = exact.abs() > 1.0
+        err = (got.view(code)[:, :n].double() - exact).abs()
+        step = 2.0 ** -3 if kind == "e4m3" else 2.0 ** -2      # spacing of the format, relative
+        assert bool((err[big] <= step * exact.abs()[big]).all())
+    else:
+        exact = alpha * (a.double().cpu() @ view.double().cpu())
+        lo, hi = (-128, 127) if kind == "s8" else (0, 255)
+        assert bool(((got.view(code)[:, :n].double() - exact.clamp(lo, hi)).abs() <= 0.51).all())
+
+
 # experts' row counts (ends of 64- and 128-row tiles, empty experts, more than
 # 64 experts), N and K in bytes off 256 / 128
 MOE_CASES = [([64, 1, 0, 129, 65, 300], 328, 208), ([3] * 70 + [0] * 30 + [200] * 3, 136, 80),
