@@ -22,8 +22,14 @@ using namespace bk;
 
 namespace {
 
-int32_t check_linear(int32_t M, int32_t C_out, int32_t K, int32_t qmin, int32_t qmax) {
-    return M < 0 || C_out < 0 || K < 0 || qmin > qmax || qmax <= 0 ? kInvalid : kOk;
+// Extents, q range and pointers of both passes, before the first launch.
+int32_t check_linear(int32_t M, int32_t C_out, int32_t K, int32_t qmin, int32_t qmax, const void *act,
+                     const void *weight_q, const void *scale_w, const void *output, const void *act_q,
+                     const void *act_scale) {
+    if (M < 0 || C_out < 0 || K < 0 || qmin > qmax || qmax <= 0) return kInvalid;
+    if ((int64_t)M * K != 0 && (!act || !act_q || !act_scale)) return kInvalid;
+    if ((int64_t)M * C_out != 0 && (!weight_q || !scale_w || !output || !act_q || !act_scale)) return kInvalid;
+    return kOk;
 }
 
 }  // namespace
@@ -166,16 +172,19 @@ int32_t baracuda_kernels_quantized_linear_w8a8_f64_gfx950_run(
 // Per-token quantization of `act` into act_q / act_scale, then the W8A8 GEMM:
 // the two launches of QuantizedLinearPlan (quantized_linear.rs:262-356) from one
 // call, which is what a caller's binding pays for at small sizes (through ctypes
-// 16 x 4096 x 4096 18.0 -> 14.7 us).
+// 16 x 4096 x 4096 18.0 -> 14.7 us).  Status and results are those of the two
+// calls, except that nothing is launched when the second would be refused and
+// that an empty output is no error.
 int32_t baracuda_kernels_quantized_linear_bf16_gfx950_run(
     int32_t M, int32_t C_out, int32_t K, int32_t qmin, int32_t qmax, const void *act, const void *weight_q, int64_t ldw,
     const void *scale_w, void *output, int64_t ldd, void *act_q, void *act_scale, void *stream) {
-    const int32_t st = check_linear(M, C_out, K, qmin, qmax);
-    if (st != kOk || (int64_t)M * C_out == 0 || K == 0) return st;
-    if (!act || !weight_q || !scale_w || !output || !act_q || !act_scale) return kInvalid;
-    const int32_t q = baracuda_kernels_dynamic_range_quantize_per_token_sym_bf16_s8_gfx950_run(
-        M, K, qmin, qmax, act, act_scale, act_q, nullptr, 0, stream);
-    if (q != kOk) return q;
+    int32_t st = check_linear(M, C_out, K, qmin, qmax, act, weight_q, scale_w, output, act_q, act_scale);
+    const bool product = (int64_t)M * C_out != 0;
+    if (st == kOk && product) st = check_rcr(M, C_out, K, K, ldw, ldd);
+    if (st != kOk) return st;
+    st = baracuda_kernels_dynamic_range_quantize_per_token_sym_bf16_s8_gfx950_run(M, K, qmin, qmax, act, act_scale, act_q,
+                                                                                 nullptr, 0, stream);
+    if (st != kOk || !product) return st;
     return baracuda_kernels_gemm_w8a8_rcr_gfx950_bf16_run(M, C_out, K, act_q, K, weight_q, ldw, (const float *)act_scale,
                                                           (const float *)scale_w, output, ldd, nullptr, 0, stream);
 }
@@ -183,12 +192,11 @@ int32_t baracuda_kernels_quantized_linear_bf16_gfx950_run(
 int32_t baracuda_kernels_quantized_linear_f32_gfx950_run(
     int32_t M, int32_t C_out, int32_t K, int32_t qmin, int32_t qmax, const void *act, const void *weight_q,
     const void *scale_w, void *output, void *act_q, void *act_scale, void *stream) {
-    const int32_t st = check_linear(M, C_out, K, qmin, qmax);
-    if (st != kOk || (int64_t)M * C_out == 0 || K == 0) return st;
-    if (!act || !weight_q || !scale_w || !output || !act_q || !act_scale) return kInvalid;
-    const int32_t q = baracuda_kernels_dynamic_range_quantize_per_token_sym_f32_s8_run(M, K, qmin, qmax, act, act_scale,
-                                                                                      act_q, nullptr, 0, stream);
-    if (q != kOk) return q;
+    int32_t st = check_linear(M, C_out, K, qmin, qmax, act, weight_q, scale_w, output, act_q, act_scale);
+    if (st != kOk) return st;
+    st = baracuda_kernels_dynamic_range_quantize_per_token_sym_f32_s8_run(M, K, qmin, qmax, act, act_scale, act_q, nullptr,
+                                                                          0, stream);
+    if (st != kOk) return st;
     return baracuda_kernels_quantized_linear_w8a8_f32_gfx950_run(M, C_out, K, weight_q, act_q, act_scale, scale_w, output,
                                                                  nullptr, 0, stream);
 }

@@ -113,7 +113,10 @@ int32_t baracuda_kernels_quantized_linear_w8a8_f64_gfx950_can_implement(
  * act_scale [M] f32 receive the per-token codes and scales
  * (dynamic_range_quantize_per_token_sym with q_min / q_max), output [M,C_out] the
  * dequantized product with weight_q [C_out,K].  bf16: activation and output bf16,
- * weight and output row pitches in elements; f32: contiguous. */
+ * weight and output row pitches in elements; f32: contiguous.  Nothing is launched
+ * when either pass would refuse its arguments.  An empty output is no error; K = 0
+ * is as in the single passes: f32 writes the empty sums (act_scale is read as
+ * given), bf16 returns 2. */
 int32_t baracuda_kernels_quantized_linear_bf16_gfx950_run(
     int32_t M, int32_t C_out, int32_t K, int32_t q_min, int32_t q_max, const void *act, const void *weight_q,
     int64_t ldw, const void *scale_w, void *output, int64_t ldd, void *act_q, void *act_scale, void *stream);

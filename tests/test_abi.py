@@ -119,6 +119,21 @@ def test_gemm_invalid_problems_rejected_before_launch():
 
 
 
+def test_quantized_linear_one_call_arguments():
+    """Refused before the first launch (which would report 5 without a GPU)."""
+    L, x = ffi.lib(), 4096      # a pointer that is never followed
+    bf16 = lambda m, n, k, ldw, ldd, qmin=-127, qmax=127, act=x: L.quantized_linear_bf16_gfx950_run(
+        m, n, k, qmin, qmax, act, x, ldw, x, x, ldd, x, x, None)
+    f32 = lambda m, n, k, qmin=-127, qmax=127, act=x: L.quantized_linear_f32_gfx950_run(
+        m, n, k, qmin, qmax, act, x, x, x, x, x, None)
+    assert bf16(2, 4, 16, 15, 4) == 2 and bf16(2, 4, 16, 16, 3) == 2       # pitches below the rows
+    assert bf16(2, 4, 0, 16, 4) == 2                                       # the bf16 GEMM refuses K = 0
+    for f in (lambda *a, **k: bf16(*a, 16, 16, **k), f32):
+        assert f(-1, 4, 16) == f(2, -4, 16) == f(2, 4, -16) == 2
+        assert f(2, 4, 16, qmax=0) == f(2, 4, 16, qmin=5, qmax=4) == f(2, 4, 16, act=None) == 2
+        assert f(0, 4, 16) == f(0, 0, 0) == 0
+
+
 def test_rrr_and_bias_can_implement():
     # gemm_s8_rrr_sm80.cu:44-52: positive extents, lda >= K, ldb >= N, ldd >= N.
     L = ffi.lib()

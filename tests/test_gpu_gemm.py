@@ -630,6 +630,34 @@ def test_quantized_linear_plan_two_pass(gpu, dtype):
         assert np.array_equal(host_bits16(out), O.f32_to_bf16_bits_fast(want))
 
 
+@pytest.mark.parametrize("shape", [(3, 5, 0), (3, 0, 64), (5, 48, 64)])
+def test_quantized_linear_f32_one_call(gpu, shape):
+    """The one-call entry does what its two passes do, also where K or C_out is empty."""
+    m, c_out, k = shape
+    print(f"case: quantized_linear one call {shape}", flush=True)
+    g = rng(31)
+    x, w = dev(g.standard_normal((m, max(k, 1))).astype(np.float32)), dev(int8_uniform(g, (max(c_out, 1), max(k, 1))))
+    sw = dev(g.uniform(0.001, 0.01, max(c_out, 1)).astype(np.float32))
+    L, s = lib(), torch.cuda.current_stream().cuda_stream
+    res = []
+    for one in (True, False):
+        q = torch.full((m, max(k, 1)), 55, dtype=torch.int8, device="cuda:0")
+        sa = torch.full((m,), 0.5, dtype=torch.float32, device="cuda:0")
+        out = torch.full((m, max(c_out, 1)), 7.0, dtype=torch.float32, device="cuda:0")
+        p = [t.data_ptr() for t in (x, w, sw, out, q, sa)]
+        if one:
+            assert L.quantized_linear_f32_gfx950_run(m, c_out, k, -127, 127, *p, s) == 0
+        else:
+            assert L.dynamic_range_quantize_per_token_sym_f32_s8_run(m, k, -127, 127, p[0], p[5], p[4], None, 0, s) == 0
+            assert L.quantized_linear_w8a8_f32_gfx950_run(m, c_out, k, p[1], p[4], p[5], p[2], p[3], None, 0, s) == 0
+        sync()
+        res.append([t.cpu() for t in (q, sa, out)])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+    if k == 0:
+        assert not bool(res[0][2].any())
+
+
 def test_i32_operand_beyond_2gib(gpu):
     # A is 16384 x 131200 int8 (2.0 GiB): past the 32-bit buffer offsets of
     # the LDS-DMA path, so the general kernel (64-bit row addressing) runs.
