@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from baracuda_amd import plans as P
+from baracuda_amd.ffi import lib
 from oracle import oracle as O
 from oracle.inputs import int8_uniform, rng, w8a8
 from tests.gpu_util import FP8_FLOOR, FP8_FLOOR_CONFIG3, bf16_ulp, dev, host_bits16, sync
