@@ -382,7 +382,8 @@ __device__ __forceinline__ void moe_store_tile(const mfma2::AccTile<P> &acc, int
             M2::store_bf16x4_staged<P>(
                 acc, scratch,
                 [&](int r, int, const v4f &v) {
-                    const float tw = p.topk_w ? p.topk_w[rows_tok[wr + r]] : 1.0f;
+                    // (padding rows are packed too: no index of theirs is followed)
+                    const float tw = p.topk_w ? p.topk_w[rows_tok[min(wr + r, seg_rows - 1)]] : 1.0f;
                     uint16_t h[4];
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {

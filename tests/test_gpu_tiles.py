@@ -220,6 +220,21 @@ def test_moe_float_tiles_and_depth_tails(gpu, shape, t, weighted):
     W._check(*W._run(t, x, w, sid, eid, topk, tw, rows), t)
 
 
+@pytest.mark.parametrize("t", ["bf16", "f16"])
+@pytest.mark.parametrize("counts,n,k", [([65, 1, 0, 130], 264, 136), ([33] * 12, 1408, 336), ([100, 300], 2312, 264)])
+def test_moe_float_weights_of_padding_rows(gpu, counts, n, k, t):
+    """Weighted pairs on tiles that end in padding rows: the weights are the
+    first elements of the operand and the ids of a padding row have no weight."""
+    print(f"case: moe {t} weighted, rows={counts[:4]} n={n} k={k}", flush=True)
+    g = rng(n + k)
+    rows = sum(counts)
+    sid = g.permutation(rows).astype(np.int32)
+    eid = np.repeat(np.arange(len(counts), dtype=np.int32), counts)
+    x = g.standard_normal((rows, k)).astype(np.float32)
+    w = (g.standard_normal((len(counts), n, k)) / np.sqrt(k)).astype(np.float32)
+    W._check(*W._run(t, x, w, sid, eid, 1, g.uniform(0.1, 1.0, rows).astype(np.float32), rows), t)
+
+
 @pytest.mark.parametrize("shape", [(1, 16), (5, 1040), (4097, 4672), (300, 3072), (130, 8176), (64, 11008), (7, 4080)])
 def test_gemv_s8w_depth_tails(gpu, shape):
     print(f"case: gemv_s8w depth tail {shape}", flush=True)
