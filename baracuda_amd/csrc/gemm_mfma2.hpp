@@ -454,6 +454,18 @@ struct DmaOperand<true> {
     int off[8];         // DMA_PER_WAVE used
 };
 
+// Rows of an operand rounded up to 256, times its row pitch, fit the 32-bit
+// buffer offsets of the LDS-DMA path.
+inline bool dma_extent_ok(int rows, int64_t ld) {
+    return ((int64_t)(rows + 255) / 256) * 256 * ld < (1ll << 31);
+}
+
+// Byte offset of row `row` of an operand of pitch ld, unsigned: rows past the
+// operand's end in 192-row tiles and 96- or 112-column groups can pass 2^31 where
+// dma_extent_ok holds (up to 191 of them against the 255 of its rounding), not
+// 2^32, and lie past the extent either way.
+__host__ __device__ constexpr int row_offset(int row, int64_t ld) { return (int)((uint32_t)row * (uint32_t)ld); }
+
 // Interior operand: tile rows r0 .. r0+255 of a row-major operand with
 // leading dimension ld (bytes), starting at byte `tile_off` of the buffer.
 template <class C, int ROWS_PER_WAVE = C::ROWS_PER_WAVE>
@@ -465,8 +477,9 @@ __device__ __forceinline__ DmaOperand<false> make_dma_interior(const int8_t *bas
     d.row_stride = 8 * ld;
     const int r0 = wave * ROWS_PER_WAVE + (lane >> 3);
     const int u0 = (lane & 7) ^ swz(r0);
-    d.even = tile_off + r0 * ld + u0 * 16;
-    d.odd = tile_off + r0 * ld + (u0 ^ 4) * 16;
+    const uint32_t off = (uint32_t)tile_off + (uint32_t)row_offset(r0, ld);
+    d.even = (int)(off + u0 * 16);
+    d.odd = (int)(off + (u0 ^ 4) * 16);
     return d;
 }
 

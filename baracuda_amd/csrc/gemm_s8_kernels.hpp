@@ -263,11 +263,7 @@ inline size_t tail_split_workspace(int M, int N, int K) {
     return t.split > 1 ? (size_t)t.tail_tiles * t.split * 65536u * sizeof(int32_t) : 0;
 }
 
-// Rows of an operand padded to whole 256-row tiles, times its row pitch,
-// fit the 32-bit buffer offsets of the LDS-DMA path.
-inline bool dma_extent_ok(int rows, int64_t ld) {
-    return ((int64_t)(rows + 255) / 256) * 256 * ld < (1ll << 31);
-}
+using mfma2::dma_extent_ok;
 
 // Fast path: 256x256 tiles (edge tiles read zeros past M / N), K % 128 == 0,
 // 16-byte aligned rows ->

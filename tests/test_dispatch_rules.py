@@ -16,6 +16,8 @@ SOURCE = r"""
 using namespace bk;
 extern "C" {
 int64_t row_b_bytes(int K, int N, int64_t ld) { return mfma2::row_b_bytes(K, N, ld); }
+int dma_extent_ok(int rows, int64_t ld) { return mfma2::dma_extent_ok(rows, ld); }
+unsigned row_offset(int row, int64_t ld) { return (unsigned)mfma2::row_offset(row, ld); }
 }
 """
 
@@ -30,6 +32,9 @@ def rules(tmp_path_factory):
     lib = ctypes.CDLL(str(d / "rules.so"))
     lib.row_b_bytes.restype = ctypes.c_int64
     lib.row_b_bytes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64]
+    lib.dma_extent_ok.argtypes = [ctypes.c_int, ctypes.c_int64]
+    lib.row_offset.restype = ctypes.c_uint32
+    lib.row_offset.argtypes = [ctypes.c_int, ctypes.c_int64]
     return lib
 
 
@@ -49,3 +54,15 @@ def test_row_major_b_extent(rules, k, n, ld):
     assert not admitted[k:].any()
     assert (off[admitted] < own).all()
     assert admitted[:k, : (n + 15) // 16].all()
+
+
+@pytest.mark.parametrize("rows", [1, 64, 200, 256, 257, 600, 12000])
+def test_row_offsets_of_padded_tiles(rules, rows):
+    """The offsets of every tile height and column group stay exact in 32 bits,
+    the rows past the operand's end included, for the widest pitch accepted."""
+    ld = (2 ** 31 - 1) // (-(-rows // 256) * 256) // 16 * 16
+    assert rules.dma_extent_ok(rows, ld) and not rules.dma_extent_ok(rows, 2 * ld)
+    for edge in (16, 32, 48, 64, 96, 112, 128, 192, 256):
+        last = -(-rows // edge) * edge - 1
+        assert rules.row_offset(last, ld) == last * ld < 2 ** 32 - ld
+        assert rules.row_offset(rows, ld) >= rows * ld      # past the extent
