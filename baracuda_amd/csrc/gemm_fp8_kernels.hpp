@@ -340,13 +340,14 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
     const int cgroup = RowB && gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
     const int n0 = cgroup * 16 * NB;
     mfma2::RowsDma<16 * RF, 16 * NB, SB, RowB> dma;
-    dma.init(mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda)),
-             mfma2::make_rsrc(p.b, (uint32_t)(RowB ? mfma2::row_b_bytes(p.K, p.N, p.ldb) : (int64_t)p.N * p.ldb)),
-             [&](int r) { return (int)((int64_t)(m0 + r) * p.lda); }, n0, (int)p.ldb);
+    auto a_off = [&](int r) { return mfma2::row_offset(m0 + r, p.lda); };
+    const int ns = (p.K + SB - 1) / SB;
+    dma.start(mfma2::make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda)),
+              mfma2::make_rsrc(p.b, (uint32_t)(RowB ? mfma2::row_b_bytes(p.K, p.N, p.ldb) : (int64_t)p.N * p.ldb)), a_off, n0,
+              (int)p.ldb, p.K, lds);
     constexpr int HI = dma.HI, LO = dma.LO;
     const bool hi = dma.hi();
-    const int ns = (p.K + SB - 1) / SB;
-    for (int st = 0; st < DEPTH && st < ns; ++st) dma.issue(st, p.K, lds + st * STAGE);
+    for (int st = 1; st < DEPTH && st < ns; ++st) dma.issue(st, p.K, lds + st * STAGE, a_off);
     const int c = wave % CH, f0 = wave / CH;
     const bool active = ALL || wave < RF * CH;   // wave-uniform
     v4f acc[FPW][NB];
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(1024) void gemm_fp8_rcr_rows_staged_kernel(F8Args p
         }
         }
         __syncthreads();   // every wave is done with this buffer
-        if (st + DEPTH < ns) dma.issue(st + DEPTH, p.K, buf);
+        if (st + DEPTH < ns) dma.issue(st + DEPTH, p.K, buf, a_off);
     }
     // partial sums of (A fragment f, B fragment nb), chunk c: part[f][nb][c][lane]
     v4f *part = reinterpret_cast<v4f *>(lds);

@@ -712,11 +712,18 @@ inline bool row_b_extent_ok(int K, int64_t ldb, int stage) {
 // RB B rows (RowB: SB k-rows of RB columns), by 16 waves.  Instruction j of a
 // stage moves units 64 j .. 64 j + 63 of the row-major stage image, lane L
 // fetching unit (64 j + L) % UPR of row (64 j + L) / UPR at slot unit ^ (row &
-// 15); wave w issues j = w, w + 16, ...  The per-lane offsets are computed
-// once and the K position travels in the scalar offset (recomputed per stage
-// behind branches, 100 x 4096 x 14336 e4m3 took 21.5 us against 19.8 now).
-// Units at or past K in a partial last stage go past the extent and land as
-// zeros.
+// 15); wave w issues j = w, w + 16, ...  Units at or past K in a partial last
+// stage go past the extent and land as zeros.  a_off(row): byte offset of A row
+// `row` of the stage.
+//
+// B [N, K]: the per-lane offsets are computed once and the K position travels
+// in the scalar offset (recomputed per stage behind branches, 100 x 4096 x 14336
+// e4m3 took 21.5 us against 19.8 now); start() issues each instruction of stage
+// 0 as soon as its offset is known (all offsets first cost 40 x 1024 x 1024 e4m3
+// 3.23 -> 3.41 us).  Row-major B: computed per stage.  Its workgroups share
+// 128-byte lines of B through their XCD's L2, and issued faster, from kept
+// offsets, the waves of a stage find fewer of them there (u8 2 x 6144 x 13824
+// 45.8 -> 52 us, e4m3 256 x 6144 x 13824 83.7 -> 94).
 template <int RA, int RB, int SB, bool RowB>
 struct RowsDma {
     static constexpr int WAVES = 16, UPR = SB / 16;
@@ -725,48 +732,76 @@ struct RowsDma {
     static_assert(RA * UPR % 64 == 0 && RB * UPR % 64 == 0, "whole instructions per operand");
     v4i ra, rb;
     int voff[HI];
-    int wave, lane, ldb;
+    int wave, lane, n0, ldb;
 
-    // a_off(row): byte offset of A row `row` of the stage
+    // stage 0 into buf
     template <class AOff>
-    __device__ __forceinline__ void init(const v4i &ra_, const v4i &rb_, AOff &&a_off, int n0, int ldb_) {
+    __device__ __forceinline__ void start(const v4i &ra_, const v4i &rb_, AOff &&a_off, int n0_, int ldb_, int K, int8_t *buf) {
         ra = ra_;
         rb = rb_;
+        n0 = n0_;
         ldb = ldb_;
         lane = threadIdx.x & 63;
         wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if constexpr (RowB) {
+            issue(0, K, buf, a_off);
+        } else {
 #pragma unroll
-        for (int i = 0; i < HI; ++i) {
-            const int idx = 64 * (wave + WAVES * i) + lane;
-            const int r = idx / UPR, unit = (idx % UPR) ^ (r & 15);
-            if (wave + WAVES * i < NA) {
-                voff[i] = a_off(r) + 16 * unit;
-            } else if constexpr (RowB) {
-                const int ib = idx - RA * UPR;   // unit of the B region: k-row ib / (RB / 16)
-                voff[i] = (ib / (RB / 16)) * ldb + n0 + 16 * (ib % (RB / 16));
-            } else {
-                voff[i] = (n0 + r - RA) * ldb + 16 * unit;
+            for (int i = 0; i < HI; ++i) {
+                const int j = wave + WAVES * i;
+                voff[i] = 0;
+                if (WAVES * (i + 1) > NI && j >= NI) break;
+                const int idx = 64 * j + lane, r = idx / UPR, unit = (idx % UPR) ^ (r & 15);
+                if (j < NA) {
+                    voff[i] = 16 * unit < K ? a_off(r) + 16 * unit : kPastExtent;
+                    dma16(ra, voff[i], 0, buf + j * 1024);
+                } else {
+                    voff[i] = 16 * unit < K ? row_offset(n0 + r - RA, ldb) + 16 * unit : kPastExtent;
+                    dma16(rb, voff[i], 0, buf + j * 1024);
+                }
             }
         }
     }
-    // this wave's instructions of stage st
-    __device__ __forceinline__ void issue(int st, int K, int8_t *buf) {
+    // stage st into buf
+    template <class AOff>
+    __device__ __forceinline__ void issue(int st, int K, int8_t *buf, AOff &&a_off) {
         const int k0 = st * SB;
-        if (k0 + SB > K) {
+        if constexpr (RowB) {
+            const int kb = __builtin_amdgcn_readfirstlane(k0 * ldb);   // k-rows past K lie past the extent
+            for (int j = wave; j < NI; j += WAVES) {
+                const uint32_t idx = 64 * j + lane;
+                if (j < NA) {
+                    const int r = idx / UPR, unit = (idx % UPR) ^ (r & 15);
+                    int off = a_off(r) + 16 * unit;
+                    if (k0 + SB > K) {
+                        asm volatile("" : "+v"(off));   // a branch, as below
+                        if (k0 + 16 * unit >= K) off = kPastExtent;
+                    }
+                    dma16(ra, off, k0, buf + j * 1024);
+                } else {
+                    const uint32_t ib = idx - RA * UPR;   // unit of the B region: k-row ib / (RB / 16)
+                    dma16(rb, (int)(ib / (RB / 16)) * ldb + n0 + 16 * (int)(ib % (RB / 16)), kb, buf + j * 1024);
+                }
+            }
+        } else {
+            if (k0 + SB > K) {
+                // (the empty asm keeps this a branch: as selects on every stage
+                // it took 16 x 512 x 13824 int8 from 10.7 to 12.3 us)
+#pragma unroll
+                for (int i = 0; i < HI; ++i) {
+                    const int idx = 64 * (wave + WAVES * i) + lane;
+                    const int unit = (idx % UPR) ^ ((idx / UPR) & 15);
+                    asm volatile("" : "+v"(voff[i]));
+                    if (k0 + 16 * unit >= K) voff[i] = kPastExtent;
+                }
+            }
 #pragma unroll
             for (int i = 0; i < HI; ++i) {
-                const int idx = 64 * (wave + WAVES * i) + lane;
-                const int unit = (idx % UPR) ^ ((idx / UPR) & 15);
-                if ((!RowB || wave + WAVES * i < NA) && k0 + 16 * unit >= K) voff[i] = kPastExtent;
+                const int j = wave + WAVES * i;
+                if (WAVES * (i + 1) > NI && j >= NI) break;
+                if (j < NA) dma16(ra, voff[i], k0, buf + j * 1024);
+                else dma16(rb, voff[i], k0, buf + j * 1024);
             }
-        }
-        const int kb = __builtin_amdgcn_readfirstlane(RowB ? k0 * ldb : k0);
-#pragma unroll
-        for (int i = 0; i < HI; ++i) {
-            const int j = wave + WAVES * i;
-            if (WAVES * (i + 1) > NI && j >= NI) break;
-            if (j < NA) dma16(ra, voff[i], k0, buf + j * 1024);
-            else dma16(rb, voff[i], kb, buf + j * 1024);
         }
     }
     // this wave issues HI instructions per stage, or LO

@@ -625,17 +625,16 @@ __global__ __launch_bounds__(1024) void moe_rows_staged_kernel(MoeArgs p) {
     for (int r = threadIdx.x; r < 16 * RF; r += blockDim.x) s_tok[r] = r < rows ? p.sorted_ids[o0 + r] : -1;
     __syncthreads();
     mfma2::RowsDma<16 * RF, 16 * NB, SB, false> dma;
-    dma.init(mfma2::make_rsrc(p.x, (uint32_t)((int64_t)x_rows * kb)),
-             mfma2::make_rsrc(p.w + (int64_t)e * p.N * kb, (uint32_t)((int64_t)p.N * kb)),
-             [&](int r) {
-                 const int tok = s_tok[r];
-                 return tok >= 0 ? (tok / in_div) * kb : x_rows * kb;   // past the input: zeros
-             },
-             n0, kb);
+    auto a_off = [&](int r) {
+        const int tok = s_tok[r];
+        return tok >= 0 ? (tok / in_div) * kb : x_rows * kb;   // past the input: zeros
+    };
+    const int ns = (kb + SB - 1) / SB;
+    dma.start(mfma2::make_rsrc(p.x, (uint32_t)((int64_t)x_rows * kb)),
+              mfma2::make_rsrc(p.w + (int64_t)e * p.N * kb, (uint32_t)((int64_t)p.N * kb)), a_off, n0, kb, kb, lds);
     constexpr int HI = dma.HI, LO = dma.LO;
     const bool hi = dma.hi();
-    const int ns = (kb + SB - 1) / SB;
-    for (int st = 0; st < DEPTH && st < ns; ++st) dma.issue(st, kb, lds + st * STAGE);
+    for (int st = 1; st < DEPTH && st < ns; ++st) dma.issue(st, kb, lds + st * STAGE, a_off);
     const int c = wave % CH, f0 = wave / CH;
     const bool active = ALL || wave < RF * CH;   // wave-uniform
     Acc acc[FPW][NB];
@@ -668,7 +667,7 @@ __global__ __launch_bounds__(1024) void moe_rows_staged_kernel(MoeArgs p) {
         }
         }
         __syncthreads();
-        if (st + DEPTH < ns) dma.issue(st + DEPTH, kb, buf);
+        if (st + DEPTH < ns) dma.issue(st + DEPTH, kb, buf, a_off);
     }
     Acc *part = reinterpret_cast<Acc *>(lds);
     if (active) {
