@@ -512,7 +512,7 @@ void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
         int rf, blk, nbb;
         mfma2::last_rows_blocks(rem, p.N, rf, blk, nbb);
 #define BK_F8RB(RF, NB, SB, DEPTH)                                                                        \
-        if (rf == (RF) && nbb == (NB)) {                                                  \
+        if (rf == (RF) && nbb == (NB) && mfma2::stages_fit(p.K, SB)) {                                       \
             hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH>),           \
                                dim3(p.N / (16 * (NB)), blk), dim3(1024), (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), \
                                stream, p, m0);                                                               \
@@ -524,7 +524,7 @@ void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
     }
     const int nb = rem <= 32 ? mfma2::last_rows_width(p.N) : mfma2::last_rows_col_frags(p.N);
 #define BK_F8ROWS(RF, NB, SB, DEPTH)                                                                     \
-    if (rem <= 16 * (RF) && nb == (NB)) {                                              \
+    if (rem <= 16 * (RF) && nb == (NB) && mfma2::stages_fit(p.K, SB)) {                                   \
         hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH>),           \
                            dim3((p.N + 16 * (NB) - 1) / (16 * (NB))), dim3(1024), (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), \
                            stream, p, m0);                                                               \
@@ -694,7 +694,7 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
                 int rf, blk, nbb;
                 mfma2::last_rows_blocks(rem, p.N, rf, blk, nbb);
 #define BK_F8RRRB(RF, NB, SB, DEPTH)                                                                      \
-                if (rf == (RF) && nbb == (NB)) {                                                             \
+                if (rf == (RF) && nbb == (NB) && mfma2::stages_fit(p.K, SB)) {                               \
                     hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH, true>), \
                                        dim3(p.N / (16 * (NB)), blk), dim3(1024),                             \
                                        (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), stream, p, pm.M);   \
@@ -706,7 +706,7 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
             }
             const int nb = mfma2::last_rows_col_frags(p.N);
 #define BK_F8RRRROWS(RF, NB, SB, DEPTH)                                                                    \
-            if (rem <= 16 * (RF) && nb == (NB)) {                                                         \
+            if (rem <= 16 * (RF) && nb == (NB) && mfma2::stages_fit(p.K, SB)) {                           \
                 hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH, true>), \
                                    dim3(p.N / (16 * (NB))), dim3(1024),                                  \
                                    (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), stream, p, pm.M);    \

@@ -18,6 +18,7 @@ extern "C" {
 int64_t row_b_bytes(int K, int N, int64_t ld) { return mfma2::row_b_bytes(K, N, ld); }
 int dma_extent_ok(int rows, int64_t ld) { return mfma2::dma_extent_ok(rows, ld); }
 unsigned row_offset(int row, int64_t ld) { return (unsigned)mfma2::row_offset(row, ld); }
+int stages_fit(int K, int SB) { return mfma2::stages_fit(K, SB); }
 }
 """
 
@@ -54,6 +55,15 @@ def test_row_major_b_extent(rules, k, n, ld):
     assert not admitted[k:].any()
     assert (off[admitted] < own).all()
     assert admitted[:k, : (n + 15) // 16].all()
+
+
+def test_stage_depths(rules):
+    """A stage deeper than 512 bytes only where K fills it as far as it fills
+    stages of 512."""
+    for k in range(16, 20000, 16):
+        assert rules.stages_fit(k, 512) and rules.stages_fit(k, 256)
+        for sb in (1024, 2048):
+            assert rules.stages_fit(k, sb) == (-(-k // 512) % (sb // 512) == 0)
 
 
 @pytest.mark.parametrize("rows", [1, 64, 200, 256, 257, 600, 12000])
