@@ -522,7 +522,7 @@ void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
         BK_F8RB(2, 1, 1024, 3) BK_F8RB(2, 2, 1024, 2)
 #undef BK_F8RB
     }
-    const int nb = rem <= 32 ? mfma2::last_rows_width(p.N) : mfma2::last_rows_col_frags(p.N);
+    const int nb = rem <= 32 ? mfma2::last_rows_width(p.N, rem, p.K) : mfma2::last_rows_col_frags(p.N);
 #define BK_F8ROWS(RF, NB, SB, DEPTH)                                                                     \
     if (rem <= 16 * (RF) && nb == (NB) && mfma2::stages_fit(p.K, SB)) {                                   \
         hipLaunchKernelGGL((gemm_fp8_rcr_rows_staged_kernel<FMT, EPI, ACT, RF, NB, SB, DEPTH>),           \

@@ -546,24 +546,25 @@ inline int last_rows_col_frags(int N, int blocks = 1) {
 
 // Column fragments per workgroup of an RCR last-rows pass of at most 32 rows,
 // any number of them (the columns past N of the last group are neither read
-// nor stored): the width with the fewest columns per CU, counting whole
-// rounds of 256 workgroups, the wider of two alike.  With one round the pass
-// streams its weights at about 4.6 TB/s; 344 workgroups in a round and a third
-// take two.  int8, 20 rows, K = 4096, rotated weights (us by 1 / 2 / 3 / 4 / 6 /
-// 7 fragments): N = 5120 8.8 / 7.8 / 9.1, N = 11008 13.9 / 13.1 / 11.7 / 12.3,
-// N = 14336 17.5 / 14.3 / 17.0 / 14.1, N = 22016 24.6 / 21.0 / 19.1 / 24.4 /
-// 19.6, N = 28672 30.1 / 27.3 / 27.0 / 28.2 / 32.8 / 25.7.
-inline int last_rows_width(int N) {
-    int best = 1, cols = 0;
-    for (const int nb : {1, 2, 3, 4, 6, 7}) {
-        const int groups = (N + 16 * nb - 1) / (16 * nb);
-        const int c = (groups + 255) / 256 * nb;
-        if (nb == 1 || c <= cols) {
-            best = nb;
-            cols = c;
-        }
-    }
-    return best;
+// nor stored).  Up to N = 16384 the narrowest width whose groups are one round
+// of the 256 CUs (three fragments for two at K = 8192: 16 x 5120 12.7 -> 10.4 us,
+// 24 x 8192 17.3 -> 16.6; at K = 4096 7.0 / 7.2 and 9.5 / 9.9, at 14336 19.3 / 22.5
+// and 22.5 / 25.6).  Past that two rounds of 48 columns (64 up to 16 rows), which
+// the LDS holds twice per CU, or for deep K or more rows one round of 96 or 112.
+// Never one fragment there: every workgroup stages all the rows.  us by 1 / 2 / 3 /
+// 4 / 6 / 7 fragments, K = 4096 unless stated, rotated weights, graph replay, int8:
+// 24 x 20480 23.5 / 23.9 / 20.2 / 25.3 / 21.8 / 21.9; 24 x 22016 26.2 / 24.7 / 20.9 /
+// 26.1 / 23.3 / 23.4, at K = 14336 71.1 / 59.6 / 53.3 / 61.1 / 48.4 / 51.0; 8 x 28672
+// 25.5 / 25.3 / 25.1 / 23.9 / 30.6 / 25.5; 24 x 28672 31.0 / 30.4 / 26.7 / 28.2 / 33.1 /
+// 26.8; 32 x 43008 46.6 / 46.9 / 39.2 / 43.3 / 42.8 / 44.8; e4m3, 16 x 43008, K = 1024:
+// 21.6 / 10.8 / 10.2 / 10.1 / 11.2 / 11.3.
+inline int last_rows_width(int N, int rem, int K) {
+    const int one_round = (N + 4095) / 4096;
+    if (one_round == 2 && K > 4096 && K <= 8192) return 3;
+    if (one_round <= 4) return one_round;
+    if (N <= 24576) return K <= 8192 ? 3 : 6;
+    if (rem <= 16) return 4;
+    return N <= 28672 ? 7 : 3;
 }
 
 // Row blocks of a last-rows pass of 33-128 rows when the rule above gives

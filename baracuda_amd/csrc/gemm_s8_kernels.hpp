@@ -1572,7 +1572,7 @@ bool launch_row_blocks(const S8Args &p, hipStream_t stream) {
 // The last `rem` (<= kRowsPathMax) rows, from row m0 (N % 16 == 0).
 template <int EPI, bool VecOut, int ACT, typename BiasT>
 void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
-    const int nb = rem <= 32 ? mfma2::last_rows_width(p.N) : mfma2::last_rows_col_frags(p.N);
+    const int nb = rem <= 32 ? mfma2::last_rows_width(p.N, rem, p.K) : mfma2::last_rows_col_frags(p.N);
     if (nb == 1 && rem > 32) {
         // 33-128 rows where 16-column workgroups would each read all
         // of them: 2-4 row blocks (last_rows_blocks).  K = 4096,
@@ -1606,7 +1606,11 @@ void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
     // 4096 6.55 / 6.93 -> 6.37 / 6.42 us, N = 2048 4.95 / 5.27 -> 4.87 / 4.90;
     // it stays ahead up to 8 rows), 8 at 32 columns, 5 at 64 (N = 14336 /
     // 12288, M = 8 14.2 / 11.6 -> 13.2 / 10.8 us staged, level at 2-5 rows).
-    if (rem <= (nb == 1 ? 10 : nb == 2 ? 8 : nb == 4 ? 5 : 1) && p.K % 1024 == 0 && p.K <= kRowsDmaMaxK) {
+    // Past N = 16384 only where two of its workgroups share a CU's LDS and each
+    // still has 3 KiB of a row to stream (M = 2, it / staged, N = 28672: K = 2048
+    // 14.5 / 12.8, 4096 22.5 / 25.3, 8192 49.0 / 44.1; N = 43008, 4096 32.3 / 34.4).
+    const int dma_rows = nb == 1 ? 10 : nb == 2 ? 8 : nb == 4 && (p.N <= 16384 || (p.K > 2048 && p.K <= 4096)) ? 5 : 1;
+    if (rem <= dma_rows && p.K % 1024 == 0 && p.K <= kRowsDmaMaxK) {
         // B rows; the 16 waves' partial sums reuse the same LDS
         const size_t lds = std::max((size_t)16 * p.K, (size_t)kRowsDmaWaves * 1024);
         hipLaunchKernelGGL((gemm_s8_rcr_rows_dma_kernel<EPI, VecOut, ACT, BiasT, 1>), dim3(p.N / 16),

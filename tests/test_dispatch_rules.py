@@ -18,6 +18,7 @@ extern "C" {
 int64_t row_b_bytes(int K, int N, int64_t ld) { return mfma2::row_b_bytes(K, N, ld); }
 int dma_extent_ok(int rows, int64_t ld) { return mfma2::dma_extent_ok(rows, ld); }
 unsigned row_offset(int row, int64_t ld) { return (unsigned)mfma2::row_offset(row, ld); }
+int last_rows_width(int N, int rem, int K) { return mfma2::last_rows_width(N, rem, K); }
 int stages_fit(int K, int SB) { return mfma2::stages_fit(K, SB); }
 }
 """
@@ -55,6 +56,23 @@ def test_row_major_b_extent(rules, k, n, ld):
     assert not admitted[k:].any()
     assert (off[admitted] < own).all()
     assert admitted[:k, : (n + 15) // 16].all()
+
+
+@pytest.mark.parametrize("rem", [1, 2, 5, 16, 17, 32])
+@pytest.mark.parametrize("k", [16, 512, 4096, 8192, 14336])
+def test_last_rows_width(rules, rem, k):
+    """One fragment only where it is one round of 256 workgroups; past one round
+    of the widest group no width needs more than a half over the fewest columns
+    per CU; the launchers have every width that the rule gives."""
+    for n in range(16, 65536, 16):
+        nb = rules.last_rows_width(n, rem, k)
+        groups = -(-n // (16 * nb))
+        assert nb in (1, 2, 3, 4, 6, 7)
+        assert nb > 1 or groups <= 256
+        if n <= 28672:
+            assert groups <= 512
+        per_cu = {w: -(-(-(-n // (16 * w))) // 256) * w for w in (1, 2, 3, 4, 6, 7)}
+        assert per_cu[nb] <= 1.5 * min(per_cu.values())
 
 
 def test_stage_depths(rules):

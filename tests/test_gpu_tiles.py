@@ -29,7 +29,7 @@ ROW_SHAPES = [(1, 4096, 4080), (1, 272, 48), (5, 512, 1040), (9, 12288, 304), (1
               (60, 12288, 304), (100, 272, 656), (120, 6144, 176), (200, 1024, 1072), (400, 1024, 208),
               (4160, 4096, 144),
               # 48-, 96- and 112-column workgroups, the last one partly past N
-              (20, 11008, 304), (12, 22016, 144), (30, 28656, 144)]
+              (20, 11008, 304), (12, 22016, 144), (30, 28656, 144), (12, 17920, 528), (20, 20464, 8720), (9, 43008, 272)]
 
 
 def _acc(a, b):
