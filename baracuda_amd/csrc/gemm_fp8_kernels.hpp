@@ -627,11 +627,11 @@ template <int FMT, int EPI, int ACT>
 void launch_fp8_rcr(const F8Args &p, hipStream_t stream) {
     const int rem = mfma2::last_rows_pass(p.M, p.N, 128);
     if (rem == p.M) {
-        if (rem > 32 && !mfma2::few_tiles(p.M, p.N)) launch_fp8_tiles<FMT, F8_RCR, EPI, ACT>(p, stream);
+        if (rem > 32 && !mfma2::row_blocks_pay(p.M, p.N, p.K)) launch_fp8_tiles<FMT, F8_RCR, EPI, ACT>(p, stream);
         else launch_fp8_rows<FMT, EPI, ACT>(p, 0, rem, stream);
         return;
     }
-    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && mfma2::few_tiles(p.M, p.N) &&
+    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && mfma2::row_blocks_pay(p.M, p.N, p.K) &&
         launch_fp8_row_blocks<FMT, EPI, ACT>(p, stream))
         return;
     if (rem != 0 && mfma2::last_rows_pay(p.M, p.N, p.K, rem)) {

@@ -207,14 +207,30 @@ inline RingTile ring_tile(int M, int N, int kbytes, float *cost = nullptr, RingT
     return (RingTile)best;
 }
 
-// Row blocks of the staged last-rows kernels instead of tiles (33-512 rows)
-// where 64 x 64 tiles would leave half of the CUs idle: they split K over
-// their waves, which a tile does not.  us, int8, blocks against the best
-// tile: 200 x 1024 x 4096 7.0 / 9.8, 128 x 4096 x 4096 8.5 / 10.0, 512 x 1024
-// x 4096 8.3 / 10.1, 128 x 4096 x 14336 25.9 / 33; past the line 200 x 4096 x
-// 4096 11.5 / 10.2, 384 x 2048 x 1024 5.7 / 4.9, 128 x 8192 x 4096 14.9 /
-// 11.7, 64 x 14336 x 4096 17.8 / 15.7.
-inline bool few_tiles(int M, int N) { return (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 128; }
+// Row blocks of the staged last-rows kernels instead of tiles (33-512 rows):
+// they split K over their waves, which a tile does not.
+//  - Where 64 x 64 tiles would leave half of the CUs idle.  us, int8, blocks
+//    against the best tile: 200 x 1024 x 4096 7.0 / 9.8, 128 x 4096 x 4096 8.5 /
+//    10.0, 512 x 1024 x 4096 8.3 / 10.1, 128 x 4096 x 14336 25.9 / 33; past the
+//    line 200 x 4096 x 4096 11.5 / 10.2, 384 x 2048 x 1024 5.7 / 4.9, 128 x 8192
+//    x 4096 14.9 / 11.7, 64 x 14336 x 4096 17.8 / 15.7.
+//  - Past one round of 64 x 64 tiles with a deep K, where the tiles wait for
+//    the weights: 160 x 6144 x 8192 27.3 / 32.0, 256 x 8192 x 8192 32.8 / 34.4, 384
+//    x 4096 x 14336 50.1 / 56.3, 300 x 5120 x 14336 45.1 / 57.0, 100 x 14336 x 8192
+//    33.7 / 35.5, but 384 x 4096 x 8192 26.6 / 24.4; 80 x 14336 x 4096 19.7 / 20.3,
+//    100 x 14336 x 4096 20.8 / 20.6.  Within one round later: 160 x 5120 x 14336
+//    32.0 / 34.5, 200 x 4096 x 11264 24.2 / 26.3, 256 x 4096 x 11264 28.4 / 26.7,
+//    256 x 4096 x 14336 35.0 / 35.9, 128 x 5120 x 14336 42.8 / 37.0, 300 x 2048 x
+//    14336 31.7 / 26.8.
+// There only as one round of workgroups (launch_row_blocks checks that for more
+// than 128 rows): 100 x 11008 x 14336 as 344 of them 69.3 / 58.4.
+inline bool row_blocks_pay(int M, int N, int kbytes) {
+    const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    if (t64 <= 128) return true;
+    if (M <= 128 && N / (16 * last_rows_col_frags(N)) > 256) return false;
+    if (t64 <= 256) return M > 128 && (M <= 224 ? kbytes >= 11264 : M <= 256 && kbytes > 12288);
+    return kbytes >= (M <= 96 ? 4096 : M <= 256 ? 8192 : 9216);
+}
 
 // Whole 256-row tiles and a last-rows pass for more than 512 rows, against
 // the cheapest tile over all rows: the pass reads the weights once more, at

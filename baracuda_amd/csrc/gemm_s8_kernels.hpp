@@ -1666,11 +1666,11 @@ void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *works
     }
     const int rem = rows_path_rows(p.M, p.N);
     if (rem == p.M) {
-        if (VecOut && rem > 32 && !mfma2::few_tiles(p.M, p.N)) launch_tiles<EPI, VecOut, ACT, BiasT>(p, stream);
+        if (VecOut && rem > 32 && !mfma2::row_blocks_pay(p.M, p.N, p.K)) launch_tiles<EPI, VecOut, ACT, BiasT>(p, stream);
         else launch_last_rows<EPI, VecOut, ACT, BiasT>(p, 0, rem, stream);
         return;
     }
-    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && (!VecOut || mfma2::few_tiles(p.M, p.N)) &&
+    if (p.M > 128 && p.M <= 512 && p.N % 16 == 0 && (!VecOut || mfma2::row_blocks_pay(p.M, p.N, p.K)) &&
         launch_row_blocks<EPI, VecOut, ACT, BiasT>(p, stream))
         return;
     if (rem != 0 && (!VecOut || mfma2::last_rows_pay(p.M, p.N, p.K, rem))) {

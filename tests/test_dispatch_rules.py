@@ -19,7 +19,11 @@ int64_t row_b_bytes(int K, int N, int64_t ld) { return mfma2::row_b_bytes(K, N, 
 int dma_extent_ok(int rows, int64_t ld) { return mfma2::dma_extent_ok(rows, ld); }
 unsigned row_offset(int row, int64_t ld) { return (unsigned)mfma2::row_offset(row, ld); }
 int last_rows_width(int N, int rem, int K) { return mfma2::last_rows_width(N, rem, K); }
+int last_rows_pass(int M, int N) { return mfma2::last_rows_pass(M, N, 128); }
+int last_rows_pay(int M, int N, int K, int rem) { return mfma2::last_rows_pay(M, N, K, rem); }
+int last_rows_col_frags(int N, int blocks) { return mfma2::last_rows_col_frags(N, blocks); }
 int stages_fit(int K, int SB) { return mfma2::stages_fit(K, SB); }
+int row_blocks_pay(int M, int N, int K) { return mfma2::row_blocks_pay(M, N, K); }
 }
 """
 
@@ -84,6 +88,19 @@ def test_stage_depths(rules):
             assert rules.stages_fit(k, sb) == (-(-k // 512) % (sb // 512) == 0)
 
 
+def test_row_blocks_or_tiles(rules):
+    """Row blocks and tiles on the sides of the line where each was measured the
+    faster (int8 and e4m3)."""
+    blocks = [(200, 1024, 4096), (128, 4096, 14336), (512, 1024, 4096), (160, 6144, 8192), (256, 8192, 8192),
+              (300, 4096, 14336), (384, 4096, 14336), (512, 4096, 14336), (300, 5120, 14336), (100, 14336, 8192),
+              (80, 14336, 14336), (160, 5120, 14336), (200, 4096, 11264), (256, 4096, 14336)]
+    tiles = [(200, 4096, 4096), (384, 2048, 1024), (128, 8192, 4096), (64, 14336, 4096), (384, 4096, 8192),
+             (128, 5120, 14336), (128, 11008, 14336), (80, 11008, 14336), (256, 4096, 11264), (300, 2048, 14336),
+             (128, 14336, 4096), (512, 4096, 4096)]
+    assert [s for s in blocks if not rules.row_blocks_pay(*s)] == []
+    assert [s for s in tiles if rules.row_blocks_pay(*s)] == []
+
+
 @pytest.mark.parametrize("rows", [1, 64, 200, 256, 257, 600, 12000])
 def test_row_offsets_of_padded_tiles(rules, rows):
     """The offsets of every tile height and column group stay exact in 32 bits,
@@ -94,3 +111,20 @@ def test_row_offsets_of_padded_tiles(rules, rows):
         last = -(-rows // edge) * edge - 1
         assert rules.row_offset(last, ld) == last * ld < 2 ** 32 - ld
         assert rules.row_offset(rows, ld) >= rows * ld      # past the extent
+
+
+def test_routes_of_wide_last_rows(rules):
+    """The shapes with which tests/test_gpu_tiles.py means the 32-column
+    kernels of four and eight fragments, and row blocks past 128 tiles, get them."""
+    assert rules.row_blocks_pay(40, 6176, 304) and rules.last_rows_col_frags(6176, 1) == 2
+    for m, rem in [(1856, 64), (1892, 100)]:
+        assert rules.last_rows_pass(m, 8224) == rem and rules.last_rows_pay(m, 8224, 144, rem)
+        assert not rules.row_blocks_pay(m, 8224, 144) and rules.last_rows_col_frags(8224, 1) == 2
+    # (rows, N, K, rows of a block, fragments): one round of workgroups each
+    for m, n, k, rb, nb in [(160, 5120, 11280, 64, 4), (384, 2720, 9232, 128, 2), (200, 8192, 8208, 128, 4)]:
+        assert rules.row_blocks_pay(m, n, k)
+        blocks = -(-m // rb)
+        assert rules.last_rows_col_frags(n, blocks) == nb and blocks * (n // (16 * nb)) <= 256
+        if rb == 128:
+            b4 = -(-m // 64)
+            assert b4 * (n // (16 * rules.last_rows_col_frags(n, b4))) > 256

@@ -24,10 +24,15 @@ pytestmark = pytest.mark.gpu
 TILE_SHAPES = [(300, 1700, 208), (450, 2896, 1040), (1000, 2500, 1136), (1500, 5120, 336), (2300, 5008, 400),
                (3070, 4100, 336), (4000, 4100, 48), (513, 2064, 16)]
 # one row (partial kilobyte), one / two / four / eight fragments, each column
-# width, row blocks, whole tiles with last rows
+# width, row blocks, whole tiles with last rows (test_dispatch_rules.py has the
+# routes of the wider ones)
 ROW_SHAPES = [(1, 4096, 4080), (1, 272, 48), (5, 512, 1040), (9, 12288, 304), (13, 6160, 1552), (24, 4096, 2752),
               (60, 12288, 304), (100, 272, 656), (120, 6144, 176), (200, 1024, 1072), (400, 1024, 208),
               (4160, 4096, 144),
+              # 32 columns with four and eight fragments (test_dispatch_rules.py
+              # has their routes), row blocks of deep K past 128 tiles
+              (40, 6176, 304), (1856, 8224, 144), (1892, 8224, 144), (100, 14336, 8208), (160, 5120, 11280),
+              (384, 2720, 9232), (200, 8192, 8208),
               # 48-, 96- and 112-column workgroups, the last one partly past N
               (20, 11008, 304), (12, 22016, 144), (30, 28656, 144), (12, 17920, 528), (20, 20464, 8720), (9, 43008, 272)]
 
