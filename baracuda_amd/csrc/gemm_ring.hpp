@@ -192,8 +192,16 @@ inline float ring_cost(const RingCost &c, int M, int N, int kbytes) {
 }
 
 // `first`: the smallest shape the caller has (row-major B tiles are 256
-// columns wide, so they start at 128 x 256).
+// columns wide, so they start at 128 x 256).  Past three rounds of 256 x 256
+// those: the last round overlaps the others, so that its idle CUs cost less than
+// the model's whole round (int8, 3072 x 17920 x 4096, 3.3 rounds: 214 us, 225 on
+// 128 x 256; e4m3, 3072 x 28672 x 2048, 5.25 rounds: 174, 186 on 192 x 256; at 2.3
+// rounds, 600 x 50176 x 4096, 178 against 141 on 128 x 256).
 inline RingTile ring_tile(int M, int N, int kbytes, float *cost = nullptr, RingTile first = RT_64x64) {
+    if ((int64_t)((M + 255) / 256) * ((N + 255) / 256) > 3 * 256) {
+        if (cost) *cost = ring_cost(kRingCost[RT_256x256], M, N, kbytes);
+        return RT_256x256;
+    }
     int best = first;
     float us = 0.0f;
     for (int i = first; i <= RT_256x256; ++i) {

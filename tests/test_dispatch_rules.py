@@ -24,6 +24,7 @@ int last_rows_pay(int M, int N, int K, int rem) { return mfma2::last_rows_pay(M,
 int last_rows_col_frags(int N, int blocks) { return mfma2::last_rows_col_frags(N, blocks); }
 int stages_fit(int K, int SB) { return mfma2::stages_fit(K, SB); }
 int row_blocks_pay(int M, int N, int K) { return mfma2::row_blocks_pay(M, N, K); }
+int ring_tile(int M, int N, int K, int first) { return mfma2::ring_tile(M, N, K, nullptr, (mfma2::RingTile)first); }
 }
 """
 
@@ -99,6 +100,16 @@ def test_row_blocks_or_tiles(rules):
              (128, 14336, 4096), (512, 4096, 4096)]
     assert [s for s in blocks if not rules.row_blocks_pay(*s)] == []
     assert [s for s in tiles if rules.row_blocks_pay(*s)] == []
+
+
+def test_tile_of_many_rounds(rules):
+    """Past three rounds of 256 x 256 tiles nothing smaller; the shapes of one
+    round keep their tile (0 .. 5: 64x64, 64x128, 128x128, 128x256, 192x256, 256x256)."""
+    for s in [(3072, 17920, 4096), (4096, 13824, 4096), (3072, 28672, 2048), (1024, 50176, 4096)]:
+        assert rules.ring_tile(*s, 0) == rules.ring_tile(*s, 3) == 5
+    for s, t in [((777, 11008, 4096), 4), ((1500, 5120, 2880), 3), ((810, 2352, 1856), 1), ((3072, 4096, 4096), 4),
+                 ((600, 50176, 4096), 3), ((1000, 17920, 1024), 4), ((4096, 4096, 4096), 5)]:
+        assert rules.ring_tile(*s, 0) == t
 
 
 @pytest.mark.parametrize("rows", [1, 64, 200, 256, 257, 600, 12000])
