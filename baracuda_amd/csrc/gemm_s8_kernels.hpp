@@ -1769,9 +1769,12 @@ bool launch_rrr_rows(const S8Args &p, hipStream_t stream) {
     // tiles 40.5 / 37.7)
     int rf, nb;
     rows_blocks_plan(p.M, p.N, rem, whole, rf, blocks, nb);
-    // more than a round of workgroups: tiles (512 x 14336 x 4096: 128 x 256
-    // tiles 28 us, four rounds of row blocks 69)
-    if (whole && blocks * (p.N / (16 * nb)) > 256) return false;
+    // more than a round and a half of workgroups: tiles (512 x 14336 x 4096: 128 x
+    // 256 tiles 28 us, four rounds of row blocks 69).  Up to there the tiles
+    // would be at most a sixth of the CUs (256 x 5120 x 14336, 320 workgroups 93
+    // us, 40 tiles 114; 160 x 2816 x 8192, 352 42, 22 tiles 48; 428 x 1440 x 512,
+    // 360 7.5, 24 tiles 8.6).
+    if (whole && blocks * (p.N / (16 * nb)) > 384) return false;
     S8Args pm = p;
     pm.M = whole ? 0 : p.M - rem;
     if (pm.M > 0 && launch_rrr_dma<ACT, BiasT>(pm, stream) != kOk) return false;
