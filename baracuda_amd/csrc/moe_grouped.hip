@@ -21,7 +21,7 @@
 // LDS counters (no global atomics, no memset: graph-capturable), and the GEMM
 // is one launch whose workgroups walk the ragged per-expert tile list.
 #include "gemm_mfma.hpp"
-#include "gemm_ring.hpp"
+#include "moe_rules.hpp"
 
 namespace bk {
 namespace {
@@ -772,26 +772,6 @@ __global__ __launch_bounds__(256) void moe_row_kernel(MoeArgs p) {
     }
 }
 
-// Tile shape by the dense tiles' model: an expert's rows end in a tile that is
-// half empty on average, so about size_m / TB + experts / 2 slots of TB rows
-// (the counts are on the GPU).  256 x 256 only where its kernel takes the
-// problem.
-inline mfma2::RingTile moe_tile_shape(int size_m, int E, int N, int kb, bool whole) {
-    int best = -1;
-    float us = 0.0f;
-    for (const int i : {mfma2::RT_64x128, mfma2::RT_128x128, mfma2::RT_128x256, mfma2::RT_256x256}) {
-        if (i == mfma2::RT_256x256 && !whole) continue;
-        const mfma2::RingCost &c = mfma2::kRingCost[i];
-        const float slots = (float)size_m / (float)c.tm + 0.5f * (float)std::min(E, size_m);
-        const float t = mfma2::ring_cost_tiles(c, (int64_t)(slots * (float)((N + c.tn - 1) / c.tn) + 0.5f), kb);
-        if (best < 0 || t < us) {
-            best = i;
-            us = t;
-        }
-    }
-    return (mfma2::RingTile)best;
-}
-
 // Offsets, then the grouped GEMM (DMA path when the problem fits it).
 template <int KIND>
 int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_counts,
@@ -799,17 +779,10 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
     constexpr int ES = MoeElem<KIND>::SIZE;
     // Upper bound on ragged m-tiles: sum_e ceil(cnt_e / BM) <= ceil(size_m / BM) + E.
     const int slots = (p.size_m + BM - 1) / BM + p.E;
-    // The DMA path needs whole 128-byte K stages, N a multiple of 256, 16-byte
-    // aligned operands, byte offsets that fit 32 bits (per input / per expert
-    // slab) and what its epilogue needs (out_ok).
     const int64_t kb = (int64_t)p.K * ES;
     const int64_t x_rows = p.topk_w ? p.size_m : (p.size_m + p.topk - 1) / p.topk;
-    const bool ring = kb % 16 == 0 && p.N % 8 == 0 && mfma::aligned16(p.x) && mfma::aligned16(p.w) &&
-                      (x_rows + 1) * kb < (1ll << 31) && (int64_t)(p.N + 256) * kb < (1ll << 31) && out_ok &&
-                      mfma::aligned16(p.out);
-    const bool fast = kb % mfma2::BK == 0 && p.N % mfma2::BN == 0 && mfma::aligned16(p.x) &&
-                      mfma::aligned16(p.w) && x_rows * kb < (1ll << 31) &&
-                      (int64_t)p.N * kb < (1ll << 31) && out_ok;
+    const MoeFit fit = moe_fit(x_rows, p.N, kb, mfma::aligned16(p.x) && mfma::aligned16(p.w) && out_ok, mfma::aligned16(p.out));
+    const bool fast = fit.tiles256;
     // Decode launches (size_m <= 64) find their rows from the ids themselves
     // and write the counts and offsets: no offsets kernel in front (N =
     // 14336, K = 4096, E = 8, top-2, 2 rotated weight sets, graph replay: 1 /
@@ -823,7 +796,7 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
         // (2 / 3 tokens: 53.4 / 53.4 -> 48.0 / 48.0 us against the staged
         // kernel's 16-row blocks; at 2 pairs 22.5 against 22.4 us, at 8
         // 65.9 against 64.8 us: those stay staged)
-        if (ring && p.size_m > 2 && p.size_m <= 6 && kb % 1024 == 0) {
+        if (fit.decode && p.size_m > 2 && p.size_m <= 6 && kb % 1024 == 0) {
             if (kb % 2048 == 0)
                 hipLaunchKernelGGL((moe_row_kernel<KIND, 2, 2>), dim3(p.N / 4, p.E), dim3(256), 0, stream, q);
             else
@@ -831,7 +804,7 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
             return launch_status();
         }
     }
-    if (ring && p.size_m <= 64) {
+    if (fit.decode && p.size_m <= 64) {
         // decode-sized.  N = 14336, K = 4096, E = 8, top-2: 1 / 4 / 16 tokens
         // (2 / 5 / 7 experts) in 27.4 / 62.3 / 99.0 us (with the offsets
         // kernel) against 43.5 / 100.5 / 117.8 on 256-row tiles; at size_m
@@ -869,7 +842,7 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
     hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(1024), 0, stream, expert_ids, p.size_m, p.E,
                        expert_counts, const_cast<int32_t *>(p.offsets));
     if (hipPeekAtLastError() != hipSuccess) return kLaunch;
-    if (ring) {
+    if (fit.ring) {
         using mfma2::Cfg;
         switch (moe_tile_shape(p.size_m, p.E, p.N, (int)kb, fast)) {
             case mfma2::RT_64x128: launch_moe_ring<KIND, Cfg<2, 2, 64, 128>, 3, 2>(p, stream); return launch_status();

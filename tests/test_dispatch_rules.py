@@ -12,12 +12,16 @@ import pytest
 from baracuda_amd import build as B
 
 SOURCE = r"""
-#include "gemm_ring.hpp"
+#include "moe_rules.hpp"
 using namespace bk;
 extern "C" {
 int64_t row_b_bytes(int K, int N, int64_t ld) { return mfma2::row_b_bytes(K, N, ld); }
 int dma_extent_ok(int rows, int64_t ld) { return mfma2::dma_extent_ok(rows, ld); }
 unsigned row_offset(int row, int64_t ld) { return (unsigned)mfma2::row_offset(row, ld); }
+int moe_fit(int64_t x_rows, int N, int64_t kb, int operands, int out16) {
+    const MoeFit f = moe_fit(x_rows, N, kb, operands != 0, out16 != 0);
+    return f.decode + 2 * f.ring + 4 * f.tiles256;
+}
 int last_rows_width(int N, int rem, int K) { return mfma2::last_rows_width(N, rem, K); }
 int last_rows_pass(int M, int N) { return mfma2::last_rows_pass(M, N, 128); }
 int last_rows_pay(int M, int N, int K, int rem) { return mfma2::last_rows_pay(M, N, K, rem); }
@@ -42,6 +46,7 @@ def rules(tmp_path_factory):
     lib.dma_extent_ok.argtypes = [ctypes.c_int, ctypes.c_int64]
     lib.row_offset.restype = ctypes.c_uint32
     lib.row_offset.argtypes = [ctypes.c_int, ctypes.c_int64]
+    lib.moe_fit.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     return lib
 
 
@@ -122,6 +127,16 @@ def test_row_offsets_of_padded_tiles(rules, rows):
         last = -(-rows // edge) * edge - 1
         assert rules.row_offset(last, ld) == last * ld < 2 ** 32 - ld
         assert rules.row_offset(rows, ld) >= rows * ld      # past the extent
+
+
+def test_moe_fit(rules):
+    """Decode-sized problems keep their kernels with an output of any alignment."""
+    decode, ring, tiles256 = 1, 2, 4
+    assert rules.moe_fit(64, 14336, 8192, 1, 1) == decode + ring + tiles256
+    assert rules.moe_fit(64, 14336, 8192, 1, 0) == decode + tiles256
+    assert rules.moe_fit(64, 1408, 2064, 1, 1) == decode + ring
+    assert rules.moe_fit(64, 1412, 2064, 1, 1) == rules.moe_fit(64, 1408, 2056, 1, 1) == 0
+    assert rules.moe_fit(64, 14336, 8192, 0, 1) == 0
 
 
 def test_routes_of_wide_last_rows(rules):
