@@ -303,8 +303,9 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void gemm_fp8_ring_ker
 // + 3).  The CH chunk partials of a fragment pair are added in chunk order
 // through LDS and the waves run the tiles' epilogue, one fragment pair at a
 // time.  Requirements (checked by the launcher): K % 16 == 0, the fast
-// path's alignment and 2^31 extents, N % (16 NB) == 0; dynamic LDS of
-// DEPTH * (16 RF + 16 NB) * SB bytes.
+// path's alignment and 2^31 extents, N % 16 == 0 (N % (16 NB) == 0 with RowB or
+// several row blocks; otherwise the last group's columns past N load as zeros and
+// are not stored); dynamic LDS of DEPTH * (16 RF + 16 NB) * SB bytes.
 //
 // RowB: B row-major [K, N] (the RRR SKUs): the stage's B region holds its SB
 // k-rows of the 16 NB columns as they lie in memory (row pitch 16 NB bytes,

@@ -416,8 +416,10 @@ __device__ __forceinline__ void mma_block(AccTile<P> &acc, const Frags<P> &f) {
 }
 
 // Buffer resource (V#) for a raw byte buffer: base, stride 0, num_records =
-// `bytes` (accesses at or past it read as zero), dword3 = the gfx9-family
-// raw-buffer format word.  Built wave-uniform so it lives in SGPRs.
+// `bytes`, dword3 = the gfx9-family raw-buffer format word.  A dword reads as zero
+// when its per-lane plus scalar offset is at or past num_records, also where the
+// scalar offset alone is or num_records is 0 (probed inside one allocation).
+// Built wave-uniform so it lives in SGPRs.
 __device__ __forceinline__ v4i make_rsrc(const void *base, uint32_t bytes) {
     const uint64_t a = reinterpret_cast<uint64_t>(base);
     v4i r;

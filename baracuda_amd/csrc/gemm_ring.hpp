@@ -156,9 +156,9 @@ __device__ __forceinline__ void mainloop_ring(int8_t *lds, D d, int K, AccTile<P
 }
 
 // ---- which tile -------------------------------------------------------------
-// Tiles of the RCR GEMMs.  The first four run the ring loop (LDS of all
-// stages; 64-row tiles leave room for two workgroups per CU), the last is the
-// 256 x 256 kernel of gemm_mfma2.hpp.
+// Tiles of the GEMMs.  The first five run the ring loop (LDS of all stages;
+// 64-row tiles leave room for two workgroups per CU), 256 x 256 the two-stage
+// kernel of gemm_mfma2.hpp, or the ring with two stages when K % 128 != 0.
 enum RingTile { RT_64x64, RT_64x128, RT_128x128, RT_128x256, RT_192x256, RT_256x256 };
 struct RingCost {
     int tm, tn;

@@ -1159,7 +1159,8 @@ __global__ __launch_bounds__(NT, 1) void gemm_u8_rrr_kernel(S8Args p) {
     for_each_fragment(acc, [&](int ml, int nl, const v4i &v) { epi(ml, nl, v, m_base, n_base); });
 }
 
-// Whole-tile problems the LDS-DMA u8 RRR kernels take.
+// Problems the LDS-DMA u8 RRR tiles take (edges and a partial last stage
+// included).
 inline bool u8_rrr_dma_eligible(const S8Args &p) {
     return p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.a) && aligned16(p.b) &&
            dma_extent_ok(p.M, p.lda) && mfma2::row_b_extent_ok(p.K, p.ldb, mfma2::BK);
@@ -1744,8 +1745,8 @@ int32_t launch_rrr_dma(const S8Args &p, hipStream_t stream) {
 
 // s8 RRR last rows (decode-sized M; M % 256 in [1, 128] when a row of tiles
 // would start another round): the staged last-rows kernel reading row-major
-// B; false when the shape does not fit it (K % 512 == 0, 16-byte rows and
-// bases, N % (16 NB) == 0, K * ldb below 2^31).
+// B; false when the shape does not fit it (K % 16 == 0, 16-byte rows and
+// bases, N % 16 == 0, K rounded up to 512 rows times ldb below 2^31).
 template <int ACT, typename BiasT>
 bool launch_rrr_rows(const S8Args &p, hipStream_t stream) {
     int rem = mfma2::last_rows_pass(p.M, p.N, 128), blocks = 1;

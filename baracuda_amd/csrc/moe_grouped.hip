@@ -223,7 +223,8 @@ __device__ __forceinline__ void moe_store_h(const MoeArgs &p, const int32_t *row
     }
 }
 
-// General path (K tail / unaligned / N not a multiple of 256).
+// General path: unaligned operands or outputs, rows that are no whole 16-byte
+// units, N % 8 != 0 and not a multiple of 256.
 template <int KIND>
 __global__ __launch_bounds__(NT, 1) void moe_grouped_kernel(MoeArgs p) {
     constexpr int ES = MoeElem<KIND>::SIZE;

@@ -1,7 +1,5 @@
 // quant.hpp -- per-token symmetric int8 quantization of a row held as 8-value
-// chunks: loads, running max, scale and codes.  Shared by the quantizer and
-// the kernels that quantize their own activation row, so that both give the
-// same scale and codes bit for bit.
+// chunks: loads, running max, scale and codes.
 #pragma once
 
 #include "bk_common.hpp"
