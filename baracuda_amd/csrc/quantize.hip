@@ -219,8 +219,10 @@ int32_t launch_quant(int32_t N, int32_t D, int32_t qmin, int32_t qmax, const voi
         const bool keep = (int64_t)N * D <= kQKeepBytes;
         // Rows of up to 4096 bf16 values, one wave each, from kQFewRows on: below
         // that the chip is idle and a row's 64 values per lane are the time (1 x
-        // 4096 bf16 3.1 -> 2.6 us, 24 x 4096 4.7 -> 3.2 in a kernel trace).
-        if (vec && sizeof(T) == 2 && N > kQFewRows && nch <= 64 * 8) {
+        // 4096 bf16 3.1 -> 2.6 us, 24 x 4096 4.7 -> 3.2 in a kernel trace).  Rows of at
+        // most one chunk per lane stay with the wave (4 x 512 2.65 us, 2.85 in a
+        // workgroup).
+        if (vec && sizeof(T) == 2 && (N > kQFewRows || nch <= 64) && nch <= 64 * 8) {
             if constexpr (sizeof(T) == 2) {
                 const uint16_t *xi = (const uint16_t *)input;
                 S *sc = (S *)scale;

@@ -269,7 +269,7 @@ def test_gemv_dense_tall_slices(gpu, dtype, n, k, batch):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("shape", [(1, 8), (3, 2056), (256, 4096), (257, 4104), (2, 16384), (1, 16392), (300, 9000)])
+@pytest.mark.parametrize("shape", [(1, 8), (5, 512), (7, 520), (3, 2056), (256, 4096), (257, 4104), (2, 16384), (1, 16392), (300, 9000)])
 def test_quantize_row_widths(gpu, dtype, shape):
     """Every chunk count and both workgroup sizes of the vector quantizer."""
     G.test_quantize_per_token_bit_exact(gpu, dtype, shape)
