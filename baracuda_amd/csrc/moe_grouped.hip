@@ -811,12 +811,7 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
         // kernel) against 43.5 / 100.5 / 117.8 on 256-row tiles; at size_m
         // 96 / 128 8 row fragments ran level with the tiles (123 us), so
         // larger size_m stays on them.
-        // Columns per workgroup: the widest of 64, 32, 16 that leaves 192
-        // workgroups with rows, of about min(E, size_m) / 2 experts (the last
-        // group may lie partly past N).
-        const int touched = std::max(1, std::min(p.E, p.size_m) / 2);
-        int nb = 4;
-        while (nb > 1 && (int64_t)((p.N + 16 * nb - 1) / (16 * nb)) * touched < 192) nb /= 2;
+        const int nb = moe_decode_width(p.size_m, p.E, p.N, kb);   // the last group may lie partly past N
         // blocks of 16 rows up to 32 pairs, of 32 above (blockIdx.z): an
         // expert's few rows stage fewer padding rows (N = 14336, K = 4096,
         // 1 / 8 / 16 / 32 tokens top-2: 22.6 / 80.7 / 95.5 / 106.6 -> 21.6 /
@@ -835,7 +830,6 @@ int32_t launch_moe(const MoeArgs &p, const int32_t *expert_ids, int32_t *expert_
         BK_MOEROWS(1, 1, 512, 3)
         BK_MOEROWS(1, 2, 512, 3)
         BK_MOEROWS(1, 4, 512, 2)
-        BK_MOEROWS(2, 1, 512, 3)
         BK_MOEROWS(2, 2, 512, 3)
         BK_MOEROWS(2, 4, 512, 3)
 #undef BK_MOEROWS

@@ -22,6 +22,7 @@ int moe_fit(int64_t x_rows, int N, int64_t kb, int operands, int out16) {
     const MoeFit f = moe_fit(x_rows, N, kb, operands != 0, out16 != 0);
     return f.decode + 2 * f.ring + 4 * f.tiles256;
 }
+int moe_decode_width(int pairs, int E, int N, int64_t kb) { return bk::moe_decode_width(pairs, E, N, kb); }
 int last_rows_width(int N, int rem, int K) { return mfma2::last_rows_width(N, rem, K); }
 int last_rows_pass(int M, int N) { return mfma2::last_rows_pass(M, N, 128); }
 int last_rows_pay(int M, int N, int K, int rem) { return mfma2::last_rows_pay(M, N, K, rem); }
@@ -46,6 +47,7 @@ def rules(tmp_path_factory):
     lib.dma_extent_ok.argtypes = [ctypes.c_int, ctypes.c_int64]
     lib.row_offset.restype = ctypes.c_uint32
     lib.row_offset.argtypes = [ctypes.c_int, ctypes.c_int64]
+    lib.moe_decode_width.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64]
     lib.moe_fit.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     return lib
 
@@ -154,3 +156,18 @@ def test_routes_of_wide_last_rows(rules):
         if rb == 128:
             b4 = -(-m // 64)
             assert b4 * (n // (16 * rules.last_rows_col_frags(n, b4))) > 256
+
+
+def test_moe_decode_width(rules):
+    """The measured best width, or one within 3% of it: (pairs, experts, N, bytes of a row)."""
+    for width, cases in {1: [(2, 8, 1024, 2048), (4, 8, 1024, 8192), (8, 8, 7168, 8192), (16, 16, 2048, 8192)],
+                         2: [(2, 8, 2048, 2048), (8, 8, 1024, 4096), (16, 8, 7168, 4096), (32, 16, 7168, 2048),
+                             (16, 16, 2048, 4096), (64, 8, 1024, 2048)],
+                         4: [(2, 8, 14336, 8192), (8, 16, 2048, 4096), (24, 64, 2048, 4096), (4, 16, 7168, 8192),
+                             (64, 8, 7168, 4096), (48, 64, 1024, 8192)]}.items():
+        assert [c for c in cases if rules.moe_decode_width(*c) != width] == []
+    for pairs in range(1, 65):                     # the launcher has these
+        for e in (1, 8, 64, 1024):
+            for n in (8, 1000, 4096, 50000):
+                for kb in (16, 4096, 28672):
+                    assert rules.moe_decode_width(pairs, e, n, kb) in ((1, 2, 4) if pairs <= 32 else (2, 4))
