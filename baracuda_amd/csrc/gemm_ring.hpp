@@ -249,5 +249,29 @@ inline bool last_rows_pay(int M, int N, int kbytes, int rem) {
     return ring_cost(kRingCost[RT_256x256], M - rem, N, kbytes) + 3.0f + (float)N * (float)kbytes / 3.6e6f < all;
 }
 
+// A last round of `tail` 256 x 256 tiles behind `full` others split along K (with
+// the caller's workspace) against the tiles and row blocks without one.  us, int8
+// to bf16, split / without, weights rotated:
+//  - No whole round: the split takes 26-30 us at any K for its slots and second
+//    launch.  512 x 512 x 8192 31.0 / 11.5, 600 x 1024 x 8192 30.5 / 19.2, 768 x
+//    1152 x 16384 40.5 / 34.0, but 768 x 768 x 20480 37.0 / 44.8, 200 x 520 x 24576
+//    40.6 / 50.4; against row blocks, which split K themselves, 256 x 256 x 24576
+//    44.8 / 27.5, 512 x 1024 x 20480 35.1 / 32.8.
+//  - One whole round: N = 4096, K = 4096, M = 4296 / 4864 / 5120 / 6144 81.2 / 85.4,
+//    91.0 / 90.4, 93.3 / 89.5, 107.0 / 101.7; M = 4296, K = 2048 / 3072 51.3 / 47.0,
+//    63.7 / 65.5; K = 6144, M = 4864 / 5120 / 6144 121.1 / 127.9, 124.7 / 127.7, 144.4
+//    / 146.0.
+//  - Two: M = 8448 K = 4096 143.1 / 132.8, 8192 244.0 / 242.7, 14336 405.3 / 414.5, M
+//    = 9216 K = 8192 262.1 / 252.8.  More, where the tiles are 256 x 256 too: M =
+//    12544, K = 4096 / 8192 190.6 / 201.6, 337.7 / 376.6.
+inline bool tail_split_pays(int M, int N, int kbytes, int full, int tail) {
+    if (full == 0) {
+        const bool blocks = N % 16 == 0 && M <= 512 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 128;
+        return kbytes > (blocks ? 24576 : 16384);
+    }
+    if (full <= 256) return kbytes >= (tail <= 16 ? 3072 : 6144);
+    return full > 512 || kbytes >= 14336;
+}
+
 }  // namespace mfma2
 }  // namespace bk

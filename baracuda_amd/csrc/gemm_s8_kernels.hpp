@@ -230,9 +230,11 @@ constexpr int kRowsStagedSB = 512;
 inline int rows_path_rows(int M, int N, int limit = kRowsPathMax) { return mfma2::last_rows_pass(M, N, limit); }
 
 // Grids of at most kSmallTilesMax 256 x 256 tiles (under half a round on
-// the 256 CUs) run smaller tiles, except that with a tail-split workspace a
-// deep K (>= 4096) on fewer than 64 tiles of 128 x 128 splits K (512 x 512 x
-// 8192: 30.5 us against 43.6 on 128 x 128 tiles of two stages).
+// the 256 CUs) run smaller tiles.  A tail-split workspace is reported for a
+// deep K (>= 4096) on fewer than 64 tiles of 128 x 128; it is used where
+// tail_split_pays, and always by outputs without vector stores, which have one
+// ring tile (W8A8 bf16, N % 8 == 4, split / without: 260 x 1004 x 8192 28.9 / 38.3
+// us, 300 x 300 x 4096 20.6 / 20.9, 1000 x 756 x 4096 28.5 / 22.1).
 constexpr int kSmallTilesMax = 128;
 inline bool small_tiles_preferred(int M, int N, int K) {
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
@@ -1656,7 +1658,8 @@ void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *works
     }
     const TailSplit ts = tail_split_plan(p.M, p.N, p.K);
     if (ts.split > 1 && workspace != nullptr && workspace_bytes >= tail_split_workspace(p.M, p.N, p.K) &&
-        (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0) {
+        (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
+        (!VecOut || mfma2::tail_split_pays(p.M, p.N, p.K, ts.full_tiles, ts.tail_tiles))) {
         int32_t *slots = static_cast<int32_t *>(workspace);
         hipLaunchKernelGGL((gemm_s8_rcr_dma_kernel<EPI, VecOut, ACT, BiasT>),
                            dim3(ts.full_tiles + ts.tail_tiles * ts.split), dim3(DmaCfg::NT), 0, stream, p, ts,
@@ -1686,7 +1689,7 @@ void launch_kernel(const S8Args &p, bool fast_k, hipStream_t stream, void *works
 
 // workspace (optional): tail_split_workspace(M, N, K) bytes, 16-byte aligned,
 // contents on entry do not matter; given it, a partial last round of tiles
-// runs split along K (tail_split_plan).
+// runs split along K (tail_split_plan) where that is the faster way.
 template <int EPI, int ACT = ACT_NONE, typename BiasT = float>
 int32_t launch(const S8Args &p, hipStream_t stream, void *workspace = nullptr, size_t workspace_bytes = 0) {
     const int out_elem = (EPI == EPI_I32 || EPI == EPI_W8A8_F32) ? 4 : EPI == EPI_W8A8_F64 ? 8 : (EPI == EPI_S8 ? 1 : 2);

@@ -28,6 +28,7 @@ int last_rows_pass(int M, int N) { return mfma2::last_rows_pass(M, N, 128); }
 int last_rows_pay(int M, int N, int K, int rem) { return mfma2::last_rows_pay(M, N, K, rem); }
 int last_rows_col_frags(int N, int blocks) { return mfma2::last_rows_col_frags(N, blocks); }
 int stages_fit(int K, int SB) { return mfma2::stages_fit(K, SB); }
+int tail_split_pays(int M, int N, int K, int full, int tail) { return mfma2::tail_split_pays(M, N, K, full, tail); }
 int row_blocks_pay(int M, int N, int K) { return mfma2::row_blocks_pay(M, N, K); }
 int ring_tile(int M, int N, int K, int first) { return mfma2::ring_tile(M, N, K, nullptr, (mfma2::RingTile)first); }
 }
@@ -117,6 +118,17 @@ def test_tile_of_many_rounds(rules):
     for s, t in [((777, 11008, 4096), 4), ((1500, 5120, 2880), 3), ((810, 2352, 1856), 1), ((3072, 4096, 4096), 4),
                  ((600, 50176, 4096), 3), ((1000, 17920, 1024), 4), ((4096, 4096, 4096), 5)]:
         assert rules.ring_tile(*s, 0) == t
+
+
+@pytest.mark.parametrize("m,n,k,full,tail,split", [
+    (512, 512, 8192, 0, 4, False), (512, 1024, 4096, 0, 8, False), (768, 1152, 16384, 0, 15, False),
+    (256, 256, 24576, 0, 1, False), (768, 768, 20480, 0, 9, True), (200, 520, 24576, 0, 3, True),
+    (4296, 4096, 4096, 256, 16, True), (4296, 4096, 2048, 256, 16, False), (5120, 4096, 4096, 256, 64, False),
+    (5120, 4096, 8192, 256, 64, True), (8448, 4096, 4096, 512, 16, False), (8448, 4096, 14336, 512, 16, True),
+    (12544, 4096, 4096, 768, 16, True)])
+def test_tail_split_where_it_was_faster(rules, m, n, k, full, tail, split):
+    """A workspace does not move a call to the slower of the two measured ways."""
+    assert bool(rules.tail_split_pays(m, n, k, full, tail)) == split
 
 
 @pytest.mark.parametrize("rows", [1, 64, 200, 256, 257, 600, 12000])

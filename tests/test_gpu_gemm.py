@@ -175,10 +175,12 @@ def test_small_tiles_all_epilogues(gpu, shape):
         assert np.array_equal(got[r], O.gemm_w8a8_bf16(a, b, sa, sw, rows=(r, r + 1), nthreads=8)[0]), r
 
 
-@pytest.mark.parametrize("shape", [(512, 512, 8192), (300, 520, 4096), (200, 256, 4096), (1024, 768, 4096)])
+@pytest.mark.parametrize("shape", [(512, 512, 8192), (300, 520, 4096), (200, 256, 4096), (1024, 768, 4096),
+                                   (200, 264, 16512), (136, 144, 24704)])
 def test_tail_split_small_grids(gpu, shape):
     # Grids of at most 128 tiles with K >= 4096 on fewer than 64 128x128
-    # tiles split every tile along K when given the workspace: int32
+    # tiles report a workspace; given it, the last two shapes (K past 16384 /
+    # 24576) split every tile along K and the others run as without it: int32
     # accumulators exact, s8 with C / beta and a bias epilogue equal the oracle.
     m, n, k = shape
     print(f"case: tail split {shape}", flush=True)

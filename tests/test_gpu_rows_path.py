@@ -140,12 +140,13 @@ def test_rows_path_quantized_linear_f32_f64(gpu, shape):
     assert np.array_equal(out64.cpu().numpy()[rows], want64)
 
 
-def test_rows_path_with_and_without_split_workspace(gpu):
-    # 100 last rows at M = 1124, N = 16384, K = 1152 (not a multiple of the
-    # staged kernel's 512-byte stages): with the tail-split workspace the
-    # split runs, without it the last-rows pass; both equal the oracle rows.
-    m, n, k = 1124, 16384, 1152
-    print("case: rows path vs tail split", flush=True)
+@pytest.mark.parametrize("shape", [(1124, 16384, 1152), (4192, 4096, 3200)])
+def test_rows_path_with_and_without_split_workspace(gpu, shape):
+    # 100 / 96 last rows, K not a multiple of the staged kernel's 512-byte
+    # stages: without a workspace the last-rows pass or tiles, with it the
+    # split at K = 3200 (at 1152 it does not pay); both equal the oracle rows.
+    m, n, k = shape
+    print(f"case: rows path vs tail split {shape}", flush=True)
     g = rng(77)
     a, b = int8_uniform(g, (m, k)), int8_uniform(g, (n, k))
     plan = P.IntGemmPlan.select(P.IntGemmDescriptor(m, n, k, output=P.ElementKind.I32))
