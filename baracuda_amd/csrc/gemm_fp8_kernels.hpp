@@ -519,7 +519,7 @@ void launch_fp8_rows(const F8Args &p, int m0, int rem, hipStream_t stream) {
                                stream, p, m0);                                                               \
             return;                                                                                     \
         }
-        BK_F8RB(4, 1, 512, 2) BK_F8RB(4, 2, 512, 2) BK_F8RB(4, 4, 512, 2)
+        BK_F8RB(4, 1, 512, 2) BK_F8RB(4, 2, 512, 2)
         BK_F8RB(2, 1, 1024, 3) BK_F8RB(2, 2, 1024, 2)
 #undef BK_F8RB
     }
@@ -701,7 +701,7 @@ int32_t launch_fp8(const F8Args &p, hipStream_t stream) {
                                        (size_t)(DEPTH) * (16 * (RF) + 16 * (NB)) * (SB), stream, p, pm.M);   \
                     return launch_status();                                                                  \
                 }
-                BK_F8RRRB(4, 1, 512, 2) BK_F8RRRB(4, 2, 512, 2) BK_F8RRRB(4, 4, 512, 2)
+                BK_F8RRRB(4, 1, 512, 2) BK_F8RRRB(4, 2, 512, 2)
                 BK_F8RRRB(2, 1, 1024, 3) BK_F8RRRB(2, 2, 1024, 2)
 #undef BK_F8RRRB
             }

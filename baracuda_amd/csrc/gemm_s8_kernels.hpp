@@ -1592,7 +1592,7 @@ void launch_last_rows(const S8Args &p, int m0, int rem, hipStream_t stream) {
                                stream, p, m0);                                                                 \
             return;                                                                                            \
         }
-        BK_S8RBLK(2, 1) BK_S8RBLK(4, 1) BK_S8RBLK(2, 2) BK_S8RBLK(4, 2) BK_S8RBLK(2, 4) BK_S8RBLK(4, 4)
+        BK_S8RBLK(2, 1) BK_S8RBLK(4, 1) BK_S8RBLK(2, 2) BK_S8RBLK(4, 2)
 #undef BK_S8RBLK
     }
     if (rem == 1) {

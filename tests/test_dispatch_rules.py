@@ -27,6 +27,11 @@ int last_rows_width(int N, int rem, int K) { return mfma2::last_rows_width(N, re
 int last_rows_pass(int M, int N) { return mfma2::last_rows_pass(M, N, 128); }
 int last_rows_pay(int M, int N, int K, int rem) { return mfma2::last_rows_pay(M, N, K, rem); }
 int last_rows_col_frags(int N, int blocks) { return mfma2::last_rows_col_frags(N, blocks); }
+int last_rows_blocks(int rem, int N) {
+    int rf, blocks, nb;
+    mfma2::last_rows_blocks(rem, N, rf, blocks, nb);
+    return rf * 100 + nb * 10 + blocks;
+}
 int stages_fit(int K, int SB) { return mfma2::stages_fit(K, SB); }
 int tail_split_pays(int M, int N, int K, int full, int tail) { return mfma2::tail_split_pays(M, N, K, full, tail); }
 int row_blocks_pay(int M, int N, int K) { return mfma2::row_blocks_pay(M, N, K); }
@@ -141,6 +146,14 @@ def test_row_offsets_of_padded_tiles(rules, rows):
         last = -(-rows // edge) * edge - 1
         assert rules.row_offset(last, ld) == last * ld < 2 ** 32 - ld
         assert rules.row_offset(rows, ld) >= rows * ld      # past the extent
+
+
+def test_last_rows_block_forms(rules):
+    """The launchers have kernels for every row-block form the rule gives: 2 or 4
+    row fragments by 1 or 2 column fragments."""
+    forms = {rules.last_rows_blocks(rem, n) // 10 for n in range(16, 70000, 16) if rules.last_rows_col_frags(n, 1) == 1
+             for rem in (33, 48, 64, 65, 96, 97, 128)}
+    assert forms == {21, 22, 41, 42}
 
 
 def test_moe_fit(rules):
